@@ -214,6 +214,12 @@ __device__ bool gp_geometry(const double *X, const double xi[3], double *dNdx, d
     }
 }
 
+}  // namespace hipfem
+
+#include "hipfem_assemble.h"
+
+namespace hipfem {
+
 // ------------------------------------------------------------ assembly kernel
 template <int ET>
 __global__ __launch_bounds__(64) void k_assemble(const int *__restrict__ elems, int nelem_color,
@@ -223,11 +229,9 @@ __global__ __launch_bounds__(64) void k_assemble(const int *__restrict__ elems, 
                                                  const double *__restrict__ state, int ngp_total, int tangent,
                                                  const int32_t *__restrict__ rowptr, double *__restrict__ val,
                                                  int *__restrict__ bad, const int8_t *__restrict__ sflag,
-                                                 const float *__restrict__ dsur, double *__restrict__ kbuf)
+                                                 const float *__restrict__ dsur)
 {
-    // elems == nullptr: every element (block = element).  kbuf: the element's
-    // 3x3 blocks are stored (9 per node pair (a, b), row-major) for
-    // k_assemble_gather, else added into val (one color per launch)
+    // one color per launch: its elements' blocks are added into val
     constexpr int NEN = ElemT<ET>::NEN, NGP = ElemT<ET>::NGP;
     __shared__ double sX[NEN * 3];
     __shared__ double sN[NGP][NEN * 3];
@@ -243,7 +247,7 @@ __global__ __launch_bounds__(64) void k_assemble(const int *__restrict__ elems, 
 
     const int ei = blockIdx.x;
     if (ei >= nelem_color) return;
-    const int e = elems ? elems[ei] : ei;
+    const int e = elems[ei];
     const int t = threadIdx.x;
     for (int k = t; k < NEN * 3; k += 64) {
         const int node = conn[(size_t)e * NEN + k / 3];
@@ -306,20 +310,8 @@ __global__ __launch_bounds__(64) void k_assemble(const int *__restrict__ elems, 
     const double G = E / (2.0 * (1. + nu));
     const double Kb = E / (3.0 * (1. - 2. * nu));
     const double lam = Kb - 2.0 * G / 3.0;
-    // stored blocks (kbuf): the pairs a <= b, each also stored transposed as
-    // (b, a), so every element matrix is exactly symmetric
-    const int npairs = kbuf ? NEN * (NEN + 1) / 2 : NEN * NEN;
-    for (int blk = t; blk < npairs; blk += 64) {
-        int a = blk / NEN, b = blk % NEN;
-        if (kbuf) {
-            int rem = blk;
-            a = 0;
-            while (rem >= NEN - a) {
-                rem -= NEN - a;
-                a++;
-            }
-            b = a + rem;
-        }
+    for (int blk = t; blk < NEN * NEN; blk += 64) {
+        const int a = blk / NEN, b = blk % NEN;
         double Kab[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
         if (!sGeneral) {
             for (int g = 0; g < NGP; g++) {
@@ -373,19 +365,6 @@ __global__ __launch_bounds__(64) void k_assemble(const int *__restrict__ elems, 
                 }
             }
         }
-        if (kbuf) {
-            double *o = kbuf + ((size_t)e * NEN * NEN + a * NEN + b) * 9;
-#pragma unroll
-            for (int k = 0; k < 9; k++) o[k] = Kab[k];
-            if (a != b) {
-                double *ot = kbuf + ((size_t)e * NEN * NEN + b * NEN + a) * 9;
-#pragma unroll
-                for (int i = 0; i < 3; i++)
-#pragma unroll
-                    for (int j = 0; j < 3; j++) ot[3 * j + i] = Kab[3 * i + j];
-            }
-            continue;
-        }
         const int off = eoff[((size_t)e * NEN + a) * NEN + b];
         if (off == 0xFFFF) continue;
 #pragma unroll
@@ -401,76 +380,6 @@ __global__ __launch_bounds__(64) void k_assemble(const int *__restrict__ elems, 
                 rnk++;
             }
         }
-    }
-}
-
-// The rows of node n from the stored element blocks.  The node's element
-// list (element * NEN + local node a, ascending element) is taken 64 / NEN
-// elements at a time; lane (slot, b) loads the block (a, b) of its element
-// with its row offset (eoff) and column dofs, so that all loads of a pass are
-// in flight together.  The slots then add into the LDS rows one after the
-// other, in ascending element order, and each of the node's rows is written
-// once.  One wave per node; the node's rows share one column list of length
-// <= ASM_LMAX.
-constexpr int ASM_LMAX = 256;
-template <int NEN>
-__global__ __launch_bounds__(64) void k_assemble_gather(int nnode, const int *__restrict__ nptr,
-                                                        const int *__restrict__ nadj, const int *__restrict__ conn,
-                                                        const int *__restrict__ eqn, const uint16_t *__restrict__ eoff,
-                                                        const double *__restrict__ kbuf,
-                                                        const int32_t *__restrict__ rowptr, double *__restrict__ val)
-{
-    static_assert(64 % NEN == 0, "element slots per pass");
-    constexpr int SLOTS = 64 / NEN;
-    __shared__ double sR[3][ASM_LMAX];
-    const int n = blockIdx.x;
-    if (n >= nnode) return;
-    const int t = threadIdx.x, k = t / NEN, b = t % NEN;
-    int q[3];
-#pragma unroll
-    for (int i = 0; i < 3; i++) q[i] = eqn[3 * (size_t)n + i];
-    const int r0 = q[0] > 0 ? q[0] : q[1] > 0 ? q[1] : q[2];
-    if (r0 <= 0) return;   // no free dof: no rows
-    const int L = rowptr[r0] - rowptr[r0 - 1];
-    for (int p = t; p < L; p += 64) sR[0][p] = sR[1][p] = sR[2][p] = 0.0;
-    const int j0 = nptr[n], cnt = nptr[n + 1] - j0;
-    for (int base = 0; base < cnt; base += SLOTS) {
-        const int slot = base + k;
-        double v[9];
-        int pos[3] = {-1, -1, -1};
-        if (slot < cnt) {
-            const int ea = nadj[j0 + slot], e = ea / NEN, a = ea % NEN;
-            const int off = eoff[((size_t)e * NEN + a) * NEN + b];
-            const int nb = conn[(size_t)e * NEN + b];
-            const double *src = kbuf + (((size_t)e * NEN + a) * NEN + b) * 9;
-#pragma unroll
-            for (int x = 0; x < 9; x++) v[x] = src[x];
-            if (off != 0xFFFF) {
-                int r = 0;
-#pragma unroll
-                for (int j = 0; j < 3; j++)
-                    if (eqn[3 * (size_t)nb + j] > 0) pos[j] = off + r++;
-            }
-        }
-        __syncthreads();
-        for (int s = 0; s < SLOTS; s++) {
-            if (k == s) {
-#pragma unroll
-                for (int i = 0; i < 3; i++) {
-                    if (q[i] <= 0) continue;
-#pragma unroll
-                    for (int j = 0; j < 3; j++)
-                        if (pos[j] >= 0) sR[i][pos[j]] += v[3 * i + j];
-                }
-            }
-            __syncthreads();
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-        if (q[i] <= 0) continue;
-        double *row = val + rowptr[q[i] - 1];
-        for (int p = t; p < L; p += 64) row[p] = sR[i][p];
     }
 }
 
@@ -1461,11 +1370,7 @@ struct hfem_model {
     // element, and the element force vectors of one evaluation
     int *d_fnptr = nullptr, *d_fnadj = nullptr;
     double *d_fbuf = nullptr;
-    // stiffness assembly by rows (LSpace): the element blocks of one
-    // assembly (64 x 9 doubles per element) and the longest row
-    double *d_kbuf = nullptr;
-    bool kbuf_failed = false;
-    int max_rowlen = 0;
+    int max_rowlen = 0;          // longest row of the stiffness
     // per element and k_mf_hex lane g: first free equation (0-based, bits
     // 0..28) and free-dof mask (bits 29..31) of the lane's node; built once
     // per mesh when every node numbers its free dofs consecutively
@@ -1502,7 +1407,7 @@ static int model_free(hfem_model *md)
     void *ps[] = {md->d_coords, md->d_mat, md->d_state, md->d_conn, md->d_emat, md->d_eqn, md->d_bad,
                   md->d_eoff,   md->d_colors, md->d_uf, md->d_up, md->d_ff, md->d_fp, md->d_out3, md->d_dofid,
                   md->d_tdesc, md->d_nptr, md->d_nadj, md->d_ebuf, md->d_ecolor, md->d_eqmask, md->d_yslot,
-                  md->d_erel, md->d_eloc, md->d_fnptr, md->d_fnadj, md->d_fbuf, md->d_kbuf};
+                  md->d_erel, md->d_eloc, md->d_fnptr, md->d_fnadj, md->d_fbuf};
     for (void *p : ps)
         if (p) HIPFEM_CHECK(hipFree(p));
     md->d_tdesc = nullptr;
@@ -1516,8 +1421,6 @@ static int model_free(hfem_model *md)
     md->eloc_checked = false;
     md->d_fnptr = md->d_fnadj = nullptr;
     md->d_fbuf = nullptr;
-    md->d_kbuf = nullptr;
-    md->kbuf_failed = false;
     md->max_rowlen = 0;
     md->d_coords = md->d_mat = md->d_state = md->d_uf = md->d_up = md->d_ff = md->d_fp = md->d_out3 = nullptr;
     md->d_conn = md->d_emat = md->d_eqn = md->d_bad = md->d_colors = nullptr;
@@ -1825,29 +1728,33 @@ extern "C" int hfem_model_assemble_stiffness(hfem_model *md, hipcsr_mtx *K, int 
     hipStream_t st = md->ctx->stream;
     int rc = reset_bad(md);
     if (rc) return rc;
-    // LSpace by rows: every element's blocks stored in one launch, then each
-    // node's rows summed in ascending element order and written once (no
-    // read-modify-write of partial lines); else one launch per color adding
-    // into the zeroed values
-    bool by_rows = md->etype == HIPFEM_LSPACE && md->nelem > 0 && md->max_rowlen <= ASM_LMAX && !md->kbuf_failed;
+    // LSpace and LTRSpace by rows: a node's elements' blocks are formed by the
+    // wave that writes its rows, each once, in ascending element order.
+    // Other elements, and meshes with a row longer than the column codes hold
+    // (hundreds of elements at one node), go color by color, adding into the
+    // zeroed values.
+    const bool hex = md->etype == HIPFEM_LSPACE;
+    const bool by_rows = (hex || md->etype == HIPFEM_LTRSPACE) && md->nelem > 0 && md->max_rowlen <= ASM_LMAX;
     if (by_rows) {
         rc = node_adjacency(md);
         if (rc) return rc;
-        if (!md->d_kbuf && hipMalloc(&md->d_kbuf, sizeof(double) * 64 * 9 * (size_t)md->nelem) != hipSuccess) {
-            (void)hipGetLastError();   // the colored form needs no buffer
-            md->d_kbuf = nullptr;
-            md->kbuf_failed = true;
-            by_rows = false;
+        const AsmArgs A = {md->nnode, md->nelem, md->d_fnptr, md->d_fnadj, md->d_conn, md->d_eqn, md->d_emat,
+                           md->d_coords, md->d_mat, md->d_eoff, md->d_state, md->ngp_total,
+                           md->sur ? md->d_sflag : nullptr, md->d_dsur, K->d_rowptr, K->d_val, md->d_bad};
+        const bool tan = md->has_mises && mode == 1;
+#define LAUNCH_ROWS(TAN, SUR)                                                                                    \
+    if (hex)                                                                                                     \
+        k_assemble_rows_hex<TAN, SUR><<<(md->nnode + 1) / 2, 64, 16 * (size_t)md->max_rowlen, st>>>(A);          \
+    else                                                                                                         \
+        k_assemble_rows_tet<TAN, SUR><<<md->nnode, 64, 16 * (size_t)md->max_rowlen, st>>>(A)
+        if (tan && A.sflag) {
+            LAUNCH_ROWS(true, true);
+        } else if (tan) {
+            LAUNCH_ROWS(true, false);
+        } else {
+            LAUNCH_ROWS(false, false);
         }
-    }
-    if (by_rows) {
-        k_assemble<HIPFEM_LSPACE><<<md->nelem, 64, 0, st>>>(nullptr, md->nelem, md->d_coords, md->d_conn, md->d_eqn,
-                                                            md->d_emat, md->d_mat, md->d_eoff, md->d_state,
-                                                            md->ngp_total, mode, K->d_rowptr, K->d_val, md->d_bad,
-                                                            md->sur ? md->d_sflag : nullptr, md->d_dsur, md->d_kbuf);
-        HIPFEM_CHECK(hipGetLastError());
-        k_assemble_gather<8><<<md->nnode, 64, 0, st>>>(md->nnode, md->d_fnptr, md->d_fnadj, md->d_conn, md->d_eqn,
-                                                       md->d_eoff, md->d_kbuf, K->d_rowptr, K->d_val);
+#undef LAUNCH_ROWS
         HIPFEM_CHECK(hipGetLastError());
         K->h_stage.clear();   // every value was written: what hipcsr_zero resets
         K->staged = false;
@@ -1862,7 +1769,7 @@ extern "C" int hfem_model_assemble_stiffness(hfem_model *md, hipcsr_mtx *K, int 
 #define LAUNCH_ASM(ET)                                                                                              \
     k_assemble<ET><<<n, 64, 0, st>>>(el, n, md->d_coords, md->d_conn, md->d_eqn, md->d_emat, md->d_mat, md->d_eoff, \
                                      md->d_state, md->ngp_total, mode, K->d_rowptr, K->d_val, md->d_bad,     \
-                                     md->sur ? md->d_sflag : nullptr, md->d_dsur, nullptr)
+                                     md->sur ? md->d_sflag : nullptr, md->d_dsur)
         if (md->etype == HIPFEM_LSPACE) LAUNCH_ASM(HIPFEM_LSPACE);
         else if (md->etype == HIPFEM_LTRSPACE) LAUNCH_ASM(HIPFEM_LTRSPACE);
         else LAUNCH_ASM(HIPFEM_QSPACE);

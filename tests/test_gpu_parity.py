@@ -579,3 +579,67 @@ def test_pcg_multiple_right_hand_sides(ctx, precision):
         assert r <= 5 * tol, (j, r)
     assert not X[:, 7].any()
     s.close()
+
+
+def _row_form_deck(kind):
+    """Meshes at the edges of the assembly by rows: every node's elements
+    repeated (more elements at a node than one pass takes), random partly
+    fixed nodes, a node without elements, an odd node count, and a star whose
+    centre row is longer than the row form takes (the color form)."""
+    rng = np.random.default_rng(11)
+    hexes = kind.startswith("hex")
+    if kind.endswith("star"):
+        m, nen = 60, 8 if hexes else 4
+        ref = meshgen._rve_mesh(1, meshgen.LSPACE) if hexes else meshgen.kuhn_tets(1, 1, 1, 1.0, 1.0, 1.0)
+        conn0, xyz = ref[1][0], ref[0]
+        coords, conn = [xyz[conn0[0]]], np.zeros((m, nen), np.int64)
+        for e in range(m):
+            s = 1.0 + 0.2 * rng.random()
+            for a in range(1, nen):
+                conn[e, a] = len(coords)
+                coords.append(xyz[conn0[0]] + s * (xyz[conn0[a]] - xyz[conn0[0]]))
+        coords = np.array(coords)
+    else:
+        if hexes:
+            b = meshgen.cantilever_hex(3, 2, 4, jitter=0.2, seed=4)
+            coords, conn = b.coords, b.conn
+        else:
+            coords, conn = meshgen.kuhn_tets(3, 2, 4, 1.0, 1.0, 1.0, jitter=0.1, seed=4)
+        conn = np.concatenate([conn] * ((3 if hexes else 2) if kind.endswith("repeated") else 1))
+        coords = np.concatenate([coords, [[9.0, 9.0, 9.0]]])
+        if len(coords) % 2 == 0:
+            coords = np.concatenate([coords, [[9.0, 9.0, 8.0]]])
+    bc = rng.random((len(coords), 3)) < (0.02 if kind.endswith("star") else 0.2)
+    mat = np.array([[meshgen.MAT_MISES, 210e3, 0.3, 250.0, 2e3, 0, 0, 0],
+                    [meshgen.MAT_ISOLE, 70e3, 0.2, 0, 0, 0, 0, 0]])
+    return meshgen.Deck(kind, meshgen.LSPACE if hexes else meshgen.LTRSPACE, coords, conn,
+                        (rng.random(len(conn)) < 0.2).astype(np.int32), mat, bc, np.zeros_like(coords))
+
+
+@pytest.mark.parametrize("tangent", [False, True])
+@pytest.mark.parametrize("kind", ["hex_partial", "hex_repeated", "hex_star", "tet_partial", "tet_repeated", "tet_star"])
+def test_row_assembly_edges_match_oracle(ctx, kind, tangent):
+    """The row form (and the color form behind it) against the oracle, with
+    the tolerances of the plain meshes: 1e-13 of the largest entry for the
+    elastic matrix, 1e-12 for the tangent of a plastic state; the second
+    assembly into the same matrix gives the same bits."""
+    from oofem_amd.hipfem import BatchedEvaluator, HipCSRSparseMtrx
+    d = _row_form_deck(kind)
+    ev = BatchedEvaluator(ctx, d)
+    K = HipCSRSparseMtrx(ctx)
+    ev.build_structure(K)
+    st = oracle.state_new(d)
+    if tangent:
+        u = np.random.default_rng(5).standard_normal(d.neq) * 4e-3
+        ev.internal_forces(u, np.zeros(d.npeq), update_state=True)
+        oracle.internal_forces(d, u, np.zeros(d.npeq), state=st, update_state=True)
+        assert (st.reshape(-1, 38)[:, 13] > 0).any()
+    rp, ci, val = oracle.csr(d, state=st, tangent=tangent)
+    for _ in range(2):
+        ev.assemble_stiffness(K, tangent=tangent)
+        grp, gci, gval = K.download()
+        np.testing.assert_array_equal(grp, rp)
+        np.testing.assert_array_equal(gci, ci)
+        assert np.abs(gval - val).max() <= (1e-12 if tangent else 1e-13) * np.abs(val).max()
+        assert _ == 0 or np.array_equal(gval, first)
+        first = gval
