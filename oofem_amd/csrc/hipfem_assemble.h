@@ -1,5 +1,7 @@
-// Stiffness assembly by rows: one wave per node recomputes the blocks
-// B_a^T D B_b of its elements and writes the node's rows once.
+// Stiffness assembly by rows, each written once, in ascending element order:
+// for LSpace and LTRSpace the wave that writes a node's rows forms the blocks
+// B_a^T D B_b of its elements on the spot, for QSpace it sums stored element
+// matrices.
 // Included by hipfem_model.hip (after the element rules).
 #pragma once
 
@@ -524,6 +526,168 @@ __global__ __launch_bounds__(64) void k_assemble_rows_tet(AsmArgs A)
         }
         wave_lds_fence();
         rows_sum_columns<12>(t, q, L, sV, sCodes, A.rowptr, A.val, base == 0);
+    }
+}
+
+// K_e of every QSpace element, 60 x 60 row-major: 256 threads an element.
+// The (point, node) pairs, the 9 entries of every point's J and the 210 node
+// pairs a <= b are each shared out over the threads; a block is stored with
+// its transpose, so every element matrix is exactly symmetric.
+//
+// Bound: LDS reads of the gradients (7 doubles a pair and point, 15 with the
+// tangent).  9,261 elements: 0.157 ms and 0.153 ms for the rows summed from
+// them (267 MB each way); eight color launches of one wave an element, which
+// leave a SIMD one wave, took 0.78 ms.
+template <bool TAN, bool SUR>
+__global__ __launch_bounds__(256) void k_element_matrices_quad(AsmArgs A, double *__restrict__ kbuf)
+{
+    constexpr int NGP = 27, NEN = 20;
+    __shared__ double sX[60];
+    __shared__ double sN[NGP][60];    // dN/dxi, then dN/dx
+    __shared__ double sJ[NGP][9];     // J, then J^-1
+    __shared__ double sQ[NGP][TAN ? 10 : 2];   // dV (< 0: surrogate D), [cd, kd, M (6)]
+    const int e = blockIdx.x, t = threadIdx.x;
+    for (int k = t; k < 60; k += 256) sX[k] = A.coords[3 * (size_t)A.conn[(size_t)e * NEN + k / 3] + k % 3];
+    for (int k = t; k < NGP * NEN; k += 256) {
+        double xi[3], w, d[3];
+        gauss_point(HIPFEM_QSPACE, k / NEN, xi, w);
+        dndxi_hexquad(k % NEN, xi, d);
+#pragma unroll
+        for (int j = 0; j < 3; j++) sN[k / NEN][3 * (k % NEN) + j] = d[j];
+    }
+    __syncthreads();
+    if (t < NGP * 9) {
+        const int g = t / 9, i = t % 9 / 3, j = t % 3;
+        double v = 0.0;
+#pragma unroll 4
+        for (int a = 0; a < NEN; a++) v += sX[3 * a + i] * sN[g][3 * a + j];
+        sJ[g][3 * i + j] = v;
+    }
+    __syncthreads();
+    const double *mp = A.mat + (size_t)HIPFEM_MATP * A.emat[e];
+    if (t < NGP) {
+        double J[9], I[9], xi[3], w;
+        gauss_point(HIPFEM_QSPACE, t, xi, w);
+#pragma unroll
+        for (int i = 0; i < 9; i++) J[i] = sJ[t][i];
+        I[0] = J[4] * J[8] - J[5] * J[7];
+        I[1] = J[2] * J[7] - J[1] * J[8];
+        I[2] = J[1] * J[5] - J[2] * J[4];
+        I[3] = J[5] * J[6] - J[3] * J[8];
+        I[4] = J[0] * J[8] - J[2] * J[6];
+        I[5] = J[2] * J[3] - J[0] * J[5];
+        I[6] = J[3] * J[7] - J[4] * J[6];
+        I[7] = J[1] * J[6] - J[0] * J[7];
+        I[8] = J[0] * J[4] - J[1] * J[3];
+        const double det = J[0] * I[0] + J[1] * I[3] + J[2] * I[6];
+        if (!(fabs(det) > 1.e-30)) atomicMin(A.bad, e);
+        const double id = 1. / det, dV = fabs(det) * w;
+#pragma unroll
+        for (int i = 0; i < 9; i++) sJ[t][i] = I[i] * id;
+        sQ[t][0] = dV;
+        if constexpr (TAN) {
+            const size_t gp = (size_t)e * NGP + t;
+            double cd, kd, m[6];
+            point_parts(mp, dV, load_point(A.state, A.ngp_total, gp), cd, kd, m);
+            sQ[t][1] = cd;
+            sQ[t][2] = kd;
+#pragma unroll
+            for (int i = 0; i < 6; i++) sQ[t][3 + i] = m[i];
+            if (SUR && A.sflag[gp]) sQ[t][0] = -dV;
+        }
+    }
+    __syncthreads();
+    for (int k = t; k < NGP * NEN; k += 256) {
+        const int g = k / NEN, a = k % NEN;
+        const double d0 = sN[g][3 * a], d1 = sN[g][3 * a + 1], d2 = sN[g][3 * a + 2];
+#pragma unroll
+        for (int j = 0; j < 3; j++) sN[g][3 * a + j] = d0 * sJ[g][j] + d1 * sJ[g][3 + j] + d2 * sJ[g][6 + j];
+    }
+    __syncthreads();
+    if (t >= NEN * (NEN + 1) / 2) return;
+    int a = 0, rem = t;
+    while (rem >= NEN - a) rem -= NEN - a++;
+    const int b = a + rem;
+    const double G = mp[1] / (2.0 * (1. + mp[2]));
+    const double lam = mp[1] / (3.0 * (1. - 2. * mp[2])) - 2.0 * G / 3.0;
+    double K[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll 3
+    for (int g = 0; g < NGP; g++) {
+        const double n[3] = {sN[g][3 * a], sN[g][3 * a + 1], sN[g][3 * a + 2]};
+        const double m[3] = {sN[g][3 * b], sN[g][3 * b + 1], sN[g][3 * b + 2]};
+        if constexpr (TAN) {
+            if (SUR && sQ[g][0] < 0.0) {
+                add_general(n, m, -sQ[g][0], A.dsur, A.ngp_total, (size_t)e * NGP + g, K);
+            } else {
+                double va[3], vb[3];
+                tensor_times(&sQ[g][3], n, va);
+                tensor_times(&sQ[g][3], m, vb);
+                add_parts(n, m, sQ[g][1], sQ[g][2], va, vb, K);
+            }
+        } else {
+            add_elastic(n, m, lam, G, sQ[g][0], K);
+        }
+    }
+    double *o = kbuf + (size_t)e * 3600;
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) o[(3 * a + i) * 60 + 3 * b + j] = K[3 * i + j];
+    if (a != b) {
+#pragma unroll
+        for (int j = 0; j < 3; j++)
+#pragma unroll
+            for (int i = 0; i < 3; i++) o[(3 * b + j) * 60 + 3 * a + i] = K[3 * i + j];
+    }
+}
+
+// The rows of node n from the stored element matrices: eight elements a pass,
+// whose three rows (3 x 3 NEN contiguous doubles) go to LDS as they lie; the
+// columns are then summed and written once.  One wave per node.
+template <int NEN>
+__global__ __launch_bounds__(64) void k_assemble_gather(AsmArgs A, const double *__restrict__ kbuf)
+{
+    constexpr int NC = 3 * NEN, ROW2 = 3 * NC / 2;   // 16-byte words of an element's three rows
+    __shared__ __align__(16) double sV[8 * 3 * NC + 2];
+    extern __shared__ __align__(16) unsigned char sDyn[];
+    uint64_t *sCodes = reinterpret_cast<uint64_t *>(sDyn);
+    const int n = blockIdx.x;
+    if (n >= A.nnode) return;
+    const int t = threadIdx.x;
+    if (t == 0) sV[8 * 3 * NC] = 0.0;
+    int q[3];
+#pragma unroll
+    for (int i = 0; i < 3; i++) q[i] = A.eqn[3 * (size_t)n + i];
+    const int r0 = q[0] > 0 ? q[0] : q[1] > 0 ? q[1] : q[2];
+    if (r0 <= 0) return;   // no free dof: no rows
+    const int L = A.rowptr[r0] - A.rowptr[r0 - 1];
+    const int j0 = A.nptr[n], cnt = A.nptr[n + 1] - j0;
+    for (int base = 0; base < cnt; base += 8) {
+        const int ns = min(8, cnt - base);
+        d2_t v[(8 * ROW2 + 63) / 64];
+#pragma unroll
+        for (int u = 0; u < (8 * ROW2 + 63) / 64; u++) {
+            const int idx = u * 64 + t, s = min(idx / ROW2, ns - 1);
+            v[u] = reinterpret_cast<const d2_t *>(kbuf + (size_t)A.nadj[j0 + base + s] * (3 * NC))[idx % ROW2];
+        }
+        clear_codes<8>(t, L, sCodes);
+        uint8_t *bytes = reinterpret_cast<uint8_t *>(sCodes);
+        for (int i = t; i < ns * NEN; i += 64) {
+            const int s = i / NEN, b = i % NEN, ea = A.nadj[j0 + base + s];
+            const int off = A.eoff[(size_t)ea * NEN + b];
+            const int nb = A.conn[(size_t)(ea / NEN) * NEN + b];
+            int r = 0;
+#pragma unroll
+            for (int j = 0; j < 3; j++)
+                if (A.eqn[3 * (size_t)nb + j] > 0 && off != 0xFFFF) bytes[(off + r++) * 8 + s] = (uint8_t)(3 * b + j);
+        }
+#pragma unroll
+        for (int u = 0; u < (8 * ROW2 + 63) / 64; u++) {
+            const int idx = u * 64 + t;
+            if (idx / ROW2 < ns) reinterpret_cast<d2_t *>(sV)[idx] = v[u];
+        }
+        wave_lds_fence();
+        rows_sum_entries<NC>(t, q[0], q[1], q[2], L, sV, 8 * 3 * NC, sCodes, A.rowptr, A.val, base == 0);
     }
 }
 

@@ -29,7 +29,7 @@
 //                    scattering it.  IsoLE uses the closed form
 //                    lambda n_i m_j + G (n_j m_i + delta_ij n.m); MisesMat
 //                    the parts c I_dev + K 1x1 - m m^T of its tangent.
-//   k_internal<ET>   one thread per Gauss point: geometry, strain B u_e, the
+//   k_internal*      one thread per Gauss point: geometry, strain B u_e, the
 //                    material update (radial return for MisesMat), B^T sigma dV
 //                    into LDS; then per element the Gauss-point sums in
 //                    ascending order are stored, and k_gather_nodal sums them
@@ -548,54 +548,191 @@ __global__ __launch_bounds__(256) void k_sur_classify(int nelem, const double *_
 }
 
 // -------------------------------------------------------- internal forces
+// elements per block of the internal-force kernels
 template <int ET>
 struct IntCfg {
-    static constexpr int NGP = ElemT<ET>::NGP;
-    static constexpr int EPB = (NGP >= 64) ? 1 : 64 / NGP;  // elements per 64-thread block
+    static constexpr int EPB = ET == HIPFEM_LSPACE ? 8 : ET == HIPFEM_LTRSPACE ? 64 : 9;
 };
 
-template <int ET>
-__global__ __launch_bounds__(64) void k_internal(const int *__restrict__ elems, int nelem_color,
-                                                 const double *__restrict__ coords, const int *__restrict__ conn,
-                                                 const int *__restrict__ eqn, const int *__restrict__ emat,
-                                                 const double *__restrict__ mat, const double *__restrict__ u_free,
-                                                 const double *__restrict__ u_presc, double *__restrict__ state,
-                                                 int ngp_total, int update_state, double *__restrict__ f_free,
-                                                 double *__restrict__ f_presc, double *__restrict__ fbuf,
-                                                 double *__restrict__ partials, int npart, int *__restrict__ bad,
-                                                 int op, SurArgs sur)
+// what one internal-force evaluation reads and writes
+struct IntArgs {
+    int nelem;
+    const double *coords;
+    const int *conn, *eqn, *emat;
+    const double *mat, *u_free, *u_presc;
+    double *state;
+    int ngp_total, update_state;
+    double *fbuf;       // element force vectors, NC per element, for k_gather_nodal
+    double *partials;   // per block and dof id: squared element forces (npart blocks)
+    int npart;
+    int *bad;
+    SurArgs sur;
+};
+
+__device__ __forceinline__ double dof_value(int q, const double *u_free, const double *u_presc)
 {
-    // elems == nullptr: every element, ei = e.  fbuf: the element force
-    // vectors are stored (NC per element) for k_gather_nodal, else added to
-    // f_free / f_presc (one color per launch)
-    constexpr int NEN = ElemT<ET>::NEN, NGP = ElemT<ET>::NGP, EPB = IntCfg<ET>::EPB, NC = 3 * NEN;
-    __shared__ double sF[EPB][NGP][NC];
+    return (q > 0 && u_free) ? u_free[q - 1] : ((q < 0 && u_presc) ? u_presc[-q - 1] : 0.0);
+}
+
+// Stress of one Gauss point.  OP 0: the material update (with the surrogate's
+// predictions where SUR) and, on request, the temp state; OP 1 / 2: the
+// product with the elastic / TangentStiffness D of the current temp state, so
+// that sum_g B^T D B u_e dV = K_e u_e.
+template <int OP, bool SUR>
+__device__ __forceinline__ void point_stress(const IntArgs &A, const double *mp, size_t gp, const double eps[6],
+                                             unsigned int *scount, double sig[6])
+{
+    const double E = mp[1], nu = mp[2];
+    double *__restrict__ state = A.state;
+    const size_t ngp_total = A.ngp_total;
+    if constexpr (OP != 0) {
+        double D[36], s[6];
+        if ((int)mp[0] == HIPFEM_MAT_MISES && OP == 2) {
+#pragma unroll
+            for (int i = 0; i < 6; i++) s[i] = state[(14 + i) * ngp_total + gp];
+            mises_tangent(E, nu, mp[3], mp[4], state[6 * ngp_total + gp], state[13 * ngp_total + gp], s, D);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 6; i++) s[i] = 0.0;
+            mises_tangent(E, nu, 0.0, 0.0, 0.0, 0.0, s, D);   // dKappa = 0: elastic D
+        }
+#pragma unroll
+        for (int r = 0; r < 6; r++) {
+            double v = 0.0;
+#pragma unroll
+            for (int c = 0; c < 6; c++) v += D[6 * r + c] * eps[c];
+            sig[r] = v;
+        }
+        return;
+    }
+    if ((int)mp[0] == HIPFEM_MAT_MISES) {
+        double epsp_n[6];
+#pragma unroll
+        for (int i = 0; i < 6; i++) epsp_n[i] = state[i * ngp_total + gp];
+        const double kappa_n = state[6 * ngp_total + gp];
+        MisesOut o;
+        bool used = false;
+        if constexpr (SUR) {
+            const SurArgs &sur = A.sur;
+            const int sl = sur.slot[gp];
+            if (sl >= 0) {
+                used = surrogate_update(E, nu, mp[3], mp[4], eps, epsp_n, kappa_n, sur.y + (size_t)27 * sl,
+                                        sur.sig_scale, sur.tan_scale, sur.tol, o);
+                atomicAdd(&scount[used ? 0 : 1], 1u);
+            }
+            if (A.update_state) {
+                sur.flag[gp] = used ? 1 : 0;
+                // a point rejected once keeps the plain update for the rest of the
+                // step, so accept/reject switches cannot repeat inside Newton
+                if (sl >= 0 && !used) sur.rejected[gp] = 1;
+                if (used) {
+                    const float *yy = sur.y + (size_t)27 * sl + 6;
+#pragma unroll
+                    for (int k = 0; k < 21; k++)
+                        sur.dsur[(size_t)k * ngp_total + gp] =
+                            (float)(elastic_upper(E, nu, k) - (double)yy[k] / (double)sur.tan_scale);
+                }
+            }
+        }
+        if (!used) mises_return(E, nu, mp[3], mp[4], eps, epsp_n, kappa_n, o);
+#pragma unroll
+        for (int i = 0; i < 6; i++) sig[i] = o.sig[i];
+        if (A.update_state) {
+#pragma unroll
+            for (int i = 0; i < 6; i++) {
+                state[(7 + i) * ngp_total + gp] = o.epsp[i];
+                state[(14 + i) * ngp_total + gp] = o.sdev[i];
+            }
+            state[13 * ngp_total + gp] = o.kappa;
+        }
+    } else {
+        // IsoLE: sigma = (2G I_dev6 + K I6_I6) eps
+        const double G = E / (2.0 * (1. + nu));
+        const double K = E / (3.0 * (1. - 2. * nu));
+        const double lam = K - 2.0 * G / 3.0;
+        const double tr = eps[0] + eps[1] + eps[2];
+        sig[0] = lam * tr + 2.0 * G * eps[0];
+        sig[1] = lam * tr + 2.0 * G * eps[1];
+        sig[2] = lam * tr + 2.0 * G * eps[2];
+        sig[3] = G * eps[3];
+        sig[4] = G * eps[4];
+        sig[5] = G * eps[5];
+    }
+    if (A.update_state) {
+#pragma unroll
+        for (int i = 0; i < 6; i++) {
+            state[(20 + i) * ngp_total + gp] = sig[i];
+            state[(26 + i) * ngp_total + gp] = eps[i];
+        }
+    }
+}
+
+// The block's element forces from its points' (sF: element, point, component,
+// rows of NC + 1 against bank conflicts; ascending points) into fbuf, and its partial squared norms per dof id
+template <int EPB, int NGP, int NC>
+__device__ __forceinline__ void store_element_forces(const IntArgs &A, int t, const double *sF, double *sh)
+{
+    double n3[3] = {0, 0, 0};
+    for (int idx = t; idx < EPB * NC; idx += 64) {
+        const int l = idx / NC, c = idx % NC, e = blockIdx.x * EPB + l;
+        if (e >= A.nelem) continue;
+        double f = 0.0;
+#pragma unroll
+        for (int g = 0; g < NGP; g++) f += sF[(l * NGP + g) * (NC + 1) + c];
+        A.fbuf[(size_t)e * NC + c] = f;
+        n3[c % 3] += f * f;
+    }
+    if (A.partials) {
+        for (int k = 0; k < 3; k++) {
+            double v = n3[k];
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+            if (t == 0) sh[k] = v;
+        }
+        if (t == 0)
+            for (int k = 0; k < 3; k++) A.partials[(size_t)k * A.npart + blockIdx.x] = sh[k];
+    }
+}
+
+template <bool SUR>
+__device__ __forceinline__ void add_sur_counts(const IntArgs &A, int t, const unsigned int *scount)
+{
+    if constexpr (SUR)
+        if (A.sur.counts && t == 0 && (scount[0] | scount[1])) {
+            atomicAdd(&A.sur.counts[0], (unsigned long long)scount[0]);
+            atomicAdd(&A.sur.counts[1], (unsigned long long)scount[1]);
+        }
+}
+
+// LTRSpace: one thread per element (its one Gauss point)
+template <int OP, bool SUR>
+__global__ __launch_bounds__(64) void k_internal_tet(IntArgs A)
+{
+    constexpr int ET = HIPFEM_LTRSPACE, NEN = 4, NGP = 1, EPB = IntCfg<ET>::EPB, NC = 3 * NEN;
+    __shared__ double sF[EPB * NGP * (NC + 1)];
     __shared__ double sh[3];
     __shared__ unsigned int scount[2];
     if (threadIdx.x < 2) scount[threadIdx.x] = 0;
     __syncthreads();
     const int t = threadIdx.x;
     const int el = t / NGP, g = t % NGP;
-    const int ei = blockIdx.x * EPB + el;
-    const bool active = (el < EPB) && (ei < nelem_color);
-    if (active) {
-        const int e = elems ? elems[ei] : ei;
+    const int e = blockIdx.x * EPB + el;
+    if (el < EPB && e < A.nelem) {
         double X[NC], ue[NC];
         for (int a = 0; a < NEN; a++) {
-            const int node = conn[(size_t)e * NEN + a];
+            const int node = A.conn[(size_t)e * NEN + a];
 #pragma unroll
             for (int d = 0; d < 3; d++) {
-                X[3 * a + d] = coords[3 * (size_t)node + d];
-                const int q = eqn[3 * (size_t)node + d];
-                ue[3 * a + d] = (q > 0 && u_free) ? u_free[q - 1] : ((q < 0 && u_presc) ? u_presc[-q - 1] : 0.0);
+                X[3 * a + d] = A.coords[3 * (size_t)node + d];
+                ue[3 * a + d] = dof_value(A.eqn[3 * (size_t)node + d], A.u_free, A.u_presc);
             }
         }
         double xi[3], w, detJ, dNdx[NC];
         gauss_point(ET, g, xi, w);
-        if (!gp_geometry<ET>(X, xi, dNdx, detJ)) atomicMin(bad, e);
+        if (!gp_geometry<ET>(X, xi, dNdx, detJ)) atomicMin(A.bad, e);
         const double dV = fabs(detJ) * w;
         // strain = B u_e (Voigt xx yy zz yz xz xy, engineering shear)
-        double eps[6] = {0, 0, 0, 0, 0, 0};
+        double eps[6] = {0, 0, 0, 0, 0, 0}, sig[6];
         for (int a = 0; a < NEN; a++) {
             const double nx = dNdx[3 * a], ny = dNdx[3 * a + 1], nz = dNdx[3 * a + 2];
             const double ux = ue[3 * a], uy = ue[3 * a + 1], uz = ue[3 * a + 2];
@@ -606,177 +743,267 @@ __global__ __launch_bounds__(64) void k_internal(const int *__restrict__ elems, 
             eps[4] += nz * ux + nx * uz;
             eps[5] += ny * ux + nx * uy;
         }
-        const double *mp = mat + (size_t)HIPFEM_MATP * emat[e];
-        const double E = mp[1], nu = mp[2];
-        const size_t gp = (size_t)e * NGP + g;
-        double sig[6];
-        if (op != 0) {
-            // tangent product: sigma = D eps with D the elastic (op 1) or the
-            // TangentStiffness (op 2) matrix of the current temp state, so that
-            // sum_g B^T D B u_e dV = K_e u_e
-            double D[36], s[6];
-            if ((int)mp[0] == HIPFEM_MAT_MISES && op == 2) {
-#pragma unroll
-                for (int i = 0; i < 6; i++) s[i] = state[(size_t)(14 + i) * ngp_total + gp];
-                mises_tangent(E, nu, mp[3], mp[4], state[(size_t)6 * ngp_total + gp],
-                              state[(size_t)13 * ngp_total + gp], s, D);
-            } else {
-#pragma unroll
-                for (int i = 0; i < 6; i++) s[i] = 0.0;
-                mises_tangent(E, nu, 0.0, 0.0, 0.0, 0.0, s, D);   // dKappa = 0: elastic D
-            }
-#pragma unroll
-            for (int r = 0; r < 6; r++) {
-                double v = 0.0;
-#pragma unroll
-                for (int c = 0; c < 6; c++) v += D[6 * r + c] * eps[c];
-                sig[r] = v;
-            }
-        } else if ((int)mp[0] == HIPFEM_MAT_MISES) {
-            double epsp_n[6];
-#pragma unroll
-            for (int i = 0; i < 6; i++) epsp_n[i] = state[(size_t)i * ngp_total + gp];
-            const double kappa_n = state[(size_t)6 * ngp_total + gp];
-            MisesOut o;
-            bool used = false;
-            if (sur.slot) {
-                const int sl = sur.slot[gp];
-                if (sl >= 0) {
-                    used = surrogate_update(E, nu, mp[3], mp[4], eps, epsp_n, kappa_n, sur.y + (size_t)27 * sl,
-                                            sur.sig_scale, sur.tan_scale, sur.tol, o);
-                    atomicAdd(&scount[used ? 0 : 1], 1u);
-                }
-                if (update_state) {
-                    sur.flag[gp] = used ? 1 : 0;
-                    // a point rejected once keeps the plain update for the rest of the
-                    // step, so accept/reject switches cannot repeat inside Newton
-                    if (sl >= 0 && !used) sur.rejected[gp] = 1;
-                    if (used) {
-                        const float *yy = sur.y + (size_t)27 * sl + 6;
-#pragma unroll
-                        for (int k = 0; k < 21; k++)
-                            sur.dsur[(size_t)k * ngp_total + gp] =
-                                (float)(elastic_upper(E, nu, k) - (double)yy[k] / (double)sur.tan_scale);
-                    }
-                }
-            }
-            if (!used) mises_return(E, nu, mp[3], mp[4], eps, epsp_n, kappa_n, o);
-#pragma unroll
-            for (int i = 0; i < 6; i++) sig[i] = o.sig[i];
-            if (update_state) {
-#pragma unroll
-                for (int i = 0; i < 6; i++) {
-                    state[(size_t)(7 + i) * ngp_total + gp] = o.epsp[i];
-                    state[(size_t)(14 + i) * ngp_total + gp] = o.sdev[i];
-                }
-                state[(size_t)13 * ngp_total + gp] = o.kappa;
-            }
-        } else {
-            // IsoLE: sigma = (2G I_dev6 + K I6_I6) eps
-            const double G = E / (2.0 * (1. + nu));
-            const double K = E / (3.0 * (1. - 2. * nu));
-            const double lam = K - 2.0 * G / 3.0;
-            const double tr = eps[0] + eps[1] + eps[2];
-            sig[0] = lam * tr + 2.0 * G * eps[0];
-            sig[1] = lam * tr + 2.0 * G * eps[1];
-            sig[2] = lam * tr + 2.0 * G * eps[2];
-            sig[3] = G * eps[3];
-            sig[4] = G * eps[4];
-            sig[5] = G * eps[5];
-        }
-        if (update_state && op == 0) {
-#pragma unroll
-            for (int i = 0; i < 6; i++) {
-                state[(size_t)(20 + i) * ngp_total + gp] = sig[i];
-                state[(size_t)(26 + i) * ngp_total + gp] = eps[i];
-            }
-        }
+        point_stress<OP, SUR>(A, A.mat + (size_t)HIPFEM_MATP * A.emat[e], (size_t)e * NGP + g, eps, scount, sig);
         // B^T sigma dV
+        double *f = sF + (el * NGP + g) * (NC + 1);
         for (int a = 0; a < NEN; a++) {
             const double nx = dNdx[3 * a], ny = dNdx[3 * a + 1], nz = dNdx[3 * a + 2];
-            sF[el][g][3 * a + 0] = (nx * sig[0] + nz * sig[4] + ny * sig[5]) * dV;
-            sF[el][g][3 * a + 1] = (ny * sig[1] + nz * sig[3] + nx * sig[5]) * dV;
-            sF[el][g][3 * a + 2] = (nz * sig[2] + ny * sig[3] + nx * sig[4]) * dV;
+            f[3 * a + 0] = (nx * sig[0] + nz * sig[4] + ny * sig[5]) * dV;
+            f[3 * a + 1] = (ny * sig[1] + nz * sig[3] + nx * sig[5]) * dV;
+            f[3 * a + 2] = (nz * sig[2] + ny * sig[3] + nx * sig[4]) * dV;
         }
     }
     __syncthreads();
-    if (sur.counts && t == 0 && (scount[0] | scount[1])) {
-        atomicAdd(&sur.counts[0], (unsigned long long)scount[0]);
-        atomicAdd(&sur.counts[1], (unsigned long long)scount[1]);
+    add_sur_counts<SUR>(A, t, scount);
+    store_element_forces<EPB, NGP, NC>(A, t, sF, sh);
+}
+
+// LSpace: 8 elements a wave, lane (el, g) is Gauss point g of element el and
+// loads node g's coordinates and displacements, which the element's lanes
+// share through LDS (10 loads a lane instead of 80).  Strain and force go
+// through the local gradients, du/dx = (sum_a u_a dN_a/dxi) J^-1 and f_a =
+// (dV sigma J^-T) dN_a/dxi, so that no lane holds the 24 dN/dx.
+//
+// Bound: the 7 state values read and 25 written a point, 2.15 GB on the
+// 64x64x256 block: 0.62 ms (3.8 TB/s with the element forces).  With every
+// lane loading its element's eight nodes and holding the 24 dN/dx, 198 VGPRs
+// left two waves a SIMD: 1.04 ms.
+template <int OP, bool SUR>
+__global__ __launch_bounds__(64) void k_internal_hex(IntArgs A)
+{
+    __shared__ double sF[64 * 25];      // first: the nodes' coordinates and displacements
+    __shared__ double sh[3];
+    __shared__ unsigned int scount[2];
+    const int t = threadIdx.x, el = t >> 3, g = t & 7;
+    if constexpr (SUR) {
+        if (t < 2) scount[t] = 0;
+        __syncthreads();
     }
-    double n3[3] = {0, 0, 0};
-    for (int idx = t; idx < EPB * NC; idx += 64) {
-        const int l = idx / NC, c = idx % NC;
-        const int ej = blockIdx.x * EPB + l;
-        if (ej >= nelem_color) continue;
-        const int e = elems ? elems[ej] : ej;
-        double f = 0.0;
-        for (int gg = 0; gg < NGP; gg++) f += sF[l][gg][c];
-        if (fbuf) {
-            fbuf[(size_t)e * NC + c] = f;
-        } else {
-            const int node = conn[(size_t)e * NEN + c / 3];
-            const int q = eqn[3 * (size_t)node + c % 3];
-            if (q > 0 && f_free) f_free[q - 1] += f;
-            if (q < 0 && f_presc) f_presc[-q - 1] += f;
-        }
-        n3[c % 3] += f * f;
-    }
-    // block partial of the EBE norms (fixed order)
-    if (partials) {
-        for (int k = 0; k < 3; k++) {
-            double v = n3[k];
+    const int ei = blockIdx.x * 8 + el;
+    const bool active = ei < A.nelem;
+    const int e = active ? ei : A.nelem - 1;   // spare lanes of the last block load the last element
+    {
+        const int node = A.conn[(size_t)e * 8 + g];
 #pragma unroll
-            for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-            if (t == 0) sh[k] = v;
+        for (int d = 0; d < 3; d++) {
+            sF[(d * 8 + g) * 8 + el] = A.coords[3 * (size_t)node + d];
+            sF[((3 + d) * 8 + g) * 8 + el] = dof_value(A.eqn[3 * (size_t)node + d], A.u_free, A.u_presc);
         }
-        if (t == 0)
-            for (int k = 0; k < 3; k++) partials[(size_t)k * npart + blockIdx.x] = sh[k];
     }
+    wave_lds_fence();
+    const double ga = 0.577350269189626;   // gauss_point
+    const double xi = (g & 4) ? ga : -ga, eta = (g & 2) ? ga : -ga, ze = (g & 1) ? ga : -ga;
+    const double xm = 1. - xi, xp = 1. + xi, ym = 1. - eta, yp = 1. + eta, zm = 1. - ze, zp = 1. + ze;
+    const double yz[4] = {0.125 * ym * zm, 0.125 * ym * zp, 0.125 * yp * zm, 0.125 * yp * zp};
+    const double xz[4] = {0.125 * xm * zm, 0.125 * xm * zp, 0.125 * xp * zm, 0.125 * xp * zp};
+    const double xy[4] = {0.125 * xm * ym, 0.125 * xm * yp, 0.125 * xp * ym, 0.125 * xp * yp};
+    auto dndxi = [&](int a, double dN[3]) {   // dndxi_hexlin at the lane's point
+        const int bx = (a & 3) >= 2, by = (a & 3) == 1 || (a & 3) == 2, bz = a < 4;
+        dN[0] = bx ? yz[2 * by + bz] : -yz[2 * by + bz];
+        dN[1] = by ? xz[2 * bx + bz] : -xz[2 * bx + bz];
+        dN[2] = bz ? xy[2 * bx + by] : -xy[2 * bx + by];
+    };
+    double J[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, gu[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int a = 0; a < 8; a++) {
+        double dN[3];
+        dndxi(a, dN);
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const double x = sF[(i * 8 + a) * 8 + el], u = sF[((3 + i) * 8 + a) * 8 + el];
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                J[3 * i + j] += x * dN[j];
+                gu[3 * i + j] += u * dN[j];
+            }
+        }
+    }
+    double I[9];   // J^-1: the cofactors times one reciprocal
+    I[0] = J[4] * J[8] - J[5] * J[7];
+    I[1] = J[2] * J[7] - J[1] * J[8];
+    I[2] = J[1] * J[5] - J[2] * J[4];
+    I[3] = J[5] * J[6] - J[3] * J[8];
+    I[4] = J[0] * J[8] - J[2] * J[6];
+    I[5] = J[2] * J[3] - J[0] * J[5];
+    I[6] = J[3] * J[7] - J[4] * J[6];
+    I[7] = J[1] * J[6] - J[0] * J[7];
+    I[8] = J[0] * J[4] - J[1] * J[3];
+    const double det = J[0] * I[0] + J[1] * I[3] + J[2] * I[6];
+    if (active && !(fabs(det) > 1.e-30)) atomicMin(A.bad, e);
+    const double id = 1. / det, dV = fabs(det);   // the rule's weights are 1
+#pragma unroll
+    for (int i = 0; i < 9; i++) I[i] *= id;
+    double H[9];   // du_i/dx_j
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) H[3 * i + j] = gu[3 * i] * I[j] + gu[3 * i + 1] * I[3 + j] + gu[3 * i + 2] * I[6 + j];
+    const double eps[6] = {H[0], H[4], H[8], H[5] + H[7], H[2] + H[6], H[1] + H[3]};
+    double sig[6] = {0, 0, 0, 0, 0, 0};
+    if (active) point_stress<OP, SUR>(A, A.mat + (size_t)HIPFEM_MATP * A.emat[e], (size_t)e * 8 + g, eps, scount, sig);
+    const double S[9] = {sig[0], sig[5], sig[4], sig[5], sig[1], sig[3], sig[4], sig[3], sig[2]};
+    double T[9];   // dV sigma J^-T
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+            T[3 * i + k] = dV * (S[3 * i] * I[3 * k] + S[3 * i + 1] * I[3 * k + 1] + S[3 * i + 2] * I[3 * k + 2]);
+    wave_lds_fence();   // the nodes' values have been read
+#pragma unroll
+    for (int a = 0; a < 8; a++) {
+        double dN[3];
+        dndxi(a, dN);
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+            sF[t * 25 + 3 * a + i] = T[3 * i] * dN[0] + T[3 * i + 1] * dN[1] + T[3 * i + 2] * dN[2];
+    }
+    __syncthreads();
+    add_sur_counts<SUR>(A, t, scount);
+    store_element_forces<8, 8, 24>(A, t, sF, sh);
+}
+
+// QSpace: nine elements a block, thread (el, g) is Gauss point g of element
+// el.  The derivatives dN/dxi at the 27 points are formed once a block in
+// LDS; strain and force go through the local gradients as in k_internal_hex,
+// the forces summed over the points straight from T = dV sigma J^-T.
+//
+// Bound: LDS reads.  9,261 elements: 0.040 ms; one wave an element with 27 of
+// 64 lanes at work and 400 registers a lane took 0.106 ms.
+template <int OP, bool SUR>
+__global__ __launch_bounds__(256) void k_internal_quad(IntArgs A)
+{
+    constexpr int NEN = 20, NGP = 27, EPB = IntCfg<HIPFEM_QSPACE>::EPB, NT = NGP + 1;
+    __shared__ double sN[60][NT];          // dN_a/dxi_k at point g: row 3 a + k
+    __shared__ double sX[EPB][2][60];      // coordinates, displacements
+    __shared__ double sT[EPB][9][NT];
+    __shared__ double sh[4][3];
+    __shared__ unsigned int scount[2];
+    const int t = threadIdx.x, el = t / NGP, g = t % NGP;
+    if (t < 2) scount[t] = 0;
+    for (int k = t; k < NGP * NEN; k += 256) {
+        double xi[3], w, d[3];
+        gauss_point(HIPFEM_QSPACE, k % NGP, xi, w);
+        dndxi_hexquad(k / NGP, xi, d);
+#pragma unroll
+        for (int j = 0; j < 3; j++) sN[3 * (k / NGP) + j][k % NGP] = d[j];
+    }
+    for (int k = t; k < EPB * 60; k += 256) {
+        const int e = blockIdx.x * EPB + k / 60;
+        if (e >= A.nelem) break;
+        const size_t dof = 3 * (size_t)A.conn[(size_t)e * NEN + k % 60 / 3] + k % 3;
+        sX[k / 60][0][k % 60] = A.coords[dof];
+        sX[k / 60][1][k % 60] = dof_value(A.eqn[dof], A.u_free, A.u_presc);
+    }
+    __syncthreads();
+    const int e = blockIdx.x * EPB + el;
+    if (el < EPB && e < A.nelem) {
+        double J[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, gu[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll 2
+        for (int a = 0; a < NEN; a++) {
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                const double d = sN[3 * a + j][g];
+#pragma unroll
+                for (int i = 0; i < 3; i++) {
+                    J[3 * i + j] += sX[el][0][3 * a + i] * d;
+                    gu[3 * i + j] += sX[el][1][3 * a + i] * d;
+                }
+            }
+        }
+        double I[9], xi[3], w;   // J^-1: the cofactors times one reciprocal
+        gauss_point(HIPFEM_QSPACE, g, xi, w);
+        I[0] = J[4] * J[8] - J[5] * J[7];
+        I[1] = J[2] * J[7] - J[1] * J[8];
+        I[2] = J[1] * J[5] - J[2] * J[4];
+        I[3] = J[5] * J[6] - J[3] * J[8];
+        I[4] = J[0] * J[8] - J[2] * J[6];
+        I[5] = J[2] * J[3] - J[0] * J[5];
+        I[6] = J[3] * J[7] - J[4] * J[6];
+        I[7] = J[1] * J[6] - J[0] * J[7];
+        I[8] = J[0] * J[4] - J[1] * J[3];
+        const double det = J[0] * I[0] + J[1] * I[3] + J[2] * I[6];
+        if (!(fabs(det) > 1.e-30)) atomicMin(A.bad, e);
+        const double id = 1. / det, dV = fabs(det) * w;
+#pragma unroll
+        for (int i = 0; i < 9; i++) I[i] *= id;
+        double H[9];   // du_i/dx_j
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int j = 0; j < 3; j++)
+                H[3 * i + j] = gu[3 * i] * I[j] + gu[3 * i + 1] * I[3 + j] + gu[3 * i + 2] * I[6 + j];
+        const double eps[6] = {H[0], H[4], H[8], H[5] + H[7], H[2] + H[6], H[1] + H[3]};
+        double sig[6];
+        point_stress<OP, SUR>(A, A.mat + (size_t)HIPFEM_MATP * A.emat[e], (size_t)e * NGP + g, eps, scount, sig);
+        const double S[9] = {sig[0], sig[5], sig[4], sig[5], sig[1], sig[3], sig[4], sig[3], sig[2]};
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+                sT[el][3 * i + k][g] =
+                    dV * (S[3 * i] * I[3 * k] + S[3 * i + 1] * I[3 * k + 1] + S[3 * i + 2] * I[3 * k + 2]);
+    }
+    __syncthreads();
+    add_sur_counts<SUR>(A, t, scount);
+    double n3[3] = {0, 0, 0};
+    for (int k = t; k < EPB * 60; k += 256) {
+        const int l = k / 60, a = k % 60 / 3, i = k % 3, eo = blockIdx.x * EPB + l;
+        if (eo >= A.nelem) break;
+        double f = 0.0;
+#pragma unroll 3
+        for (int p = 0; p < NGP; p++)
+            f += sT[l][3 * i][p] * sN[3 * a][p] + sT[l][3 * i + 1][p] * sN[3 * a + 1][p] +
+                 sT[l][3 * i + 2][p] * sN[3 * a + 2][p];
+        A.fbuf[(size_t)eo * 60 + k % 60] = f;
+        n3[0] += i == 0 ? f * f : 0.0;
+        n3[1] += i == 1 ? f * f : 0.0;
+        n3[2] += i == 2 ? f * f : 0.0;
+    }
+    if (!A.partials) return;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) n3[i] += __shfl_xor(n3[i], off, 64);
+        if (t % 64 == 0) sh[t / 64][i] = n3[i];
+    }
+    __syncthreads();
+    if (t < 3) A.partials[(size_t)t * A.npart + blockIdx.x] = sh[0][t] + sh[1][t] + sh[2][t] + sh[3][t];
 }
 
 // f per dof = the sum of the stored element force vectors over the elements
-// at the node, FP64, in the fixed order of the node's list (nptr / nadj:
-// element * nen + local node, ascending element); one thread per node
-__global__ void k_gather_nodal(int nnode, int nen, const int *__restrict__ nptr, const int *__restrict__ nadj,
-                               const int *__restrict__ eqn, const double *__restrict__ fbuf,
-                               double *__restrict__ f_free, double *__restrict__ f_presc)
+// at the node (nptr / nadj: element * nen + local node), FP64, in a fixed
+// order: eight lanes a node, lane l adding entries l, l + 8, ... of the list,
+// then the lanes pairwise.  A line of fbuf serves several neighbouring nodes, so
+// each XCD takes a contiguous run of them.  Bound: the forces read, 231 MB on
+// the 70x70x82 tetrahedral block: 0.105 ms (one thread a node 0.168, without
+// the XCD order 0.122); 201 MB on the 64x64x256 block: 0.105 ms (0.104, 0.117).
+__global__ __launch_bounds__(256) void k_gather_nodal(int nnode, int nen, const int *__restrict__ nptr,
+                                                      const int *__restrict__ nadj, const int *__restrict__ eqn,
+                                                      const double *__restrict__ fbuf, double *__restrict__ f_free,
+                                                      double *__restrict__ f_presc)
 {
-    for (int n = blockIdx.x * blockDim.x + threadIdx.x; n < nnode; n += gridDim.x * blockDim.x) {
-        double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+    const int l = threadIdx.x & 7;
+    // gridDim.x is a multiple of 8
+    const int b = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    for (int n = b * 32 + threadIdx.x / 8; n < nnode; n += gridDim.x * 32) {
+        double s[3] = {0.0, 0.0, 0.0};
         const int j1 = nptr[n + 1];
-        int j = nptr[n];
-        // four list entries' loads in flight before their sums (same order)
-        for (; j + 4 <= j1; j += 4) {
-            double v[4][3];
+        for (int j = nptr[n] + l; j < j1; j += 8) {
+            const double *f = fbuf + 3 * (size_t)nadj[j];
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const int ea = nadj[j + k];
-                const double *f = fbuf + (size_t)(ea / nen) * 3 * nen + 3 * (ea % nen);
-                v[k][0] = f[0];
-                v[k][1] = f[1];
-                v[k][2] = f[2];
-            }
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                s0 += v[k][0];
-                s1 += v[k][1];
-                s2 += v[k][2];
-            }
+            for (int d = 0; d < 3; d++) s[d] += f[d];
         }
-        for (; j < j1; j++) {
-            const int ea = nadj[j];
-            const double *f = fbuf + (size_t)(ea / nen) * 3 * nen + 3 * (ea % nen);
-            s0 += f[0];
-            s1 += f[1];
-            s2 += f[2];
-        }
-        const double sv[3] = {s0, s1, s2};
 #pragma unroll
         for (int d = 0; d < 3; d++) {
-            const int q = eqn[3 * (size_t)n + d];
-            if (q > 0 && f_free) f_free[q - 1] = sv[d];
-            if (q < 0 && f_presc) f_presc[-q - 1] = sv[d];
+            s[d] += __shfl_xor(s[d], 1, 8);
+            s[d] += __shfl_xor(s[d], 2, 8);
+            s[d] += __shfl_xor(s[d], 4, 8);
+        }
+        if (l < 3) {
+            const int q = eqn[3 * (size_t)n + l];
+            const double v = l == 0 ? s[0] : l == 1 ? s[1] : s[2];
+            if (q > 0 && f_free) f_free[q - 1] = v;
+            if (q < 0 && f_presc) f_presc[-q - 1] = v;
         }
     }
 }
@@ -1206,22 +1433,29 @@ __global__ void k_zero_f32(int64_t n, float *__restrict__ a)
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) a[i] = 0.f;
 }
 
+// out[k] = sum of partials[k np .. k np + np), block k; eight loads of a thread
+// in flight before their adds (one block for all three, one load at a time,
+// took 168 us for the 3 x 131,072 partials of the 64x64x256 block)
 __global__ __launch_bounds__(1024) void k_reduce3(const double *__restrict__ partials, int np, double *out)
 {
     __shared__ double sh[16];
-    for (int k = 0; k < 3; k++) {
-        double s = 0.0;
-        for (int i = threadIdx.x; i < np; i += 1024) s += partials[(size_t)k * np + i];
+    const double *p = partials + (size_t)blockIdx.x * np;
+    double s = 0.0;
+    for (int i0 = threadIdx.x; i0 < np; i0 += 8 * 1024) {
+        double v[8];
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-        if (threadIdx.x % 64 == 0) sh[threadIdx.x / 64] = s;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            double tt = 0.0;
-            for (int i = 0; i < 16; i++) tt += sh[i];
-            out[k] = tt;
-        }
-        __syncthreads();
+        for (int j = 0; j < 8; j++) v[j] = i0 + j * 1024 < np ? p[i0 + j * 1024] : 0.0;
+#pragma unroll
+        for (int j = 0; j < 8; j++) s += v[j];
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if (threadIdx.x % 64 == 0) sh[threadIdx.x / 64] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = 0.0;
+        for (int i = 0; i < 16; i++) t += sh[i];
+        out[blockIdx.x] = t;
     }
 }
 
@@ -1370,7 +1604,11 @@ struct hfem_model {
     // element, and the element force vectors of one evaluation
     int *d_fnptr = nullptr, *d_fnadj = nullptr;
     double *d_fbuf = nullptr;
-    int max_rowlen = 0;          // longest row of the stiffness
+    // stiffness assembly by rows: the QSpace element matrices of one assembly
+    // (60 x 60 doubles per element) and the longest row
+    double *d_kbuf = nullptr;
+    bool kbuf_failed = false;
+    int max_rowlen = 0;
     // per element and k_mf_hex lane g: first free equation (0-based, bits
     // 0..28) and free-dof mask (bits 29..31) of the lane's node; built once
     // per mesh when every node numbers its free dofs consecutively
@@ -1407,7 +1645,7 @@ static int model_free(hfem_model *md)
     void *ps[] = {md->d_coords, md->d_mat, md->d_state, md->d_conn, md->d_emat, md->d_eqn, md->d_bad,
                   md->d_eoff,   md->d_colors, md->d_uf, md->d_up, md->d_ff, md->d_fp, md->d_out3, md->d_dofid,
                   md->d_tdesc, md->d_nptr, md->d_nadj, md->d_ebuf, md->d_ecolor, md->d_eqmask, md->d_yslot,
-                  md->d_erel, md->d_eloc, md->d_fnptr, md->d_fnadj, md->d_fbuf};
+                  md->d_erel, md->d_eloc, md->d_fnptr, md->d_fnadj, md->d_fbuf, md->d_kbuf};
     for (void *p : ps)
         if (p) HIPFEM_CHECK(hipFree(p));
     md->d_tdesc = nullptr;
@@ -1421,6 +1659,8 @@ static int model_free(hfem_model *md)
     md->eloc_checked = false;
     md->d_fnptr = md->d_fnadj = nullptr;
     md->d_fbuf = nullptr;
+    md->d_kbuf = nullptr;
+    md->kbuf_failed = false;
     md->max_rowlen = 0;
     md->d_coords = md->d_mat = md->d_state = md->d_uf = md->d_up = md->d_ff = md->d_fp = md->d_out3 = nullptr;
     md->d_conn = md->d_emat = md->d_eqn = md->d_bad = md->d_colors = nullptr;
@@ -1728,16 +1968,25 @@ extern "C" int hfem_model_assemble_stiffness(hfem_model *md, hipcsr_mtx *K, int 
     hipStream_t st = md->ctx->stream;
     int rc = reset_bad(md);
     if (rc) return rc;
-    // LSpace and LTRSpace by rows: a node's elements' blocks are formed by the
-    // wave that writes its rows, each once, in ascending element order.
-    // Other elements, and meshes with a row longer than the column codes hold
-    // (hundreds of elements at one node), go color by color, adding into the
-    // zeroed values.
-    const bool hex = md->etype == HIPFEM_LSPACE;
-    const bool by_rows = (hex || md->etype == HIPFEM_LTRSPACE) && md->nelem > 0 && md->max_rowlen <= ASM_LMAX;
+    // By rows: for LSpace and LTRSpace the wave that writes a node's rows forms
+    // its elements' blocks; for QSpace, where a block takes 27 points, the
+    // element matrices are stored first.  Meshes with a row longer than the
+    // column codes hold (hundreds of elements at one node), and QSpace meshes
+    // whose matrices (28.8 KB an element) do not fit in memory, go color by
+    // color, adding into the zeroed values.
+    const bool hex = md->etype == HIPFEM_LSPACE, quad = md->etype == HIPFEM_QSPACE;
+    bool by_rows = md->nelem > 0 && md->max_rowlen <= ASM_LMAX && !(quad && md->kbuf_failed);
     if (by_rows) {
         rc = node_adjacency(md);
         if (rc) return rc;
+        if (quad && !md->d_kbuf && hipMalloc(&md->d_kbuf, sizeof(double) * 3600 * (size_t)md->nelem) != hipSuccess) {
+            (void)hipGetLastError();   // the colored form needs no buffer
+            md->d_kbuf = nullptr;
+            md->kbuf_failed = true;
+            by_rows = false;
+        }
+    }
+    if (by_rows) {
         const AsmArgs A = {md->nnode, md->nelem, md->d_fnptr, md->d_fnadj, md->d_conn, md->d_eqn, md->d_emat,
                            md->d_coords, md->d_mat, md->d_eoff, md->d_state, md->ngp_total,
                            md->sur ? md->d_sflag : nullptr, md->d_dsur, K->d_rowptr, K->d_val, md->d_bad};
@@ -1745,6 +1994,8 @@ extern "C" int hfem_model_assemble_stiffness(hfem_model *md, hipcsr_mtx *K, int 
 #define LAUNCH_ROWS(TAN, SUR)                                                                                    \
     if (hex)                                                                                                     \
         k_assemble_rows_hex<TAN, SUR><<<(md->nnode + 1) / 2, 64, 16 * (size_t)md->max_rowlen, st>>>(A);          \
+    else if (quad)                                                                                               \
+        k_element_matrices_quad<TAN, SUR><<<md->nelem, 256, 0, st>>>(A, md->d_kbuf);                             \
     else                                                                                                         \
         k_assemble_rows_tet<TAN, SUR><<<md->nnode, 64, 16 * (size_t)md->max_rowlen, st>>>(A)
         if (tan && A.sflag) {
@@ -1756,6 +2007,10 @@ extern "C" int hfem_model_assemble_stiffness(hfem_model *md, hipcsr_mtx *K, int 
         }
 #undef LAUNCH_ROWS
         HIPFEM_CHECK(hipGetLastError());
+        if (quad) {
+            k_assemble_gather<20><<<md->nnode, 64, 8 * (size_t)md->max_rowlen, st>>>(A, md->d_kbuf);
+            HIPFEM_CHECK(hipGetLastError());
+        }
         K->h_stage.clear();   // every value was written: what hipcsr_zero resets
         K->staged = false;
     } else {
@@ -2045,23 +2300,34 @@ static int internal_dev(hfem_model *md, const double *uf, const double *up, doub
         // every element in one launch (the Gauss-point state is read and
         // written in whole lines), each storing its force vector; then one
         // FP64 sum per node in the fixed order of its element list
-#define LAUNCH_INT(ET)                                                                                              \
-    k_internal<ET><<<npart, 64, 0, st>>>(nullptr, md->nelem, md->d_coords, md->d_conn, md->d_eqn, md->d_emat,        \
-                                         md->d_mat, uf, up, md->d_state, md->ngp_total, update, nullptr, nullptr,    \
-                                         md->d_fbuf, part, npart, md->d_bad, op, sur)
-        if (md->etype == HIPFEM_LSPACE) LAUNCH_INT(HIPFEM_LSPACE);
-        else if (md->etype == HIPFEM_LTRSPACE) LAUNCH_INT(HIPFEM_LTRSPACE);
-        else LAUNCH_INT(HIPFEM_QSPACE);
+        const IntArgs A = {md->nelem, md->d_coords, md->d_conn, md->d_eqn, md->d_emat, md->d_mat, uf, up, md->d_state,
+                           md->ngp_total, update, md->d_fbuf, ebe3 ? part : nullptr, npart, md->d_bad, sur};
+#define LAUNCH_INT(OP, SUR)                                              \
+    if (md->etype == HIPFEM_LSPACE)                                      \
+        k_internal_hex<OP, SUR><<<npart, 64, 0, st>>>(A);                \
+    else if (md->etype == HIPFEM_LTRSPACE)                               \
+        k_internal_tet<OP, SUR><<<npart, 64, 0, st>>>(A);                \
+    else                                                                 \
+        k_internal_quad<OP, SUR><<<npart, 256, 0, st>>>(A)
+        if (op == 1) {
+            LAUNCH_INT(1, false);
+        } else if (op == 2) {
+            LAUNCH_INT(2, false);
+        } else if (sur.slot) {
+            LAUNCH_INT(0, true);
+        } else {
+            LAUNCH_INT(0, false);
+        }
 #undef LAUNCH_INT
         HIPFEM_CHECK(hipGetLastError());
         if (ff || fp) {
-            k_gather_nodal<<<std::min(8192, (md->nnode + 255) / 256), 256, 0, st>>>(
+            k_gather_nodal<<<std::min(65536, (md->nnode + 255) / 256 * 8), 256, 0, st>>>(
                 md->nnode, md->nen, md->d_fnptr, md->d_fnadj, md->d_eqn, md->d_fbuf, ff, fp);
             HIPFEM_CHECK(hipGetLastError());
         }
     }
     if (ebe3) {
-        k_reduce3<<<1, 1024, 0, st>>>(part, npart, md->d_out3);
+        k_reduce3<<<3, 1024, 0, st>>>(part, npart, md->d_out3);
         HIPFEM_CHECK(hipGetLastError());
         HIPFEM_CHECK(hipMemcpyAsync(ebe3, md->d_out3, 3 * sizeof(double), hipMemcpyDeviceToHost, st));
     }

@@ -588,6 +588,14 @@ def _row_form_deck(kind):
     centre row is longer than the row form takes (the color form)."""
     rng = np.random.default_rng(11)
     hexes = kind.startswith("hex")
+    mat = np.array([[meshgen.MAT_MISES, 210e3, 0.3, 250.0, 2e3, 0, 0, 0],
+                    [meshgen.MAT_ISOLE, 70e3, 0.2, 0, 0, 0, 0, 0]])
+    if kind.startswith("quad"):
+        coords, conn = meshgen._rve_mesh(2, meshgen.QSPACE)
+        coords = np.concatenate([coords + 0.02 * rng.standard_normal(coords.shape), [[9.0, 9.0, 9.0]]])
+        conn = np.concatenate([conn] * (2 if kind.endswith("repeated") else 1))
+        return meshgen.Deck(kind, meshgen.QSPACE, coords, conn, (rng.random(len(conn)) < 0.2).astype(np.int32), mat,
+                            rng.random((len(coords), 3)) < 0.2, np.zeros_like(coords))
     if kind.endswith("star"):
         m, nen = 60, 8 if hexes else 4
         ref = meshgen._rve_mesh(1, meshgen.LSPACE) if hexes else meshgen.kuhn_tets(1, 1, 1, 1.0, 1.0, 1.0)
@@ -610,14 +618,13 @@ def _row_form_deck(kind):
         if len(coords) % 2 == 0:
             coords = np.concatenate([coords, [[9.0, 9.0, 8.0]]])
     bc = rng.random((len(coords), 3)) < (0.02 if kind.endswith("star") else 0.2)
-    mat = np.array([[meshgen.MAT_MISES, 210e3, 0.3, 250.0, 2e3, 0, 0, 0],
-                    [meshgen.MAT_ISOLE, 70e3, 0.2, 0, 0, 0, 0, 0]])
     return meshgen.Deck(kind, meshgen.LSPACE if hexes else meshgen.LTRSPACE, coords, conn,
                         (rng.random(len(conn)) < 0.2).astype(np.int32), mat, bc, np.zeros_like(coords))
 
 
 @pytest.mark.parametrize("tangent", [False, True])
-@pytest.mark.parametrize("kind", ["hex_partial", "hex_repeated", "hex_star", "tet_partial", "tet_repeated", "tet_star"])
+@pytest.mark.parametrize("kind", ["hex_partial", "hex_repeated", "hex_star", "tet_partial", "tet_repeated", "tet_star",
+                                  "quad_partial", "quad_repeated"])
 def test_row_assembly_edges_match_oracle(ctx, kind, tangent):
     """The row form (and the color form behind it) against the oracle, with
     the tolerances of the plain meshes: 1e-13 of the largest entry for the
@@ -632,8 +639,12 @@ def test_row_assembly_edges_match_oracle(ctx, kind, tangent):
     if tangent:
         u = np.random.default_rng(5).standard_normal(d.neq) * 4e-3
         ev.internal_forces(u, np.zeros(d.npeq), update_state=True)
-        oracle.internal_forces(d, u, np.zeros(d.npeq), state=st, update_state=True)
-        assert (st.reshape(-1, 38)[:, 13] > 0).any()
+        assert (ev.get_state()[:, 13] > 0).any()
+        f, fp, ebe = ev.internal_forces(u, np.zeros(d.npeq))
+        fo, fpo, ebeo = oracle.internal_forces(d, u, np.zeros(d.npeq), state=st, update_state=True)
+        for a, b in ((f, fo), (fp, fpo)):
+            assert np.abs(a - b).max() <= 1e-12 * np.abs(fo).max()
+        np.testing.assert_allclose(ebe, ebeo, rtol=1e-12)
     rp, ci, val = oracle.csr(d, state=st, tangent=tangent)
     for _ in range(2):
         ev.assemble_stiffness(K, tangent=tangent)
