@@ -17,8 +17,7 @@
 // each path starts virgin and takes 1..maxsteps Gaussian increments of
 // every Voigt strain component; every step is one sample.
 // Training: mean-squared error over the 27 scaled outputs, Adam, batches
-// drawn with replacement by a counter-based hash; forward and backward are
-// the FP32 kernels below (tiled GEMM with fused bias/SiLU epilogues).
+// drawn with replacement by a counter-based hash; three FP32 launches a step.
 // Inference: BF16 operands on MFMA (v_mfma_f32_32x32x16_bf16) with FP32
 // accumulation, weights staged in LDS in operand order.
 
@@ -42,7 +41,7 @@ constexpr int OFF_B3 = OFF_W3 + MLP_H * MLP_H;
 constexpr int OFF_W4 = OFF_B3 + MLP_H;
 constexpr int OFF_B4 = OFF_W4 + MLP_OUT * MLP_H;
 constexpr int MLP_NPARAM = OFF_B4 + MLP_OUT;
-constexpr int MLP_SPLITK = 32;   // weight-gradient slabs (workspace MLP_SPLITK x 128 x 128)
+constexpr int MLP_SLABS = 64;   // most weight-gradient slabs of a batch
 
 // --------------------------------------------------------------- hashing RNG
 __host__ __device__ inline uint64_t mix64(uint64_t x)
@@ -105,171 +104,336 @@ __global__ void k_mlp_paths(int64_t npaths, const int64_t *__restrict__ off, int
 }
 
 // ------------------------------------------------------------- FP32 kernels
+// A training step is three launches: k_mlp_step (forward and backward of the
+// batch, 16 rows a workgroup), k_mlp_wgrad (weight-gradient slabs over the
+// rows) and k_mlp_apply (slabs summed, Adam).  All products run on the FP32
+// matrix instructions (FP32 operands and accumulation).
+//
+// Besides the parameters the device holds copies that the products can read
+// along their contiguous dimension: W1 padded to 16 columns, and W2, W3, W4
+// transposed (W4's rows padded to 32).
+constexpr int AUX_W1 = 0;                        // 128 x 16
+constexpr int AUX_T2 = AUX_W1 + MLP_H * 16;      // 128 x 128: [in][out]
+constexpr int AUX_T3 = AUX_T2 + MLP_H * MLP_H;
+constexpr int AUX_T4 = AUX_T3 + MLP_H * MLP_H;   // 128 x 32: [in][out]
+constexpr int MLP_NAUX = AUX_T4 + MLP_H * 32;
+
+// where parameter i has a copy (-1: a bias)
+__device__ __forceinline__ int aux_of(int i)
+{
+    if (i < OFF_B1) return AUX_W1 + (i / MLP_IN) * 16 + i % MLP_IN;
+    if (i >= OFF_W2 && i < OFF_B2) return AUX_T2 + (i - OFF_W2) % MLP_H * MLP_H + (i - OFF_W2) / MLP_H;
+    if (i >= OFF_W3 && i < OFF_B3) return AUX_T3 + (i - OFF_W3) % MLP_H * MLP_H + (i - OFF_W3) / MLP_H;
+    if (i >= OFF_W4 && i < OFF_B4) return AUX_T4 + (i - OFF_W4) % MLP_H * 32 + (i - OFF_W4) / MLP_H;
+    return -1;
+}
+
+__global__ void k_zero_pad(int n, float *__restrict__ a)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) a[i] = 0.f;
+}
+
+__global__ void k_mlp_aux(const float *__restrict__ p, float *__restrict__ aux)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= MLP_NPARAM) return;
+    const int j = aux_of(i);
+    if (j >= 0) aux[j] = p[i];
+}
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((__vector_size__(16 * sizeof(float))));
+
 __device__ __forceinline__ float sigmoidf_(float z) { return 1.f / (1.f + expf(-z)); }
 
-// C[M x N] = sum_k A(m,k) B(k,n) with A(m,k) = A[m*sam + k*sak] and
-// B(k,n) = B[k*sbk + n*sbn]; 64x64 tiles, 16-deep K slices, 4x4 outputs per
-// thread; every output is one thread's fixed-order sum (deterministic).
-// EPI 0: C = acc; 1: Z = acc + bias, C = silu(Z); 2: C = acc + bias.
-template <int EPI>
-__global__ __launch_bounds__(256) void k_gemm(int M, int N, int K, const float *__restrict__ A, int64_t sam,
-                                              int64_t sak, const float *__restrict__ B, int64_t sbk, int64_t sbn,
-                                              const float *__restrict__ bias, float *__restrict__ C, int64_t ldc,
-                                              float *__restrict__ Z)
+constexpr int TR = 16;            // batch rows per workgroup of k_mlp_step
+constexpr int TLD = MLP_H + 4;    // LDS row of an activation tile
+
+// acc += A (16 rows in LDS, row stride TLD) times the 16 columns whose
+// operand rows b holds: lane (c, q) of b is the row of column c, entries
+// [4 NV q, 4 NV (q + 1)); the four lane groups take the four quarters of the
+// inner dimension, so both operands are read 16 bytes at a time
+template <int NV>
+__device__ __forceinline__ f32x4 tile_product(const float *sA, const f32x4 b[NV], int c, int q, f32x4 acc)
 {
-    __shared__ float As[16][65];
-    __shared__ float Bs[16][65];
-    const int tm = threadIdx.x / 16, tn = threadIdx.x % 16;
-    const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-    // split K: slice z of gridDim.z sums k in [kb, ke) into its own C slab
-    const int kc = (((K + gridDim.z - 1) / gridDim.z) + 15) / 16 * 16;
-    const int kb = blockIdx.z * kc, ke = min(K, kb + kc);
-    C += (int64_t)blockIdx.z * M * ldc;
-    float acc[4][4];
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int v = 0; v < NV; v++) {
+        const f32x4 a = *reinterpret_cast<const f32x4 *>(sA + c * TLD + 4 * NV * q + 4 * v);
 #pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = 0.f;
-    for (int k0 = kb; k0 < ke; k0 += 16) {
-        for (int t = threadIdx.x; t < 1024; t += 256) {
-            int mm, kk;
-            if (sam == 1) { mm = t % 64; kk = t / 64; } else { kk = t % 16; mm = t / 16; }
-            const int m = m0 + mm, k = k0 + kk;
-            As[kk][mm] = (m < M && k < ke) ? A[m * sam + k * sak] : 0.f;
-        }
-        for (int t = threadIdx.x; t < 1024; t += 256) {
-            int nn, kk;
-            if (sbn == 1) { nn = t % 64; kk = t / 64; } else { kk = t % 16; nn = t / 16; }
-            const int n = n0 + nn, k = k0 + kk;
-            Bs[kk][nn] = (n < N && k < ke) ? B[k * sbk + n * sbn] : 0.f;
-        }
-        __syncthreads();
+        for (int i = 0; i < 4; i++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[v][i], acc, 0, 0, 0);
+    }
+    return acc;
+}
+
+template <int NV>
+__device__ __forceinline__ void load_operand(const float *__restrict__ row, int q, f32x4 b[NV])
+{
 #pragma unroll
-        for (int kk = 0; kk < 16; kk++) {
-            float a[4], b[4];
+    for (int v = 0; v < NV; v++) b[v] = *reinterpret_cast<const f32x4 *>(row + 4 * NV * q + 4 * v);
+}
+
+// what a step reads and writes; row r of the batch is sample
+// hash(seed, step, r) mod nsamples (drawn with replacement), or row r of X, Y
+struct StepArgs {
+    int B;
+    const float *X, *Y;
+    int64_t nsamples;      // 0: rows as they lie
+    uint64_t seed;
+    int64_t step;
+    const float *p, *aux;
+    float scale;           // 1 / (27 B)
+    float *xb;             // B16 x 16 inputs
+    float *h;              // 3 x B16 x 128 activations
+    float *dz;             // 3 x B16 x 128 gradients before the activation
+    float *dy;             // B16 x 32 output gradients
+    float *yp;             // predictions (forward only), B x 27
+    double *loss;          // per workgroup: sum of squared errors
+};
+
+// Forward (and, BWD, backward) of 16 rows: eight waves, wave w owns units
+// 16 w .. 16 w + 15 of every hidden layer.  Activations pass through LDS; the
+// derivative of SiLU stays in the registers of the lane that meets the same
+// (row, unit) again on the way back.  Each layer's weights are loaded before
+// the barrier that ends the layer before it.
+//
+// Bound: the chain of seven dependent products, each 32 matrix instructions
+// a wave and its weights from L2: 21 us for 4,096 rows (256 workgroups).  With
+// one launch a product (64 x 64 tiles on the vector units, 64 to 128 workgroups)
+// and one for each elementwise pass a training step took 503 us; it takes 50.
+template <bool BWD>
+__global__ __launch_bounds__(512) void k_mlp_step(StepArgs A)
+{
+    __shared__ __align__(16) float sA[2][TR * TLD];
+    __shared__ double sL[8];
+    const int t = threadIdx.x, w = t >> 6, l = t & 63, c = l & 15, q = l >> 4;
+    const int r0 = blockIdx.x * TR, B16 = gridDim.x * TR, u = 16 * w + c;
+    const float *P = A.p;
+    f32x4 b1[1], b[8];
+    load_operand<1>(A.aux + AUX_W1 + u * 16, q, b1);
+    load_operand<8>(P + OFF_W2 + u * MLP_H, q, b);
+    auto sample = [&](int r) -> int64_t {
+        r = min(r, A.B - 1);   // the rows past the batch repeat its last one, with no gradient
+        if (!A.nsamples) return r;
+        return (int64_t)(mix64(A.seed ^ mix64((uint64_t)A.step * 0x9E3779B97F4A7C15ull + (uint64_t)r)) %
+                         (uint64_t)A.nsamples);
+    };
+    if (t < TR * 16) {
+        const int r = t >> 4, k = t & 15;
+        const float x = k < MLP_IN ? A.X[sample(r0 + r) * MLP_IN + k] : 0.f;
+        sA[0][r * TLD + k] = x;
+        if constexpr (BWD) A.xb[(size_t)(r0 + r) * 16 + k] = x;
+    }
+    __syncthreads();
+    float dsilu[3][4];
+    f32x4 acc;
 #pragma unroll
-            for (int i = 0; i < 4; i++) a[i] = As[kk][tm * 4 + i];
+    for (int L = 0; L < 3; L++) {
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        if (L == 0)
+            acc = tile_product<1>(sA[0], b1, c, q, zero);
+        else
+            acc = tile_product<8>(sA[L & 1], b, c, q, zero);
+        if (L == 1) load_operand<8>(P + OFF_W3 + u * MLP_H, q, b);
+        if (L == 2) load_operand<8>(P + OFF_W4 + min(u, MLP_OUT - 1) * MLP_H, q, b);
+        const float bias = P[(L == 0 ? OFF_B1 : L == 1 ? OFF_B2 : OFF_B3) + u];
 #pragma unroll
-            for (int j = 0; j < 4; j++) b[j] = Bs[kk][tn * 4 + j];
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
+        for (int i = 0; i < 4; i++) {
+            const float z = acc[i] + bias, s = sigmoidf_(z), h = z * s;
+            dsilu[L][i] = s * (1.f + z * (1.f - s));
+            sA[(L + 1) & 1][(4 * q + i) * TLD + u] = h;
+            if constexpr (BWD) A.h[((size_t)L * B16 + r0 + 4 * q + i) * MLP_H + u] = h;
         }
         __syncthreads();
     }
+    // output layer on the first two waves: 27 of 32 columns
+    double loss = 0.0;
+    if (w < 2) {
+        acc = tile_product<8>(sA[1], b, c, q, f32x4{0.f, 0.f, 0.f, 0.f});
+        const float bias = u < MLP_OUT ? P[OFF_B4 + u] : 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int m = m0 + tm * 4 + i;
-        if (m >= M) continue;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int n = n0 + tn * 4 + j;
-            if (n >= N) continue;
-            float v = acc[i][j];
-            if (EPI == 1) {
-                v += bias[n];
-                Z[m * ldc + n] = v;
-                v = v * sigmoidf_(v);
-            } else if (EPI == 2) {
-                v += bias[n];
+        for (int i = 0; i < 4; i++) {
+            const int r = r0 + 4 * q + i;
+            const bool live = r < A.B && u < MLP_OUT;
+            const float y = acc[i] + bias;
+            if constexpr (BWD) {
+                const float d = live ? y - A.Y[sample(r) * MLP_OUT + u] : 0.f;
+                const float dy = 2.f * A.scale * d;
+                loss += (double)d * (double)d;
+                sA[0][(4 * q + i) * TLD + u] = dy;
+                A.dy[(size_t)r * 32 + u] = dy;
+            } else {
+                if (live) A.yp[(size_t)r * MLP_OUT + u] = y;
             }
-            C[m * ldc + n] = v;
+        }
+    }
+    if constexpr (!BWD) return;
+    f32x4 b4[2];
+    load_operand<2>(A.aux + AUX_T4 + u * 32, q, b4);
+    load_operand<8>(A.aux + AUX_T3 + u * MLP_H, q, b);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off, 64);
+    if (l == 0) sL[w] = loss;
+    __syncthreads();
+    if (t == 0) A.loss[blockIdx.x] = sL[0] + sL[1];
+#pragma unroll
+    for (int L = 2; L >= 0; L--) {
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        if (L == 2)
+            acc = tile_product<2>(sA[0], b4, c, q, zero);
+        else
+            acc = tile_product<8>(sA[L & 1 ? 1 : 0], b, c, q, zero);
+        if (L == 1) load_operand<8>(A.aux + AUX_T2 + u * MLP_H, q, b);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float d = acc[i] * dsilu[L][i];
+            if (L) sA[L & 1 ? 0 : 1][(4 * q + i) * TLD + u] = d;
+            A.dz[((size_t)L * B16 + r0 + 4 * q + i) * MLP_H + u] = d;
+        }
+        if (L) __syncthreads();
+    }
+}
+
+// acc (32 x 32 tiles NM x NN) += sum over rows [k0, k1) of a[k][m] b[k][n]
+// (row strides lda, ldb); lanes 32..63 take the odd rows.  MB / NB: columns of
+// a / b past which a tile's operand is zero.  csum: per lane, the sum of a's
+// first-tile columns (the bias gradient).
+template <int NM, int NN>
+__device__ __forceinline__ void rank_update(const float *__restrict__ a, int lda, const float *__restrict__ b, int ldb,
+                                            int k0, int k1, int l, f32x16 acc[NM][NN], float csum[NM])
+{
+    const int m = l & 31;
+#pragma unroll 8
+    for (int k = k0 + (l >> 5); k < k1; k += 2) {
+        float x[NM], y[NN];
+#pragma unroll
+        for (int i = 0; i < NM; i++) x[i] = a[(size_t)k * lda + 32 * i + m];
+#pragma unroll
+        for (int j = 0; j < NN; j++) y[j] = b[(size_t)k * ldb + 32 * j + m];
+#pragma unroll
+        for (int i = 0; i < NM; i++) {
+            csum[i] += x[i];
+#pragma unroll
+            for (int j = 0; j < NN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[i], y[j], acc[i][j], 0, 0, 0);
         }
     }
 }
 
-// out = sum over the S split-K slabs of ws (fixed order)
-__global__ void k_sum_slabs(int S, int64_t n, const float *__restrict__ ws, float *__restrict__ out)
+// row of value r of lane l in a 32 x 32 tile (column l % 32)
+__device__ __forceinline__ int tile_row(int l, int r) { return 8 * (r >> 2) + 4 * (l >> 5) + (r & 3); }
+
+template <int NM, int NN>
+__device__ __forceinline__ void store_tiles(const f32x16 acc[NM][NN], int l, float *__restrict__ out, int m0, int mmax,
+                                            int n0, int nmax)
 {
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+#pragma unroll
+    for (int i = 0; i < NM; i++)
+#pragma unroll
+        for (int j = 0; j < NN; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int m = m0 + 32 * i + tile_row(l, r), n = n0 + 32 * j + (l & 31);
+                if (m < mmax && n < nmax) out[m * nmax + n] = acc[i][j][r];
+            }
+}
+
+// Gradient slab z of the parameters: sums over rows [rows z, rows (z + 1)) of
+// dZ_L^T H_{L-1} and of dZ_L.  Blocks (0, z) and (1, z): layers 2 and 3, a
+// 64 x 64 quarter a wave; block (2, z): layer 1 (32 units a wave) and the
+// output layer (32 inputs a wave).
+//
+// Bound: the latency of the row loads, 32 pairs of rows a slab: 23 us for 4,096
+// rows in 64 slabs.
+__global__ __launch_bounds__(256) void k_mlp_wgrad(int B16, int rows, const float *__restrict__ xb,
+                                                   const float *__restrict__ h, const float *__restrict__ dz,
+                                                   const float *__restrict__ dy, float *__restrict__ slabs)
+{
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63, z = blockIdx.y;
+    const int k0 = z * rows, k1 = min(B16, k0 + rows);
+    float *out = slabs + (size_t)z * MLP_NPARAM;
+    const size_t layer = (size_t)B16 * MLP_H;
+    if (blockIdx.x < 2) {
+        const int L = blockIdx.x + 1, m0 = 64 * (w >> 1), n0 = 64 * (w & 1);
+        f32x16 acc[2][2] = {};
+        float cs[2] = {0.f, 0.f};
+        rank_update<2, 2>(dz + L * layer + m0, MLP_H, h + (L - 1) * layer + n0, MLP_H, k0, k1, l, acc, cs);
+        store_tiles<2, 2>(acc, l, out + (L == 1 ? OFF_W2 : OFF_W3), m0, MLP_H, n0, MLP_H);
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            cs[i] += __shfl_xor(cs[i], 32, 64);
+            if (n0 == 0 && l < 32) out[(L == 1 ? OFF_B2 : OFF_B3) + m0 + 32 * i + l] = cs[i];
+        }
+    } else {
+        f32x16 acc[1][1] = {};
+        float cs[1] = {0.f};
+        const int m = l & 31;
+#pragma unroll 8
+        for (int k = k0 + (l >> 5); k < k1; k += 2) {
+            const float x = dz[(size_t)k * MLP_H + 32 * w + m], y = m < 16 ? xb[(size_t)k * 16 + m] : 0.f;
+            cs[0] += x;
+            acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, acc[0][0], 0, 0, 0);
+        }
+        store_tiles<1, 1>(acc, l, out + OFF_W1, 32 * w, MLP_H, 0, MLP_IN);
+        cs[0] += __shfl_xor(cs[0], 32, 64);
+        if (l < 32) out[OFF_B1 + 32 * w + l] = cs[0];
+        f32x16 acc4[1][1] = {};
+        cs[0] = 0.f;
+        rank_update<1, 1>(dy, 32, h + 2 * layer + 32 * w, MLP_H, k0, k1, l, acc4, cs);
+        // the tile's columns are inputs 32 w ..: rows of W4 are 128 long
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int u = tile_row(l, r);
+            if (u < MLP_OUT) out[OFF_W4 + u * MLP_H + 32 * w + (l & 31)] = acc4[0][0][r];
+        }
+        cs[0] += __shfl_xor(cs[0], 32, 64);
+        if (w == 0 && l < MLP_OUT) out[OFF_B4 + l] = cs[0];
+    }
+}
+
+// g = sum of the S slabs (in order), and with adam the Adam update of the
+// parameters and their copies; block 0 also sums the loss partials
+__global__ __launch_bounds__(256) void k_mlp_apply(int S, const float *__restrict__ slabs, int nloss,
+                                                   const double *__restrict__ lossp, double lscale,
+                                                   double *__restrict__ loss, float *__restrict__ g,
+                                                   float *__restrict__ p, float *__restrict__ aux,
+                                                   float *__restrict__ m, float *__restrict__ v, int adam, float lr, float b1,
+                                                   float b2, float eps, float bc1, float bc2)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < MLP_NPARAM) {
         float s = 0.f;
-        for (int z = 0; z < S; z++) s += ws[(int64_t)z * n + i];
-        out[i] = s;
+        for (int z0 = 0; z0 < S; z0 += 16) {
+            float x[16];
+#pragma unroll
+            for (int j = 0; j < 16; j++) x[j] = z0 + j < S ? slabs[(size_t)(z0 + j) * MLP_NPARAM + i] : 0.f;
+#pragma unroll
+            for (int j = 0; j < 16; j++) s += x[j];
+        }
+        g[i] = s;
+        if (adam) {
+            const float mi = b1 * m[i] + (1.f - b1) * s;
+            const float vi = b2 * v[i] + (1.f - b2) * s * s;
+            m[i] = mi;
+            v[i] = vi;
+            const float pi = p[i] - lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
+            p[i] = pi;
+            const int j = aux_of(i);
+            if (j >= 0) aux[j] = pi;
+        }
     }
-}
-
-// dZ = dH * silu'(Z), in place on dH
-__global__ void k_silu_back(int64_t n, const float *__restrict__ Z, float *__restrict__ dH)
-{
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const float z = Z[i], s = sigmoidf_(z);
-        dH[i] *= s * (1.f + z * (1.f - s));
-    }
-}
-
-// column sums of a [rows x cols] row-major matrix (bias gradients), fixed order
-__global__ void k_colsum(int rows, int cols, const float *__restrict__ A, float *__restrict__ out)
-{
-    __shared__ float sh[256];
-    const int c = blockIdx.x;
-    float s = 0.f;
-    for (int r = threadIdx.x; r < rows; r += 256) s += A[(int64_t)r * cols + c];
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[c] = sh[0];
-}
-
-// dY = 2 (Yp - Y) / (rows * 27); per-block partial sums of the squared error
-__global__ __launch_bounds__(256) void k_mse(int64_t n, const float *__restrict__ Yp, const float *__restrict__ Y,
-                                             float scale, float *__restrict__ dY, double *__restrict__ partials)
-{
-    __shared__ double sh[256];
+    if (blockIdx.x != 0) return;
+    __shared__ double sh[4];
     double s = 0.0;
-    for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-        const float d = Yp[i] - Y[i];
-        dY[i] = 2.f * scale * d;
-        s += (double)d * (double)d;
-    }
-    sh[threadIdx.x] = s;
+    for (int k = threadIdx.x; k < nloss; k += 256) s += lossp[k];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if (threadIdx.x % 64 == 0) sh[threadIdx.x / 64] = s;
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) partials[blockIdx.x] = sh[0];
-}
-
-__global__ void k_sum_partials(int nb, const double *__restrict__ partials, double scale, double *__restrict__ out)
-{
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    double s = 0.0;
-    for (int i = 0; i < nb; i++) s += partials[i];
-    *out = s * scale;
-}
-
-// batch rows drawn with replacement: row = hash(seed, step, i) mod nsamples
-__global__ void k_gather_batch(int64_t nsamples, const float *__restrict__ X, const float *__restrict__ Y, int B,
-                               uint64_t seed, int64_t step, float *__restrict__ Xb, float *__restrict__ Yb)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= B) return;
-    const int64_t r = (int64_t)(mix64(seed ^ mix64((uint64_t)step * 0x9E3779B97F4A7C15ull + (uint64_t)i)) %
-                                (uint64_t)nsamples);
-    for (int k = 0; k < MLP_IN; k++) Xb[(int64_t)i * MLP_IN + k] = X[r * MLP_IN + k];
-    for (int k = 0; k < MLP_OUT; k++) Yb[(int64_t)i * MLP_OUT + k] = Y[r * MLP_OUT + k];
-}
-
-__global__ void k_adam(int n, float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m,
-                       float *__restrict__ v, float lr, float b1, float b2, float eps, float bc1, float bc2)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.f - b1) * gi;
-    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    p[i] -= lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
+    if (threadIdx.x == 0) *loss = (sh[0] + sh[1] + sh[2] + sh[3]) * lscale;
 }
 
 // --------------------------------------------------------- BF16 inference
 typedef __bf16 bf16x8 __attribute__((__vector_size__(8 * sizeof(__bf16))));
-typedef float f32x16 __attribute__((__vector_size__(16 * sizeof(float))));
 
 __host__ __device__ inline uint16_t f2bf(float f)
 {
@@ -293,10 +457,6 @@ __device__ __forceinline__ float bf2f(uint16_t b)
     memcpy(&f, &u, 4);
     return f;
 }
-
-// one 32x32 output tile of 64 lanes: value r of lane l is row
-// 8 (r/4) + 4 (l/32) + r%4, column l%32
-__device__ __forceinline__ int tile_row(int l, int r) { return 8 * (r >> 2) + 4 * (l >> 5) + (r & 3); }
 
 // the activation tile of a wave is private to it: LDS operations of one
 // wave complete in order, so a wave-level barrier (no block barrier) orders
@@ -431,11 +591,18 @@ struct hfem_mlp {
     // training set
     int64_t nsamples = 0;
     float *d_X = nullptr, *d_Y = nullptr;
-    // work buffers for a batch of up to cap rows
+    // copies of the weights that the FP32 products read (valid when
+    // aux_version == param_version)
+    float *d_aux = nullptr;
+    long aux_version = -1;
+    // work buffers for batches of up to cap rows (a multiple of TR)
     int cap = 0;
-    float *d_xb = nullptr, *d_yb = nullptr, *d_z[3] = {nullptr, nullptr, nullptr}, *d_h[3] = {nullptr, nullptr, nullptr};
-    float *d_yp = nullptr, *d_dy = nullptr, *d_dh = nullptr;
-    float *d_ws = nullptr;       // split-K workspace of the weight gradients
+    float *d_xb = nullptr, *d_h = nullptr, *d_dz = nullptr, *d_dy = nullptr;
+    double *d_lossp = nullptr;   // per workgroup
+    float *d_ws = nullptr;       // gradient slabs
+    // host-array rows and predictions of hfem_mlp_forward / _gradients
+    int io_cap = 0;
+    float *d_ix = nullptr, *d_iy = nullptr;
     double *d_loss = nullptr;
     // BF16 operand-order weights (valid when packed_version == param_version)
     uint16_t *d_wpk = nullptr;
@@ -445,98 +612,86 @@ struct hfem_mlp {
 static int mlp_ensure_batch(hfem_mlp *m, int B)
 {
     if (B <= m->cap) return 0;
-    void *ps[] = {m->d_xb, m->d_yb, m->d_z[0], m->d_z[1], m->d_z[2], m->d_h[0], m->d_h[1], m->d_h[2],
-                  m->d_yp, m->d_dy, m->d_dh};
+    HIPFEM_CHECK(hipStreamSynchronize(m->ctx->stream));   // a step may still use the buffers
+    void *ps[] = {m->d_xb, m->d_h, m->d_dz, m->d_dy, m->d_lossp};
+    m->d_xb = m->d_h = m->d_dz = m->d_dy = nullptr;
+    m->d_lossp = nullptr;
+    m->cap = 0;
     for (void *p : ps)
         if (p) HIPFEM_CHECK(hipFree(p));
-    const size_t b = (size_t)B;
-    HIPFEM_CHECK(hipMalloc(&m->d_xb, sizeof(float) * b * MLP_IN));
-    HIPFEM_CHECK(hipMalloc(&m->d_yb, sizeof(float) * b * MLP_OUT));
-    for (int i = 0; i < 3; i++) {
-        HIPFEM_CHECK(hipMalloc(&m->d_z[i], sizeof(float) * b * MLP_H));
-        HIPFEM_CHECK(hipMalloc(&m->d_h[i], sizeof(float) * b * MLP_H));
-    }
-    HIPFEM_CHECK(hipMalloc(&m->d_yp, sizeof(float) * b * MLP_OUT));
-    HIPFEM_CHECK(hipMalloc(&m->d_dy, sizeof(float) * b * MLP_OUT));
-    HIPFEM_CHECK(hipMalloc(&m->d_dh, sizeof(float) * b * MLP_H));
-    if (!m->d_ws) HIPFEM_CHECK(hipMalloc(&m->d_ws, sizeof(float) * MLP_SPLITK * MLP_H * MLP_H));
-    m->cap = B;
+    const size_t b = ((size_t)B + TR - 1) / TR * TR;
+    HIPFEM_REQUIRE(b <= INT32_MAX, HIPFEM_ETOOBIG, "batch of %d rows too large", B);
+    HIPFEM_CHECK(hipMalloc(&m->d_xb, sizeof(float) * b * 16));
+    HIPFEM_CHECK(hipMalloc(&m->d_h, sizeof(float) * b * 3 * MLP_H));
+    HIPFEM_CHECK(hipMalloc(&m->d_dz, sizeof(float) * b * 3 * MLP_H));
+    HIPFEM_CHECK(hipMalloc(&m->d_dy, sizeof(float) * b * 32));
+    HIPFEM_CHECK(hipMalloc(&m->d_lossp, sizeof(double) * (b / TR)));
+    if (!m->d_ws) HIPFEM_CHECK(hipMalloc(&m->d_ws, sizeof(float) * (size_t)MLP_SLABS * MLP_NPARAM));
+    m->cap = (int)b;
     return 0;
 }
 
-static dim3 gemm_grid(int M, int N) { return dim3((N + 63) / 64, (M + 63) / 64); }
-
-// forward pass of B rows of xb: z/h of the hidden layers kept for backward
-static int mlp_forward(hfem_mlp *m, int B, const float *xb, float *yp)
+// device buffers for n host rows (inputs, targets or predictions)
+static int mlp_ensure_io(hfem_mlp *m, int n)
 {
+    if (n <= m->io_cap) return 0;
+    void *ps[] = {m->d_ix, m->d_iy};
+    m->d_ix = m->d_iy = nullptr;
+    m->io_cap = 0;
+    for (void *p : ps)
+        if (p) HIPFEM_CHECK(hipFree(p));
+    HIPFEM_CHECK(hipMalloc(&m->d_ix, sizeof(float) * (size_t)n * MLP_IN));
+    HIPFEM_CHECK(hipMalloc(&m->d_iy, sizeof(float) * (size_t)n * MLP_OUT));
+    m->io_cap = n;
+    return 0;
+}
+
+// the weight copies of the current parameters
+static int mlp_ensure_aux(hfem_mlp *m)
+{
+    if (m->d_aux && m->aux_version == m->param_version) return 0;
     hipStream_t s = m->ctx->stream;
-    const float *P = m->d_p;
-    k_gemm<1><<<gemm_grid(B, MLP_H), 256, 0, s>>>(B, MLP_H, MLP_IN, xb, MLP_IN, 1, P + OFF_W1, 1, MLP_IN, P + OFF_B1,
-                                                  m->d_h[0], MLP_H, m->d_z[0]);
-    k_gemm<1><<<gemm_grid(B, MLP_H), 256, 0, s>>>(B, MLP_H, MLP_H, m->d_h[0], MLP_H, 1, P + OFF_W2, 1, MLP_H,
-                                                  P + OFF_B2, m->d_h[1], MLP_H, m->d_z[1]);
-    k_gemm<1><<<gemm_grid(B, MLP_H), 256, 0, s>>>(B, MLP_H, MLP_H, m->d_h[1], MLP_H, 1, P + OFF_W3, 1, MLP_H,
-                                                  P + OFF_B3, m->d_h[2], MLP_H, m->d_z[2]);
-    k_gemm<2><<<gemm_grid(B, MLP_OUT), 256, 0, s>>>(B, MLP_OUT, MLP_H, m->d_h[2], MLP_H, 1, P + OFF_W4, 1, MLP_H,
-                                                    P + OFF_B4, yp, MLP_OUT, nullptr);
+    if (!m->d_aux) {
+        HIPFEM_CHECK(hipMalloc(&m->d_aux, sizeof(float) * MLP_NAUX));
+        k_zero_pad<<<(MLP_NAUX + 255) / 256, 256, 0, s>>>(MLP_NAUX, m->d_aux);
+    }
+    k_mlp_aux<<<(MLP_NPARAM + 255) / 256, 256, 0, s>>>(m->d_p, m->d_aux);
     HIPFEM_CHECK(hipGetLastError());
+    m->aux_version = m->param_version;
     return 0;
 }
 
-// gradients of the mean-squared error of B rows into d_g; loss into d_loss
-static int mlp_backward(hfem_mlp *m, int B, const float *xb, const float *yb)
+// forward, backward and gradients of the B rows that a names into d_g, loss
+// into d_loss; with adam the Adam update (bias corrections bc1, bc2)
+static int mlp_step(hfem_mlp *m, StepArgs a, bool adam, float lr, float bc1, float bc2)
 {
     hipStream_t s = m->ctx->stream;
-    const float *P = m->d_p;
-    float *G = m->d_g;
-    int rc = ensure_partials(m->ctx, 1024);
-    if (rc) return rc;
-    const int64_t ny = (int64_t)B * MLP_OUT;
-    const int nbm = (int)std::min<int64_t>(1024, (ny + 255) / 256);
-    k_mse<<<nbm, 256, 0, s>>>(ny, m->d_yp, yb, 1.f / (float)ny, m->d_dy, m->ctx->d_partials);
-    k_sum_partials<<<1, 64, 0, s>>>(nbm, m->ctx->d_partials, 1.0 / (double)ny, m->d_loss);
-    // weight gradients reduce over the batch: split K into S slabs of at
-    // least 256 rows, then sum the slabs in order
-    const int S = std::max(1, std::min(MLP_SPLITK, B / 256));
-    auto wgrad = [&](int M, int N, const float *A, int64_t sam, int64_t sak, const float *Bm, int64_t sbk,
-                     int64_t sbn, float *out) {
-        dim3 g = gemm_grid(M, N);
-        g.z = S;
-        k_gemm<0><<<g, 256, 0, s>>>(M, N, B, A, sam, sak, Bm, sbk, sbn, nullptr, m->d_ws, N, nullptr);
-        const int64_t mn = (int64_t)M * N;
-        k_sum_slabs<<<(int)std::min<int64_t>(1024, (mn + 255) / 256), 256, 0, s>>>(S, mn, m->d_ws, out);
-    };
-    // layer 4: dW4 = dY^T H3, db4 = colsum dY, dH3 = dY W4
-    wgrad(MLP_OUT, MLP_H, m->d_dy, 1, MLP_OUT, m->d_h[2], MLP_H, 1, G + OFF_W4);
-    k_colsum<<<MLP_OUT, 256, 0, s>>>(B, MLP_OUT, m->d_dy, G + OFF_B4);
-    k_gemm<0><<<gemm_grid(B, MLP_H), 256, 0, s>>>(B, MLP_H, MLP_OUT, m->d_dy, MLP_OUT, 1, P + OFF_W4, MLP_H, 1,
-                                                  nullptr, m->d_dh, MLP_H, nullptr);
-    const int64_t nh = (int64_t)B * MLP_H;
-    const int nbe = (int)std::min<int64_t>(4096, (nh + 255) / 256);
-    const int offW[3] = {OFF_W1, OFF_W2, OFF_W3}, offB[3] = {OFF_B1, OFF_B2, OFF_B3};
-    for (int L = 2; L >= 0; L--) {
-        k_silu_back<<<nbe, 256, 0, s>>>(nh, m->d_z[L], m->d_dh);   // dZ_L
-        const float *in = L == 0 ? xb : m->d_h[L - 1];
-        const int nin = L == 0 ? MLP_IN : MLP_H;
-        wgrad(MLP_H, nin, m->d_dh, 1, MLP_H, in, nin, 1, G + offW[L]);
-        k_colsum<<<MLP_H, 256, 0, s>>>(B, MLP_H, m->d_dh, G + offB[L]);
-        if (L > 0) {
-            // dH_{L-1} = dZ_L W_L: uses d_dh as input, so write into the z
-            // buffer of layer L (no longer needed) and swap
-            k_gemm<0><<<gemm_grid(B, MLP_H), 256, 0, s>>>(B, MLP_H, MLP_H, m->d_dh, MLP_H, 1, P + offW[L], MLP_H, 1,
-                                                          nullptr, m->d_z[L], MLP_H, nullptr);
-            std::swap(m->d_z[L], m->d_dh);
-        }
-    }
+    const int nwg = (a.B + TR - 1) / TR, B16 = nwg * TR;
+    a.p = m->d_p;
+    a.aux = m->d_aux;
+    a.scale = 1.f / (float)((int64_t)a.B * MLP_OUT);
+    a.xb = m->d_xb;
+    a.h = m->d_h;
+    a.dz = m->d_dz;
+    a.dy = m->d_dy;
+    a.yp = nullptr;
+    a.loss = m->d_lossp;
+    k_mlp_step<true><<<nwg, 512, 0, s>>>(a);
+    // slabs of at least 64 rows, an even number each (two rows an instruction)
+    const int rows = std::max(64, ((B16 + MLP_SLABS - 1) / MLP_SLABS + 1) / 2 * 2), S = (B16 + rows - 1) / rows;
+    k_mlp_wgrad<<<dim3(3, S), 256, 0, s>>>(B16, rows, m->d_xb, m->d_h, m->d_dz, m->d_dy, m->d_ws);
+    k_mlp_apply<<<(MLP_NPARAM + 255) / 256, 256, 0, s>>>(S, m->d_ws, nwg, m->d_lossp,
+                                                         1.0 / (double)((int64_t)a.B * MLP_OUT), m->d_loss, m->d_g,
+                                                         m->d_p, m->d_aux, m->d_m, m->d_v, adam, lr, 0.9f, 0.999f, 1e-8f,
+                                                         bc1, bc2);
     HIPFEM_CHECK(hipGetLastError());
     return 0;
 }
 
 static int mlp_free(hfem_mlp *m)
 {
-    void *ps[] = {m->d_p, m->d_g, m->d_m, m->d_v, m->d_X, m->d_Y, m->d_xb, m->d_yb, m->d_z[0], m->d_z[1],
-                  m->d_z[2], m->d_h[0], m->d_h[1], m->d_h[2], m->d_yp, m->d_dy, m->d_dh, m->d_loss, m->d_wpk,
-                  m->d_ws};
+    void *ps[] = {m->d_p, m->d_g, m->d_m, m->d_v, m->d_X, m->d_Y, m->d_xb, m->d_h, m->d_dz, m->d_dy, m->d_lossp,
+                  m->d_ix, m->d_iy, m->d_aux, m->d_loss, m->d_wpk, m->d_ws};
     for (void *p : ps)
         if (p) HIPFEM_CHECK(hipFree(p));
     return 0;
@@ -676,24 +831,27 @@ extern "C" int hfem_mlp_train(hfem_mlp *m, int steps, int batch, double lr, doub
     hipStream_t s = m->ctx->stream;
     int rc = mlp_ensure_batch(m, batch);
     if (rc) return rc;
+    rc = mlp_ensure_aux(m);
+    if (rc) return rc;
     const float b1 = 0.9f, b2 = 0.999f;
     for (int it = 0; it < steps; it++) {
-        k_gather_batch<<<(batch + 255) / 256, 256, 0, s>>>(m->nsamples, m->d_X, m->d_Y, batch, seed, it, m->d_xb,
-                                                           m->d_yb);
-        rc = mlp_forward(m, batch, m->d_xb, m->d_yp);
-        if (rc) return rc;
-        rc = mlp_backward(m, batch, m->d_xb, m->d_yb);
-        if (rc) return rc;
         m->adam_t++;
         // cosine decay from lr to lr_final
         const double c = 0.5 * (1.0 + std::cos(3.141592653589793 * (double)it / std::max(1, steps)));
         const float lrt = (float)(lr_final + (lr - lr_final) * c);
         const float bc1 = 1.f - std::pow(b1, (float)m->adam_t), bc2 = 1.f - std::pow(b2, (float)m->adam_t);
-        k_adam<<<(MLP_NPARAM + 255) / 256, 256, 0, s>>>(MLP_NPARAM, m->d_p, m->d_g, m->d_m, m->d_v, lrt, b1, b2, 1e-8f,
-                                                         bc1, bc2);
-        HIPFEM_CHECK(hipGetLastError());
+        StepArgs a = {};
+        a.B = batch;
+        a.X = m->d_X;
+        a.Y = m->d_Y;
+        a.nsamples = m->nsamples;
+        a.seed = seed;
+        a.step = it;
+        rc = mlp_step(m, a, true, lrt, bc1, bc2);
+        if (rc) return rc;
     }
     m->param_version++;
+    m->aux_version = m->param_version;   // the update wrote the copies too
     if (final_loss) {
         HIPFEM_CHECK(hipMemcpyAsync(final_loss, m->d_loss, sizeof(double), hipMemcpyDeviceToHost, s));
     }
@@ -706,13 +864,22 @@ extern "C" int hfem_mlp_forward(hfem_mlp *m, int n, const float *X, float *Y)
 {
     HIPFEM_REQUIRE(m && n >= 0 && X && Y, HIPFEM_EINVAL, "forward: bad arguments");
     DeviceGuard g(m->ctx->device);
-    int rc = mlp_ensure_batch(m, std::max(n, 1));
+    if (n == 0) return 0;
+    int rc = mlp_ensure_io(m, n);
+    if (rc) return rc;
+    rc = mlp_ensure_aux(m);
     if (rc) return rc;
     hipStream_t s = m->ctx->stream;
-    HIPFEM_CHECK(hipMemcpyAsync(m->d_xb, X, sizeof(float) * n * MLP_IN, hipMemcpyHostToDevice, s));
-    rc = mlp_forward(m, n, m->d_xb, m->d_yp);
-    if (rc) return rc;
-    HIPFEM_CHECK(hipMemcpyAsync(Y, m->d_yp, sizeof(float) * n * MLP_OUT, hipMemcpyDeviceToHost, s));
+    HIPFEM_CHECK(hipMemcpyAsync(m->d_ix, X, sizeof(float) * n * MLP_IN, hipMemcpyHostToDevice, s));
+    StepArgs a = {};
+    a.B = n;
+    a.X = m->d_ix;
+    a.p = m->d_p;
+    a.aux = m->d_aux;
+    a.yp = m->d_iy;
+    k_mlp_step<false><<<(n + TR - 1) / TR, 512, 0, s>>>(a);
+    HIPFEM_CHECK(hipGetLastError());
+    HIPFEM_CHECK(hipMemcpyAsync(Y, m->d_iy, sizeof(float) * n * MLP_OUT, hipMemcpyDeviceToHost, s));
     HIPFEM_CHECK(hipStreamSynchronize(s));
     return 0;
 }
@@ -723,12 +890,18 @@ extern "C" int hfem_mlp_gradients(hfem_mlp *m, int n, const float *X, const floa
     DeviceGuard g(m->ctx->device);
     int rc = mlp_ensure_batch(m, n);
     if (rc) return rc;
-    hipStream_t s = m->ctx->stream;
-    HIPFEM_CHECK(hipMemcpyAsync(m->d_xb, X, sizeof(float) * n * MLP_IN, hipMemcpyHostToDevice, s));
-    HIPFEM_CHECK(hipMemcpyAsync(m->d_yb, Y, sizeof(float) * n * MLP_OUT, hipMemcpyHostToDevice, s));
-    rc = mlp_forward(m, n, m->d_xb, m->d_yp);
+    rc = mlp_ensure_io(m, n);
     if (rc) return rc;
-    rc = mlp_backward(m, n, m->d_xb, m->d_yb);
+    rc = mlp_ensure_aux(m);
+    if (rc) return rc;
+    hipStream_t s = m->ctx->stream;
+    HIPFEM_CHECK(hipMemcpyAsync(m->d_ix, X, sizeof(float) * n * MLP_IN, hipMemcpyHostToDevice, s));
+    HIPFEM_CHECK(hipMemcpyAsync(m->d_iy, Y, sizeof(float) * n * MLP_OUT, hipMemcpyHostToDevice, s));
+    StepArgs a = {};
+    a.B = n;
+    a.X = m->d_ix;
+    a.Y = m->d_iy;
+    rc = mlp_step(m, a, false, 0.f, 1.f, 1.f);
     if (rc) return rc;
     HIPFEM_CHECK(hipMemcpyAsync(grad, m->d_g, sizeof(float) * MLP_NPARAM, hipMemcpyDeviceToHost, s));
     if (loss) HIPFEM_CHECK(hipMemcpyAsync(loss, m->d_loss, sizeof(double), hipMemcpyDeviceToHost, s));

@@ -45,6 +45,27 @@ def test_gradients_match_oracle(net):
         assert np.linalg.norm(g[a:b] - gref[a:b]) <= 1e-4 * np.linalg.norm(gref[a:b]), (a, b)
 
 
+@pytest.mark.parametrize("rows", [1, 15, 17, 64, 4099])
+def test_step_edges_match_oracle(net, rows):
+    """Forward and gradients at the edges of the 16-row tiles and the 64-row
+    gradient slabs (one row, partial last tiles, a last slab shorter than the
+    others), with the tolerances of the plain cases; the same bits twice."""
+    rng = np.random.default_rng(rows)
+    X = rng.standard_normal((rows, 13)).astype(np.float32)
+    Y = rng.standard_normal((rows, 27)).astype(np.float32)
+    p64 = net.params().astype(np.float64)
+    ref = M.forward(p64, X.astype(np.float64))
+    assert np.abs(net.forward(X) - ref).max() <= 1e-5 * max(1.0, np.abs(ref).max())
+    loss, g = net.gradients(X, Y)
+    lref, gref = M.loss_and_grad(p64, X.astype(np.float64), Y.astype(np.float64))
+    assert abs(loss - lref) <= 1e-5 * lref
+    offs = np.cumsum([0] + [int(np.prod(s)) for s in M.SHAPES])
+    for a, b in zip(offs[:-1], offs[1:]):
+        assert np.linalg.norm(g[a:b] - gref[a:b]) <= 1e-4 * np.linalg.norm(gref[a:b]), (a, b)
+    loss2, g2 = net.gradients(X, Y)
+    assert loss2 == loss and np.array_equal(g2, g)
+
+
 def test_training_samples_follow_the_return_mapping(net):
     """Every generated sample is the plain return mapping (oracle) of its own
     inputs: stress and consistent tangent at (eps, epsp_n, kappa_n)."""
