@@ -15,6 +15,8 @@
 //   k_reduce_alpha alpha = rho / sum(p.q)                 (one block)
 //   k_pcg_update   x += alpha p; r -= alpha q; z = D^-1 r; partials r.z, r.r
 //   k_reduce_beta  convergence test, beta, rho            (one block)
+// On small systems, where launches count, the two reductions are done by
+// every workgroup of the kernel that follows: three launches (MERGE_MAX).
 // On request (hippcg_set_fused) p = z + beta p_old is formed inside the
 // SpMV gather instead and written by the row owner, saving the first launch;
 // on gfx950 that form is slower (the gather reads two vectors).  Summing the
@@ -49,6 +51,14 @@ namespace hipfem {
 constexpr int RED_THREADS = 1024;
 constexpr int MAX_GRID = 4096;
 constexpr int GRP_MAX_GRID = 16384;   // row-group and node-block PCG products: more resident workgroups
+// Up to this product grid the one-block reductions go into the kernels that
+// follow them (merged iteration), every workgroup summing all partials: the
+// launches saved are worth about 8 us an iteration, the sums cost grid^2.
+// Measured for a whole solve, five launches / merged: hex 6x6x22 (grid 198)
+// 5.47 / 4.25 ms, hex 16x16x64 (1088) 16.8 / 14.8, tet 35x35x41 (3300)
+// 33.5 / 33.2; beyond the limit hex 26x26x100 (9112) 49.7 / 54.5 and tet
+// 50x50x60 87.8 / 105.8.
+constexpr int MERGE_MAX = 4096;
 
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v)
@@ -429,6 +439,185 @@ __global__ __launch_bounds__(RED_THREADS) void k_reduce_beta(PcgState *st, const
     if (threadIdx.x == 0) step_beta(st, rz, rr, iter, hist, hist_cap);
 }
 
+// ---- merged iteration (small and middle sizes) ----
+// Three launches instead of five: the reductions are done by every block of
+// the kernel that needs their result, from the same partials in the same order
+// as the one-block kernels (the same bits).  The state alternates between two
+// slots, so that no block reads what another block of its launch writes: the
+// direction update of iteration i reads slot (i - 1) & 1 and writes slot i & 1,
+// which the product and the update of iteration i read.
+
+// Sums of K arrays of nb partials (array k at p + k nb) in the order of
+// reduce_partials, by 256 threads: thread t stands for t, t + 256, t + 512 and
+// t + 768.  load() takes the loads and the threads' sums, which do not wait
+// for the state; sum() gives every thread the result.
+template <int K>
+struct MergedSums {
+    double s[K][4];
+    __device__ __forceinline__ void load(const double *__restrict__ p, int nb)
+    {
+#pragma unroll
+        for (int k = 0; k < K; k++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) s[k][j] = 0.0;
+#pragma unroll 4
+        for (int i0 = threadIdx.x; i0 < nb; i0 += RED_THREADS) {
+            double v[K][4];
+#pragma unroll
+            for (int k = 0; k < K; k++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[k][j] = i0 + 256 * j < nb ? p[(size_t)k * nb + i0 + 256 * j] : 0.0;
+#pragma unroll
+            for (int k = 0; k < K; k++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) s[k][j] += v[k][j];
+        }
+    }
+    // sh: K x 16 doubles
+    __device__ __forceinline__ void sum(int nb, double *sh, double out[K])
+    {
+        const int nj = min(4, (nb + 255) / 256);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (j >= nj) break;
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                const double v = wave_sum(s[k][j]);
+                if (threadIdx.x % 64 == 0) sh[16 * k + 4 * j + threadIdx.x / 64] = v;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < K; k++) out[k] = 0.0;
+        for (int i = 0; i < 4 * nj; i++)
+#pragma unroll
+            for (int k = 0; k < K; k++) out[k] += sh[16 * k + i];
+    }
+};
+
+// The convergence test after iteration `iter` and the beta of the next one
+// (step_beta), from the state *in and the update's partials (v, loaded):
+// returns done, sets beta.  The first thread of the writer block stores the
+// new state in *out.  iter 0: the initial state passes on unchanged.
+__device__ __forceinline__ int merged_advance(const PcgState *__restrict__ in, PcgState *__restrict__ out,
+                                              MergedSums<2> &v, int nb, int iter, double *__restrict__ hist,
+                                              int hist_cap, bool writer, double *sh, double &beta)
+{
+    const double rho = in->rho, normb = in->normb, tol = in->tol;
+    int done = in->done;
+    const bool store = writer && threadIdx.x == 0;
+    beta = 0.0;
+    if (done || iter == 0) {
+        if (store) *out = *in;
+        return done;
+    }
+    double s2[2];
+    v.sum(nb, sh, s2);
+    const double rz = s2[0], res = sqrt(s2[1]) / normb;
+    const bool bad = !(res == res);
+    done = bad || res <= tol;
+    beta = rz / rho;
+    if (store) {
+        out->normb = normb;
+        out->tol = tol;
+        out->iter = iter;
+        out->res = res;
+        out->done = done;
+        out->bad = bad;
+        out->pause = out->restart = 0;
+        out->rho = done ? rho : rz;
+        out->beta = beta;
+        if (iter < hist_cap) hist[iter] = res;
+    }
+    return done;
+}
+
+// the check alone (one block), for the host at the end of a chunk
+__global__ __launch_bounds__(256) void k_merged_check(const PcgState *__restrict__ in, PcgState *__restrict__ out,
+                                                      const double *__restrict__ part, int nb, int iter,
+                                                      double *__restrict__ hist, int hist_cap)
+{
+    __shared__ double sh[2 * (RED_THREADS / 64)];
+    double beta;
+    MergedSums<2> v;
+    v.load(part, nb);
+    (void)merged_advance(in, out, v, nb, iter, hist, hist_cap, true, sh, beta);
+}
+
+// k_pcg_pupdate with beta from the update's partials
+template <typename VT>
+__global__ __launch_bounds__(256) void k_merged_pupdate(int n, const VT *__restrict__ z, VT *__restrict__ p,
+                                                        const PcgState *__restrict__ in, PcgState *__restrict__ out,
+                                                        const double *__restrict__ vpart, int nv, int it,
+                                                        double *__restrict__ hist, int hist_cap)
+{
+    __shared__ double sh[2 * (RED_THREADS / 64)];
+    MergedSums<2> v;
+    if (it > 1) v.load(vpart, nv);
+    // the thread's first entries are in flight with the partials and the state
+    int i = blockIdx.x * 256 + threadIdx.x;
+    VT zi = i < n ? z[i] : VT(0), pi = i < n && it > 1 ? p[i] : VT(0);
+    double b;
+    if (merged_advance(in, out, v, nv, it - 1, hist, hist_cap, blockIdx.x == 0, sh, b)) return;
+    const VT beta = (VT)b;
+    while (i < n) {
+        p[i] = it == 1 ? zi : fma(beta, pi, zi);
+        i += gridDim.x * 256;
+        if (i < n) {
+            zi = z[i];
+            pi = p[i];
+        }
+    }
+}
+
+// k_pcg_update with alpha from the product's partials
+template <typename XT, typename VT>
+__global__ __launch_bounds__(256) void k_merged_update(int n, XT *__restrict__ x, VT *__restrict__ r,
+                                                       VT *__restrict__ z, const VT *__restrict__ p,
+                                                       const VT *__restrict__ q, const VT *__restrict__ dinv,
+                                                       const PcgState *__restrict__ st,
+                                                       const double *__restrict__ spart, int ns,
+                                                       double *__restrict__ partials)
+{
+    __shared__ double sh[RED_THREADS / 64];
+    MergedSums<1> v;
+    v.load(spart, ns);
+    int i = blockIdx.x * 256 + threadIdx.x;
+    const bool any = i < n;
+    XT xi = any ? x[i] : XT(0);
+    VT pi = any ? p[i] : VT(0), qi = any ? q[i] : VT(0), ro = any ? r[i] : VT(0), di = any ? dinv[i] : VT(0);
+    const double rho = st->rho;
+    if (st->done) return;
+    double pq[1];
+    v.sum(ns, sh, pq);
+    const VT a = (VT)(rho / pq[0]);
+    double rz = 0.0, rr = 0.0;
+    while (i < n) {
+        x[i] = fma((XT)a, (XT)pi, xi);
+        const VT ri = fma(-a, qi, ro);
+        r[i] = ri;
+        const VT zi = di * ri;
+        z[i] = zi;
+        rz += (double)ri * (double)zi;
+        rr += (double)ri * (double)ri;
+        i += gridDim.x * 256;
+        if (i < n) {
+            xi = x[i];
+            pi = p[i];
+            qi = q[i];
+            ro = r[i];
+            di = dinv[i];
+        }
+    }
+    __syncthreads();   // sh
+    const double s1 = block_sum<256>(rz, sh);
+    const double s2 = block_sum<256>(rr, sh);
+    if (threadIdx.x == 0) {
+        partials[blockIdx.x] = s1;
+        partials[gridDim.x + blockIdx.x] = s2;
+    }
+}
+
 __global__ void k_dinv(int n, const int32_t *__restrict__ diag, const double *__restrict__ val, int use_diag,
                        double *__restrict__ dinv, float *__restrict__ dinv32, int *__restrict__ zero_row)
 {
@@ -750,7 +939,7 @@ static int solver_alloc(hippcg_solver *s, int n)
     const size_t nd = sizeof(double) * std::max(1, n), nf = sizeof(float) * std::max(1, n);
     for (double **p : {&s->dinv, &s->r, &s->z, &s->p0, &s->p1, &s->q, &s->hx, &s->hb}) HIPFEM_CHECK(hipMalloc(p, nd));
     for (float **p : {&s->dinv32, &s->fr, &s->fz, &s->fp0, &s->fp1, &s->fq, &s->fx, &s->fb}) HIPFEM_CHECK(hipMalloc(p, nf));
-    HIPFEM_CHECK(hipMalloc(&s->st, sizeof(PcgState)));
+    HIPFEM_CHECK(hipMalloc(&s->st, 2 * sizeof(PcgState)));   // two slots: the merged iteration alternates
     HIPFEM_CHECK(hipMalloc(&s->zero_row, sizeof(int)));
     HIPFEM_CHECK(hipMalloc(&s->scal, 2 * sizeof(double)));
     s->n = n;
@@ -841,7 +1030,9 @@ static int pcg_run(hippcg_solver *s, const PcgRunBufs &bufs, hipcsr_mtx *A, cons
     // p = z + beta p formed in the product's gather (the lane, node-block
     // and row-group forms), or in a pass of its own
     const bool fused = s->fused && !sh.stream;
-    const size_t need = 3 * (size_t)std::max(gv, gs);
+    const bool merged = (nodeblock || grouped) && !s->fused && gs <= MERGE_MAX;
+    // the merged form keeps the product's partials apart from the update's
+    const size_t need = 3 * (size_t)std::max(gv, gs) + (merged ? gs : 0);
     double *part = bufs.part;
     int rc = 0;
     if (!part) {
@@ -885,6 +1076,26 @@ static int pcg_run(hippcg_solver *s, const PcgRunBufs &bufs, hipcsr_mtx *A, cons
             rc = ensure_events(s, (size_t)stop);
             if (rc) return rc;
         }
+        for (; merged && it <= stop; it++) {
+            double *const spart = part + 3 * (size_t)std::max(gv, gs);
+            PcgState *cur = pst + (it & 1);
+            k_merged_pupdate<VT><<<gv, 256, 0, st>>>(n, z, p0, pst + ((it - 1) & 1), cur, part, gv, it, bufs.hist,
+                                                     bufs.hist_cap);
+            if (prof) HIPFEM_CHECK(hipEventRecord(s->ev[2 * (it - 1)], st));
+            if (nodeblock)
+                k_pcg_spmv_p_nb<VT, MT, false><<<gs, 256, 0, st>>>(A->nbr, A->d_bptr, A->d_bcol, val, p0, z, nullptr, q,
+                                                                   cur, spart, 0);
+            else
+                k_pcg_spmv_p_grp<VT, MT, false><<<gs, 256, 0, st>>>(A->ngrp, A->d_grow, A->d_gch, A->d_ccol,
+                                                                    A->d_rowptr, val, p0, z, nullptr, q, cur, spart, 0);
+            if (prof) HIPFEM_CHECK(hipEventRecord(s->ev[2 * (it - 1) + 1], st));
+            k_merged_update<XT, VT><<<gv, 256, 0, st>>>(n, x, r, z, p0, q, dinv, cur, spart, gs, part);
+        }
+        // the check of the chunk's last iteration, into the slot that the next
+        // direction update overwrites
+        if (merged)
+            k_merged_check<<<1, 256, 0, st>>>(pst + (stop & 1), pst + ((stop + 1) & 1), part, gv, stop, bufs.hist,
+                                              bufs.hist_cap);
         for (; it <= stop; it++) {
             const int first = (it == 1);
             if (!fused) k_pcg_pupdate<VT><<<gv, 256, 0, st>>>(n, z, p0, pst, first);
@@ -921,7 +1132,7 @@ static int pcg_run(hippcg_solver *s, const PcgRunBufs &bufs, hipcsr_mtx *A, cons
             if (fused) std::swap(pold, pnew);
         }
         HIPFEM_CHECK(hipGetLastError());
-        rc = read_state_at(s->ctx, pst, &h);
+        rc = read_state_at(s->ctx, merged ? pst + ((stop + 1) & 1) : pst, &h);
         if (rc) return rc;
         if (h.done) break;
         chunk = std::min(chunk * 2, 64);
@@ -1172,12 +1383,12 @@ static int solve_dev(hippcg_solver *s, hipcsr_mtx *A, const double *db, double *
 // and the zero-diagonal flag.  Host code never uses the array's name as an
 // address: it takes the device's address once from hipGetSymbolAddress.
 constexpr size_t NA_N = HIPPCG_NOALLOC_MAX_N;
-constexpr size_t NA_PART = 3 * (size_t)std::max(MAX_GRID, GRP_MAX_GRID);
+constexpr size_t NA_PART = 4 * (size_t)std::max(MAX_GRID, GRP_MAX_GRID);
 constexpr size_t NA_OFF_PART = 6 * NA_N * sizeof(double);
 constexpr size_t NA_OFF_STATE = NA_OFF_PART + NA_PART * sizeof(double);
 constexpr size_t NA_OFF_FLAG = NA_OFF_STATE + 256;
 constexpr size_t NA_BYTES = NA_OFF_FLAG + 256;
-static_assert(sizeof(PcgState) <= 256, "PcgState exceeds its scratch slot");
+static_assert(2 * sizeof(PcgState) <= 256, "the two states exceed their scratch slot");
 static __device__ __align__(256) unsigned char scratch[NA_BYTES];
 
 static std::mutex na_mutex;

@@ -117,6 +117,36 @@ def test_spmv_shapes_match_oracle(ctx, name, shape):
         assert np.linalg.norm(u - uo) <= 1e-9 * np.linalg.norm(uo)
 
 
+@pytest.mark.parametrize("name,form", [("lspace", 1), ("qspace", 2)])
+@pytest.mark.parametrize("maxit", [0, 1, 15, 16, 17, 48, 20000])
+def test_merged_iteration_matches_separate_reductions(ctx, name, form, maxit):
+    """The small-system iteration whose reductions sit in the kernels that
+    follow them, stopped around the host's chunks of 16 and 32, from a
+    non-zero guess: bit for bit the iteration with one-block reductions, which
+    the in-gather direction keeps (same partials, same order)."""
+    from oofem_amd.hipfem import HipCSRSparseMtrx, HipPCGSolver
+    d = SHAPE_DECKS[name]
+    rp, ci, val = oracle.csr(d)
+    K = HipCSRSparseMtrx(ctx)
+    K.buildInternalStructureCSR(rp, ci)
+    K.upload_values(val)
+    assert K.is_nodeblocked() == form
+    rng = np.random.default_rng(4)
+    b, x0 = rng.standard_normal(d.neq), 1e-6 * rng.standard_normal(d.neq)
+    out = []
+    for fused in (0, 1):
+        s = HipPCGSolver(ctx, lstol=1e-10, lsiter=maxit, lsprecond=1)
+        s.set_fused(fused)
+        s.set_history(20001)
+        x = x0.copy()
+        reason, it, res = s.solve(K, b, x)
+        out.append((reason, it, res, x, s.history()))
+    (ra, ia, ea, xa, ha), (rb, ib, eb, xb, hb) = out
+    assert (ra, ia, ea) == (rb, ib, eb)
+    assert (ra == 1) == (maxit == 20000) and ia <= maxit
+    assert np.array_equal(xa, xb) and np.array_equal(ha, hb)
+
+
 def test_config0_linear_static_parity(ctx):
     from oofem_amd.drivers import linear_static, reaction_sums
     d = meshgen.config0()
