@@ -26,10 +26,11 @@
 // are therefore solved first, together, in a bulk-synchronous phase: every
 // launch covers all their rows in tiles of TILE_ROWS rows (one workgroup
 // each, the whole GPU; the products use a 3x3 node-block form when the
-// pattern has one), per-tile partial dots are summed per block by a
-// reduction launch, and the same per-column scalars, reliable updates and
+// pattern has one), and the same per-column scalars, reliable updates and
 // stopping rule as the persistent kernel live in a BulkBlock record per
-// block.  Finished blocks drop out of the tile list when the host next looks
+// block.  An iteration is four launches: every workgroup of a block sums the
+// block's tile partials itself at the start of the kernel that needs them,
+// and the block's first one writes the record, to the other of two places.  Finished blocks drop out of the tile list when the host next looks
 // (every BULK_CHECK iterations); until then their tiles return at once.
 
 #include <algorithm>
@@ -286,7 +287,6 @@ constexpr int NPART = 2 * NRHS;  // partial sums per tile
 
 struct BulkBlock {
     double rho[NRHS], normb[NRHS], rmax[NRHS], res[NRHS];
-    float alpha[NRHS], beta[NRHS];
     int conv;      // bit k: column k meets the tolerance
     int it, nupd;
     int refresh;   // 1: this iteration replaces the residuals by b - A x
@@ -295,10 +295,13 @@ struct BulkBlock {
 };
 
 struct BulkArgs {
-    const int4 *tiles;       // {first row, end row, bulk index, 0}; node-aligned in the node-block form
+    const int4 *tiles;       // {first row, end row, bulk index, position in act}; node-aligned in the node-block form
     const int *act;          // bulk indices of the blocks in the tile list
     const int *act_t0;       // their tile ranges [act_t0[a], act_t0[a + 1])
-    BulkBlock *st;
+    // block states: st is what the product, the update and the step read and
+    // the finish writes, st1 the other way round, so that no workgroup reads
+    // what another of its launch writes
+    BulkBlock *st, *st1;
     const int32_t *rowptr, *col;
     const int32_t *bptr, *bcol;  // node-block view (node rows, block columns) when the pattern has one
     const float4 *vwide;         // wide form: FP32 values block-major, 12 floats per block
@@ -307,7 +310,7 @@ struct BulkArgs {
     const double *b;
     double *x;
     float *r, *z, *p, *q;
-    double *part;            // [tile][NPART]
+    double *part, *part_rz, *part_tr;   // [tile][NPART]: p.q; r.z and r.r; those of a reliable update
     double tol, delta;
     int maxit;
     int *iters, *updates;
@@ -339,7 +342,7 @@ __global__ __launch_bounds__(BULK_TILE) void k_bulk_init(BulkArgs A)
             v[NRHS + k] = bi * bi;
         }
     }
-    block_sums<BULK_TILE, NPART>(v, sh, A.part + (size_t)blockIdx.x * NPART);
+    block_sums<BULK_TILE, NPART>(v, sh, A.part_rz + (size_t)blockIdx.x * NPART);
 }
 
 // q = A p (FP32) for the tile's rows, LPR lanes per row; partials p.q
@@ -388,13 +391,33 @@ __global__ __launch_bounds__(BULK_TILE) void k_bulk_spmv(BulkArgs A)
     block_sums<BULK_TILE, NRHS>(v, sh, A.part + (size_t)blockIdx.x * NPART);
 }
 
-// x += alpha p (FP64), r -= alpha q, z = D^-1 r; partials r.z and r.r
+// The sums of a block's tile partials, by every workgroup of the block that
+// needs them (256 threads, a fixed order): no launch of its own for the
+// reductions, whose cost was its latency
+template <int NV>
+__device__ __forceinline__ void tile_sums(const BulkArgs &A, int pos, const double *__restrict__ part, double *sh,
+                                          double *red)
+{
+    double v[NV];
+#pragma unroll
+    for (int k = 0; k < NV; k++) v[k] = 0.0;
+    for (int ti = A.act_t0[pos] + threadIdx.x; ti < A.act_t0[pos + 1]; ti += BULK_TILE)
+#pragma unroll
+        for (int k = 0; k < NV; k++) v[k] += part[(size_t)ti * NPART + k];
+    block_sums<BULK_TILE, NV>(v, sh, red);
+}
+
+// alpha from the product's partials (0 for a converged column and where the
+// curvature p.q is not positive), then x += alpha p (FP64), r -= alpha q,
+// z = D^-1 r; partials r.z and r.r
 __global__ __launch_bounds__(BULK_TILE) void k_bulk_update(BulkArgs A)
 {
     __shared__ double sh[NPART * (BULK_TILE / 64)];
+    __shared__ double red[NRHS];
     const int4 t = A.tiles[blockIdx.x];
     const BulkBlock &S = A.st[t.z];
     if (S.done) return;
+    tile_sums<NRHS>(A, t.w, A.part, sh, red);
     double v[NPART];
 #pragma unroll
     for (int k = 0; k < NPART; k++) v[k] = 0.0;
@@ -404,7 +427,7 @@ __global__ __launch_bounds__(BULK_TILE) void k_bulk_update(BulkArgs A)
 #pragma unroll
         for (int k = 0; k < NRHS; k++) {
             const size_t o = (size_t)i * NRHS + k;
-            const float al = S.alpha[k];
+            const float al = (!(S.conv >> k & 1) && red[k] > 0.0) ? (float)(S.rho[k] / red[k]) : 0.f;
             A.x[o] += (double)al * (double)A.p[o];
             const float ri = fmaf(-al, A.q[o], A.r[o]);
             A.r[o] = ri;
@@ -414,18 +437,121 @@ __global__ __launch_bounds__(BULK_TILE) void k_bulk_update(BulkArgs A)
             v[NRHS + k] = (double)ri * (double)ri;
         }
     }
-    block_sums<BULK_TILE, NPART>(v, sh, A.part + (size_t)blockIdx.x * NPART);
+    block_sums<BULK_TILE, NPART>(v, sh, A.part_rz + (size_t)blockIdx.x * NPART);
 }
 
-// reliable update for the tiles of blocks that asked for one:
+__device__ void bulk_finish(const BulkArgs &A, BulkBlock &S, bool all)
+{
+    double mx = 0.0;
+    for (int k = 0; k < NRHS; k++) mx = fmax(mx, S.res[k]);
+    A.iters[S.blk] = S.it;
+    A.updates[S.blk] = S.nupd;
+    A.resid[S.blk] = all ? mx : -mx;
+    S.done = 1;
+}
+
+// p = z + beta p of the tile's rows
+__device__ __forceinline__ void tile_direction(const BulkArgs &A, const int4 &t, const float beta[NRHS])
+{
+    const int i = t.x + threadIdx.x;
+    if (i >= t.y) return;
+#pragma unroll
+    for (int k = 0; k < NRHS; k++) {
+        const size_t o = (size_t)i * NRHS + k;
+        A.p[o] = fmaf(beta[k], A.p[o], A.z[o]);
+    }
+}
+
+// After the update: does the block ask for a reliable update (a residual met
+// the tolerance or dropped by delta)?  Returns true for its tiles if so, which
+// then form b - A x; else the direction is updated here.  The block's first
+// tile writes the new state to st1.
+__device__ __forceinline__ bool bulk_step(const BulkArgs &A, const int4 &t, double *sh, double *red)
+{
+    const BulkBlock &S = A.st[t.z];
+    const bool writer = (int)blockIdx.x == A.act_t0[t.w] && threadIdx.x == 0;
+    if (S.done) {
+        if (writer) A.st1[t.z] = S;
+        return false;
+    }
+    tile_sums<NPART>(A, t.w, A.part_rz, sh, red);
+    bool refresh = false;
+    double res[NRHS];
+    float beta[NRHS];
+#pragma unroll
+    for (int k = 0; k < NRHS; k++) {
+        const bool c = S.conv >> k & 1;
+        res[k] = sqrt(red[NRHS + k]) / S.normb[k];
+        if (!c && (res[k] <= A.tol || res[k] < A.delta * S.rmax[k])) refresh = true;
+        beta[k] = c ? 0.f : (float)(red[k] / S.rho[k]);
+    }
+    if (writer) {
+        BulkBlock &N = A.st1[t.z];
+        N = S;
+        N.it = S.it + 1;
+        N.refresh = refresh;
+#pragma unroll
+        for (int k = 0; k < NRHS; k++) {
+            N.res[k] = res[k];
+            if (!refresh && !(S.conv >> k & 1)) N.rho[k] = red[k];
+        }
+        if (!refresh && N.it >= A.maxit) bulk_finish(A, N, false);
+    }
+    if (!refresh) tile_direction(A, t, beta);
+    return refresh;
+}
+
+// After a reliable update: beta from the true residual and the direction; for
+// every block its first tile brings the state back to st
+__global__ __launch_bounds__(BULK_TILE) void k_bulk_finish(BulkArgs A)
+{
+    __shared__ double sh[NPART * (BULK_TILE / 64)];
+    __shared__ double red[NPART];
+    const int4 t = A.tiles[blockIdx.x];
+    const BulkBlock &S = A.st1[t.z];
+    const bool writer = (int)blockIdx.x == A.act_t0[t.w] && threadIdx.x == 0;
+    if (S.done || !S.refresh) {
+        if (writer) A.st[t.z] = S;
+        return;
+    }
+    tile_sums<NPART>(A, t.w, A.part_tr, sh, red);
+    bool all = true;
+    int conv = 0;
+    double res[NRHS];
+    float beta[NRHS];
+#pragma unroll
+    for (int k = 0; k < NRHS; k++) {
+        res[k] = sqrt(red[NRHS + k]) / S.normb[k];
+        const bool c = res[k] <= A.tol;
+        if (c) conv |= 1 << k;
+        all = all && c;
+        beta[k] = c ? 0.f : (float)(red[k] / S.rho[k]);
+    }
+    if (writer) {
+        BulkBlock &N = A.st[t.z];
+        N = S;
+        N.nupd = S.nupd + 1;
+        N.conv = conv;
+        N.refresh = 0;
+#pragma unroll
+        for (int k = 0; k < NRHS; k++) {
+            N.res[k] = N.rmax[k] = res[k];
+            N.rho[k] = red[k];
+        }
+        if (all || N.it >= A.maxit) bulk_finish(A, N, all);
+    }
+    tile_direction(A, t, beta);
+}
+
+// bulk_step, and for the tiles of blocks that ask for a reliable update
 // r = b - A x (FP64 values and solution), z = D^-1 r; partials r.z and |r|^2
 template <int LPR>
 __global__ __launch_bounds__(BULK_TILE) void k_bulk_refresh(BulkArgs A)
 {
     __shared__ double sh[NPART * (BULK_TILE / 64)];
+    __shared__ double red[NPART];
     const int4 t = A.tiles[blockIdx.x];
-    const BulkBlock &S = A.st[t.z];
-    if (S.done || !S.refresh) return;
+    if (!bulk_step(A, t, sh, red)) return;
     double v[NPART];
 #pragma unroll
     for (int k = 0; k < NPART; k++) v[k] = 0.0;
@@ -468,7 +594,7 @@ __global__ __launch_bounds__(BULK_TILE) void k_bulk_refresh(BulkArgs A)
             }
         }
     }
-    block_sums<BULK_TILE, NPART>(v, sh, A.part + (size_t)blockIdx.x * NPART);
+    block_sums<BULK_TILE, NPART>(v, sh, A.part_tr + (size_t)blockIdx.x * NPART);
 }
 
 // Node-block forms of the two products, for patterns whose rows come in
@@ -653,14 +779,15 @@ __global__ void k_bulk_widen(int nbr, const int32_t *__restrict__ bptr, const fl
     }
 }
 
-// reliable update in the node-block form: r = b - A x (FP64), z = D^-1 r
+// bulk_step and the reliable update in the node-block form: r = b - A x (FP64),
+// z = D^-1 r
 template <int LPR>
 __global__ __launch_bounds__(BULK_TILE) void k_bulk_refresh_nb(BulkArgs A)
 {
     __shared__ double sh[NPART * (BULK_TILE / 64)];
+    __shared__ double red[NPART];
     const int4 t = A.tiles[blockIdx.x];
-    const BulkBlock &S = A.st[t.z];
-    if (S.done || !S.refresh) return;
+    if (!bulk_step(A, t, sh, red)) return;
     double v[NPART];
 #pragma unroll
     for (int k = 0; k < NPART; k++) v[k] = 0.0;
@@ -684,107 +811,32 @@ __global__ __launch_bounds__(BULK_TILE) void k_bulk_refresh_nb(BulkArgs A)
             }
         }
     }
-    block_sums<BULK_TILE, NPART>(v, sh, A.part + (size_t)blockIdx.x * NPART);
+    block_sums<BULK_TILE, NPART>(v, sh, A.part_tr + (size_t)blockIdx.x * NPART);
 }
 
-// p = z + beta p
-__global__ __launch_bounds__(BULK_TILE) void k_bulk_pupdate(BulkArgs A)
+// one workgroup per block: the initial scalars from the init partials
+__global__ __launch_bounds__(BULK_TILE) void k_bulk_start(BulkArgs A)
 {
-    const int4 t = A.tiles[blockIdx.x];
-    const BulkBlock &S = A.st[t.z];
-    if (S.done) return;
-    const int i = t.x + threadIdx.x;
-    if (i < t.y) {
-#pragma unroll
-        for (int k = 0; k < NRHS; k++) {
-            const size_t o = (size_t)i * NRHS + k;
-            A.p[o] = fmaf(S.beta[k], A.p[o], A.z[o]);
-        }
-    }
-}
-
-enum BulkPhase { BP_INIT, BP_ALPHA, BP_BETA, BP_REFRESH };
-
-__device__ void bulk_finish(const BulkArgs &A, BulkBlock &S, bool all)
-{
-    double mx = 0.0;
-    for (int k = 0; k < NRHS; k++) mx = fmax(mx, S.res[k]);
-    A.iters[S.blk] = S.it;
-    A.updates[S.blk] = S.nupd;
-    A.resid[S.blk] = all ? mx : -mx;
-    S.done = 1;
-}
-
-// one workgroup per block of the tile list: sum the block's tile partials
-// and advance its scalars (the same rules as k_batch_pcg)
-template <int PHASE>
-__global__ __launch_bounds__(256) void k_bulk_reduce(BulkArgs A)
-{
-    __shared__ double sh[NPART * 4];
+    __shared__ double sh[NPART * (BULK_TILE / 64)];
     __shared__ double red[NPART];
     BulkBlock &S = A.st[A.act[blockIdx.x]];
-    if (S.done) return;
-    if (PHASE == BP_REFRESH && !S.refresh) return;
-    constexpr int NV = PHASE == BP_ALPHA ? NRHS : NPART;
-    double v[NV];
-#pragma unroll
-    for (int k = 0; k < NV; k++) v[k] = 0.0;
-    for (int ti = A.act_t0[blockIdx.x] + threadIdx.x; ti < A.act_t0[blockIdx.x + 1]; ti += 256)
-#pragma unroll
-        for (int k = 0; k < NV; k++) v[k] += A.part[(size_t)ti * NPART + k];
-    block_sums<256, NV>(v, sh, red);
+    tile_sums<NPART>(A, blockIdx.x, A.part_rz, sh, red);
     if (threadIdx.x != 0) return;
-    if (PHASE == BP_INIT) {
-        bool all = true;
-        S.conv = 0;
-        for (int k = 0; k < NRHS; k++) {
-            S.rho[k] = red[k];
-            const double nb = sqrt(red[NRHS + k]);
-            S.normb[k] = nb == 0.0 ? 1.0 : nb;
-            S.res[k] = nb / S.normb[k];
-            S.rmax[k] = S.res[k];
-            if (S.res[k] <= A.tol) S.conv |= 1 << k;
-            all = all && (S.conv >> k & 1);
-        }
-        S.it = 0;
-        S.nupd = 0;
-        S.refresh = 0;
-        if (all || A.maxit <= 0) bulk_finish(A, S, all);
-    } else if (PHASE == BP_ALPHA) {
-        S.it++;
-        for (int k = 0; k < NRHS; k++)
-            S.alpha[k] = (!(S.conv >> k & 1) && red[k] > 0.0) ? (float)(S.rho[k] / red[k]) : 0.f;
-    } else if (PHASE == BP_BETA) {
-        bool refresh = false;
-        for (int k = 0; k < NRHS; k++) {
-            S.res[k] = sqrt(red[NRHS + k]) / S.normb[k];
-            if (!(S.conv >> k & 1) && (S.res[k] <= A.tol || S.res[k] < A.delta * S.rmax[k])) refresh = true;
-        }
-        S.refresh = refresh;
-        if (!refresh) {
-            for (int k = 0; k < NRHS; k++) {
-                const bool c = S.conv >> k & 1;
-                S.beta[k] = c ? 0.f : (float)(red[k] / S.rho[k]);
-                if (!c) S.rho[k] = red[k];
-            }
-            if (S.it >= A.maxit) bulk_finish(A, S, false);
-        }
-    } else {
-        S.nupd++;
-        bool all = true;
-        S.conv = 0;
-        for (int k = 0; k < NRHS; k++) {
-            S.res[k] = sqrt(red[NRHS + k]) / S.normb[k];
-            const bool c = S.res[k] <= A.tol;
-            if (c) S.conv |= 1 << k;
-            all = all && c;
-            S.beta[k] = c ? 0.f : (float)(red[k] / S.rho[k]);
-            S.rho[k] = red[k];
-            S.rmax[k] = S.res[k];
-        }
-        S.refresh = 0;
-        if (all || S.it >= A.maxit) bulk_finish(A, S, all);
+    bool all = true;
+    S.conv = 0;
+    for (int k = 0; k < NRHS; k++) {
+        S.rho[k] = red[k];
+        const double nb = sqrt(red[NRHS + k]);
+        S.normb[k] = nb == 0.0 ? 1.0 : nb;
+        S.res[k] = nb / S.normb[k];
+        S.rmax[k] = S.res[k];
+        if (S.res[k] <= A.tol) S.conv |= 1 << k;
+        all = all && (S.conv >> k & 1);
     }
+    S.it = 0;
+    S.nupd = 0;
+    S.refresh = 0;
+    if (all || A.maxit <= 0) bulk_finish(A, S, all);
 }
 
 typedef void (*bulk_kernel_t)(BulkArgs);
@@ -935,11 +987,11 @@ extern "C" int hfem_batch_create(hipcsr_mtx *A, int nblocks, const int32_t *rows
         hipMalloc(&bt->d_ctl, sizeof(BatchCtl)) != hipSuccess || hipMalloc(&bt->d_iters, sizeof(int) * nblocks) != hipSuccess ||
         hipMalloc(&bt->d_upd, sizeof(int) * nblocks) != hipSuccess || hipMalloc(&bt->d_zero, sizeof(int)) != hipSuccess ||
         hipMalloc(&bt->d_res, sizeof(double) * nblocks) != hipSuccess ||
-        hipMalloc(&bt->d_bst, sizeof(BulkBlock) * nblocks) != hipSuccess ||
+        hipMalloc(&bt->d_bst, 2 * sizeof(BulkBlock) * nblocks) != hipSuccess ||
         hipMalloc(&bt->d_tiles, sizeof(int4) * bt->tiles_cap) != hipSuccess ||
         hipMalloc(&bt->d_act, sizeof(int) * nblocks) != hipSuccess ||
         hipMalloc(&bt->d_act_t0, sizeof(int) * (nblocks + 1)) != hipSuccess ||
-        hipMalloc(&bt->d_part, sizeof(double) * NPART * bt->tiles_cap) != hipSuccess) {
+        hipMalloc(&bt->d_part, 3 * sizeof(double) * NPART * bt->tiles_cap) != hipSuccess) {
         set_error("hfem_batch_create: out of device memory");
         return fail(HIPFEM_ENOMEM);
     }
@@ -1143,11 +1195,11 @@ static int bulk_tiles(hfem_batch *bt, const std::vector<int> &act)
         bt->tile_bytes += !nb ? 8.0 * nnz + 4.0 * rows + 48.0 * rows
                           : (bt->wide ? 16.0 / 3.0 : 4.0) * nnz + 4.0 * nnz / 9.0 + 4.0 * rows / 3.0 + 48.0 * rows;
     }
-    for (int a : act) {
-        const int blk = bt->h_bulk[a];
+    for (size_t pos = 0; pos < act.size(); pos++) {
+        const int a = act[pos], blk = bt->h_bulk[a];
         bt->h_act_t0.push_back((int)bt->h_tiles.size());
         for (int r = bt->h_rows[blk]; r < bt->h_rows[blk + 1]; r += TILE_ROWS)
-            bt->h_tiles.push_back(make_int4(r, std::min(r + TILE_ROWS, bt->h_rows[blk + 1]), a, 0));
+            bt->h_tiles.push_back(make_int4(r, std::min(r + TILE_ROWS, bt->h_rows[blk + 1]), a, (int)pos));
     }
     bt->h_act_t0.push_back((int)bt->h_tiles.size());
     HIPFEM_REQUIRE((int)bt->h_tiles.size() <= bt->tiles_cap, HIPFEM_EINVAL, "bulk tiles exceed their capacity");
@@ -1179,6 +1231,7 @@ static int bulk_solve(hfem_batch *bt, const double *db, double *dx, int maxit)
     A.act = bt->d_act;
     A.act_t0 = bt->d_act_t0;
     A.st = bt->d_bst;
+    A.st1 = bt->d_bst + bt->nblocks;
     A.rowptr = M->d_rowptr;
     A.col = M->d_colind;
     A.bptr = M->d_bptr;
@@ -1193,6 +1246,8 @@ static int bulk_solve(hfem_batch *bt, const double *db, double *dx, int maxit)
     A.p = bt->d_p;
     A.q = bt->d_q;
     A.part = bt->d_part;
+    A.part_rz = A.part + (size_t)NPART * bt->tiles_cap;
+    A.part_tr = A.part_rz + (size_t)NPART * bt->tiles_cap;
     A.tol = bt->tol;
     A.delta = bt->delta;
     A.maxit = maxit;
@@ -1212,9 +1267,10 @@ static int bulk_solve(hfem_batch *bt, const double *db, double *dx, int maxit)
     A.vwide = reinterpret_cast<const float4 *>(bt->d_vwide);
     const bulk_kernel_t spmv = wide ? sh.spmv_nbw : nb ? sh.spmv_nb : sh.spmv;
     const bulk_kernel_t refresh = nb ? sh.refresh_nb : sh.refresh;
-    int ntiles = (int)bt->h_tiles.size(), nact = nbulk;
+    int ntiles = (int)bt->h_tiles.size();
+    const int nact = nbulk;
     k_bulk_init<<<ntiles, BULK_TILE, 0, st>>>(A);
-    k_bulk_reduce<BP_INIT><<<nact, 256, 0, st>>>(A);
+    k_bulk_start<<<nact, BULK_TILE, 0, st>>>(A);
     HIPFEM_CHECK(hipGetLastError());
     // every block is done once maxit iterations have run: the loop ends by then
     for (int it = 0;; it++) {
@@ -1242,19 +1298,15 @@ static int bulk_solve(hfem_batch *bt, const double *db, double *dx, int maxit)
                 rc = bulk_tiles(bt, act);
                 if (rc) return rc;
                 ntiles = (int)bt->h_tiles.size();
-                nact = (int)act.size();
             }
         }
         const bool timed = bt->profiling && bt->ev_used < BULK_CHECK;
         if (timed) HIPFEM_CHECK(hipEventRecord(bt->ev[2 * bt->ev_used], st));
         hipLaunchKernelGGL(spmv, dim3(ntiles), dim3(BULK_TILE), 0, st, A);
         if (timed) HIPFEM_CHECK(hipEventRecord(bt->ev[2 * bt->ev_used++ + 1], st));
-        k_bulk_reduce<BP_ALPHA><<<nact, 256, 0, st>>>(A);
         k_bulk_update<<<ntiles, BULK_TILE, 0, st>>>(A);
-        k_bulk_reduce<BP_BETA><<<nact, 256, 0, st>>>(A);
         hipLaunchKernelGGL(refresh, dim3(ntiles), dim3(BULK_TILE), 0, st, A);
-        k_bulk_reduce<BP_REFRESH><<<nact, 256, 0, st>>>(A);
-        k_bulk_pupdate<<<ntiles, BULK_TILE, 0, st>>>(A);
+        k_bulk_finish<<<ntiles, BULK_TILE, 0, st>>>(A);
         HIPFEM_CHECK(hipGetLastError());
     }
     return 0;
