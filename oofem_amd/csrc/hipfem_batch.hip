@@ -29,9 +29,11 @@
 // pattern has one), and the same per-column scalars, reliable updates and
 // stopping rule as the persistent kernel live in a BulkBlock record per
 // block.  An iteration is four launches: every workgroup of a block sums the
-// block's tile partials itself at the start of the kernel that needs them,
-// and the block's first one writes the record, to the other of two places.  Finished blocks drop out of the tile list when the host next looks
-// (every BULK_CHECK iterations); until then their tiles return at once.
+// block's tile partials itself at the start of the kernel that needs them
+// (large blocks: a launch for it, FOLD_TILES), and the block's first one
+// writes the record, to the other of two places.  Finished blocks drop out of
+// the tile list when the host next looks (every BULK_CHECK iterations); until
+// then their tiles return at once.
 
 #include <algorithm>
 #include <cmath>
@@ -281,7 +283,20 @@ __global__ __launch_bounds__(BS) void k_batch_pcg(int nblocks, const int *__rest
 
 // ------------------------------------------------------------ bulk phase
 constexpr int BULK_TILE = 256;   // threads per workgroup
-constexpr int TILE_ROWS = 255;   // rows per tile: 85 whole nodes, one row per thread
+// rows per tile: 32 whole nodes, eight lanes each; two threads per row
+// elsewhere.  24 RVEs of n = 8 to 16, all six solves: 96 rows 29.4 ms, 255
+// rows (85 nodes in three uneven passes, 1.7 workgroups per CU) 37.2, 126
+// rows 32.6 (before the loads of the sums were batched, where 96 took 31.9),
+// 48 rows 36.2 (twice the partials to sum).
+constexpr int TILE_ROWS = 96;
+constexpr int SUM_GROUPS = 21;   // BULK_TILE / NPART
+// Blocks of up to FOLD_TILES tiles are summed by each of their workgroups;
+// beyond it, where that costs tiles^2, by a launch per sum.  Measured for one
+// RVE's six solves, summed by all / by a launch / with seven launches and tiles
+// of 255 rows: LSpace n = 16 (105 tiles) 3.3 / 3.9 / 5.9 ms, QSpace 16 (442)
+// 15.1 / 17.3 / 23.4, LSpace 32 (930) 13.0 / 13.6 / 14.3, QSpace 22 (1198)
+// 41.4 / 41.3 / 41.1, LSpace 48 (3244) 65 / 40.6 / 40.6.
+constexpr int FOLD_TILES = 1024;
 constexpr int BULK_CHECK = 16;   // iterations between host looks at the done flags
 constexpr int NPART = 2 * NRHS;  // partial sums per tile
 
@@ -311,6 +326,7 @@ struct BulkArgs {
     double *x;
     float *r, *z, *p, *q;
     double *part, *part_rz, *part_tr;   // [tile][NPART]: p.q; r.z and r.r; those of a reliable update
+    int fold;                // the partials of a block are summed into its first tile's by a launch of their own
     double tol, delta;
     int maxit;
     int *iters, *updates;
@@ -392,52 +408,90 @@ __global__ __launch_bounds__(BULK_TILE) void k_bulk_spmv(BulkArgs A)
 }
 
 // The sums of a block's tile partials, by every workgroup of the block that
-// needs them (256 threads, a fixed order): no launch of its own for the
-// reductions, whose cost was its latency
-template <int NV>
-__device__ __forceinline__ void tile_sums(const BulkArgs &A, int pos, const double *__restrict__ part, double *sh,
+// needs them (a fixed order): no launch of its own for the reductions, whose
+// cost (5 to 7 us each) was its latency.  A thread sums one value over every SUM_GROUPS-th tile
+// (coalesced, no wave reduction), then one thread per value sums the groups.
+template <int NV, int G = SUM_GROUPS>
+__device__ __forceinline__ void tile_sums(const BulkArgs &A, int pos, const double *part, bool fold, double *sh,
                                           double *red)
 {
-    double v[NV];
+    const int g = threadIdx.x / NV, k = threadIdx.x % NV;
+    if (g < G) {
+        double s = 0.0;
+        const int t0 = A.act_t0[pos], t1 = fold ? t0 + 1 : A.act_t0[pos + 1];
+        for (int ti = t0 + g; ti < t1; ti += 8 * G) {   // eight loads in flight
+            double w[8];
 #pragma unroll
-    for (int k = 0; k < NV; k++) v[k] = 0.0;
-    for (int ti = A.act_t0[pos] + threadIdx.x; ti < A.act_t0[pos + 1]; ti += BULK_TILE)
+            for (int j = 0; j < 8; j++) w[j] = part[(size_t)min(ti + j * G, t1 - 1) * NPART + k];
 #pragma unroll
-        for (int k = 0; k < NV; k++) v[k] += part[(size_t)ti * NPART + k];
-    block_sums<BULK_TILE, NV>(v, sh, red);
+            for (int j = 0; j < 8; j++) s += ti + j * G < t1 ? w[j] : 0.0;
+        }
+        sh[g * NV + k] = s;
+    }
+    __syncthreads();
+    if (threadIdx.x < NV) {
+        double s = 0.0;
+#pragma unroll
+        for (int i = 0; i < G; i++) s += sh[i * NV + threadIdx.x];
+        red[threadIdx.x] = s;
+    }
+    __syncthreads();
+}
+
+// The same sums once per block (one workgroup), left in its first tile's place
+template <int NV>
+__global__ __launch_bounds__(1024) void k_bulk_fold(BulkArgs A, const BulkBlock *st, double *part, bool refreshed)
+{
+    __shared__ double sh[NV * (1024 / NV)];
+    __shared__ double red[NV];
+    const BulkBlock &S = st[A.act[blockIdx.x]];
+    if (S.done || (refreshed && !S.refresh)) return;
+    tile_sums<NV, 1024 / NV>(A, blockIdx.x, part, false, sh, red);
+    if (threadIdx.x < NV) part[(size_t)A.act_t0[blockIdx.x] * NPART + threadIdx.x] = red[threadIdx.x];
 }
 
 // alpha from the product's partials (0 for a converged column and where the
 // curvature p.q is not positive), then x += alpha p (FP64), r -= alpha q,
-// z = D^-1 r; partials r.z and r.r
+// z = D^-1 r; partials r.z and r.r.  Two threads per row, three columns each.
 __global__ __launch_bounds__(BULK_TILE) void k_bulk_update(BulkArgs A)
 {
-    __shared__ double sh[NPART * (BULK_TILE / 64)];
+    __shared__ double sh[NPART * SUM_GROUPS];
     __shared__ double red[NRHS];
     const int4 t = A.tiles[blockIdx.x];
     const BulkBlock &S = A.st[t.z];
     if (S.done) return;
-    tile_sums<NRHS>(A, t.w, A.part, sh, red);
-    double v[NPART];
-#pragma unroll
-    for (int k = 0; k < NPART; k++) v[k] = 0.0;
-    const int i = t.x + threadIdx.x;
+    tile_sums<NRHS>(A, t.w, A.part, A.fold, sh, red);
+    double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    const int i = t.x + threadIdx.x / 2, h = 3 * (threadIdx.x % 2);
     if (i < t.y) {
         const float d = A.dinv[i];
+        const size_t o = (size_t)i * NRHS + h;
 #pragma unroll
-        for (int k = 0; k < NRHS; k++) {
-            const size_t o = (size_t)i * NRHS + k;
-            const float al = (!(S.conv >> k & 1) && red[k] > 0.0) ? (float)(S.rho[k] / red[k]) : 0.f;
-            A.x[o] += (double)al * (double)A.p[o];
-            const float ri = fmaf(-al, A.q[o], A.r[o]);
-            A.r[o] = ri;
+        for (int k = 0; k < 3; k++) {
+            const float al = (!(S.conv >> (h + k) & 1) && red[h + k] > 0.0) ? (float)(S.rho[h + k] / red[h + k]) : 0.f;
+            A.x[o + k] += (double)al * (double)A.p[o + k];
+            const float ri = fmaf(-al, A.q[o + k], A.r[o + k]);
+            A.r[o + k] = ri;
             const float zi = d * ri;
-            A.z[o] = zi;
+            A.z[o + k] = zi;
             v[k] = (double)ri * (double)zi;
-            v[NRHS + k] = (double)ri * (double)ri;
+            v[3 + k] = (double)ri * (double)ri;
         }
     }
-    block_sums<BULK_TILE, NPART>(v, sh, A.part_rz + (size_t)blockIdx.x * NPART);
+    const int w = threadIdx.x / 64, l = threadIdx.x % 64;
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+#pragma unroll
+        for (int off = 32; off > 1; off >>= 1) v[k] += __shfl_xor(v[k], off, 64);
+        if (l < 2) sh[w * NPART + (k / 3) * NRHS + 3 * l + k % 3] = v[k];
+    }
+    __syncthreads();
+    if (threadIdx.x < NPART) {
+        double s = 0.0;
+#pragma unroll
+        for (int j = 0; j < BULK_TILE / 64; j++) s += sh[j * NPART + threadIdx.x];
+        A.part_rz[(size_t)blockIdx.x * NPART + threadIdx.x] = s;
+    }
 }
 
 __device__ void bulk_finish(const BulkArgs &A, BulkBlock &S, bool all)
@@ -453,13 +507,11 @@ __device__ void bulk_finish(const BulkArgs &A, BulkBlock &S, bool all)
 // p = z + beta p of the tile's rows
 __device__ __forceinline__ void tile_direction(const BulkArgs &A, const int4 &t, const float beta[NRHS])
 {
-    const int i = t.x + threadIdx.x;
+    const int i = t.x + threadIdx.x / 2, h = threadIdx.x % 2;
     if (i >= t.y) return;
+    const size_t o = (size_t)i * NRHS + 3 * h;
 #pragma unroll
-    for (int k = 0; k < NRHS; k++) {
-        const size_t o = (size_t)i * NRHS + k;
-        A.p[o] = fmaf(beta[k], A.p[o], A.z[o]);
-    }
+    for (int k = 0; k < 3; k++) A.p[o + k] = fmaf(h ? beta[3 + k] : beta[k], A.p[o + k], A.z[o + k]);
 }
 
 // After the update: does the block ask for a reliable update (a residual met
@@ -474,7 +526,7 @@ __device__ __forceinline__ bool bulk_step(const BulkArgs &A, const int4 &t, doub
         if (writer) A.st1[t.z] = S;
         return false;
     }
-    tile_sums<NPART>(A, t.w, A.part_rz, sh, red);
+    tile_sums<NPART>(A, t.w, A.part_rz, A.fold, sh, red);
     bool refresh = false;
     double res[NRHS];
     float beta[NRHS];
@@ -505,7 +557,7 @@ __device__ __forceinline__ bool bulk_step(const BulkArgs &A, const int4 &t, doub
 // every block its first tile brings the state back to st
 __global__ __launch_bounds__(BULK_TILE) void k_bulk_finish(BulkArgs A)
 {
-    __shared__ double sh[NPART * (BULK_TILE / 64)];
+    __shared__ double sh[NPART * SUM_GROUPS];
     __shared__ double red[NPART];
     const int4 t = A.tiles[blockIdx.x];
     const BulkBlock &S = A.st1[t.z];
@@ -514,7 +566,7 @@ __global__ __launch_bounds__(BULK_TILE) void k_bulk_finish(BulkArgs A)
         if (writer) A.st[t.z] = S;
         return;
     }
-    tile_sums<NPART>(A, t.w, A.part_tr, sh, red);
+    tile_sums<NPART>(A, t.w, A.part_tr, A.fold, sh, red);
     bool all = true;
     int conv = 0;
     double res[NRHS];
@@ -548,7 +600,7 @@ __global__ __launch_bounds__(BULK_TILE) void k_bulk_finish(BulkArgs A)
 template <int LPR>
 __global__ __launch_bounds__(BULK_TILE) void k_bulk_refresh(BulkArgs A)
 {
-    __shared__ double sh[NPART * (BULK_TILE / 64)];
+    __shared__ double sh[NPART * SUM_GROUPS];
     __shared__ double red[NPART];
     const int4 t = A.tiles[blockIdx.x];
     if (!bulk_step(A, t, sh, red)) return;
@@ -784,7 +836,7 @@ __global__ void k_bulk_widen(int nbr, const int32_t *__restrict__ bptr, const fl
 template <int LPR>
 __global__ __launch_bounds__(BULK_TILE) void k_bulk_refresh_nb(BulkArgs A)
 {
-    __shared__ double sh[NPART * (BULK_TILE / 64)];
+    __shared__ double sh[NPART * SUM_GROUPS];
     __shared__ double red[NPART];
     const int4 t = A.tiles[blockIdx.x];
     if (!bulk_step(A, t, sh, red)) return;
@@ -817,10 +869,10 @@ __global__ __launch_bounds__(BULK_TILE) void k_bulk_refresh_nb(BulkArgs A)
 // one workgroup per block: the initial scalars from the init partials
 __global__ __launch_bounds__(BULK_TILE) void k_bulk_start(BulkArgs A)
 {
-    __shared__ double sh[NPART * (BULK_TILE / 64)];
+    __shared__ double sh[NPART * SUM_GROUPS];
     __shared__ double red[NPART];
     BulkBlock &S = A.st[A.act[blockIdx.x]];
-    tile_sums<NPART>(A, blockIdx.x, A.part_rz, sh, red);
+    tile_sums<NPART>(A, blockIdx.x, A.part_rz, false, sh, red);
     if (threadIdx.x != 0) return;
     bool all = true;
     S.conv = 0;
@@ -1267,8 +1319,13 @@ static int bulk_solve(hfem_batch *bt, const double *db, double *dx, int maxit)
     A.vwide = reinterpret_cast<const float4 *>(bt->d_vwide);
     const bulk_kernel_t spmv = wide ? sh.spmv_nbw : nb ? sh.spmv_nb : sh.spmv;
     const bulk_kernel_t refresh = nb ? sh.refresh_nb : sh.refresh;
-    int ntiles = (int)bt->h_tiles.size();
-    const int nact = nbulk;
+    auto most_tiles = [&] {
+        int m = 0;
+        for (size_t pos = 0; pos + 1 < bt->h_act_t0.size(); pos++) m = std::max(m, bt->h_act_t0[pos + 1] - bt->h_act_t0[pos]);
+        return m;
+    };
+    int ntiles = (int)bt->h_tiles.size(), nact = nbulk;
+    A.fold = most_tiles() > FOLD_TILES;
     k_bulk_init<<<ntiles, BULK_TILE, 0, st>>>(A);
     k_bulk_start<<<nact, BULK_TILE, 0, st>>>(A);
     HIPFEM_CHECK(hipGetLastError());
@@ -1298,14 +1355,19 @@ static int bulk_solve(hfem_batch *bt, const double *db, double *dx, int maxit)
                 rc = bulk_tiles(bt, act);
                 if (rc) return rc;
                 ntiles = (int)bt->h_tiles.size();
+                nact = (int)act.size();
+                A.fold = most_tiles() > FOLD_TILES;
             }
         }
         const bool timed = bt->profiling && bt->ev_used < BULK_CHECK;
         if (timed) HIPFEM_CHECK(hipEventRecord(bt->ev[2 * bt->ev_used], st));
         hipLaunchKernelGGL(spmv, dim3(ntiles), dim3(BULK_TILE), 0, st, A);
         if (timed) HIPFEM_CHECK(hipEventRecord(bt->ev[2 * bt->ev_used++ + 1], st));
+        if (A.fold) k_bulk_fold<NRHS><<<nact, 1024, 0, st>>>(A, A.st, A.part, false);
         k_bulk_update<<<ntiles, BULK_TILE, 0, st>>>(A);
+        if (A.fold) k_bulk_fold<NPART><<<nact, 1024, 0, st>>>(A, A.st, A.part_rz, false);
         hipLaunchKernelGGL(refresh, dim3(ntiles), dim3(BULK_TILE), 0, st, A);
+        if (A.fold) k_bulk_fold<NPART><<<nact, 1024, 0, st>>>(A, A.st1, A.part_tr, true);
         k_bulk_finish<<<ntiles, BULK_TILE, 0, st>>>(A);
         HIPFEM_CHECK(hipGetLastError());
     }

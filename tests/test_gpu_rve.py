@@ -54,6 +54,33 @@ def test_batch_homogenized_stiffness_matches_oracle(ctx, mode):
     B.close()
 
 
+@pytest.mark.parametrize("form", [0, 1, 2])
+@pytest.mark.parametrize("sizes", [(2, 3, 4, 5, 6), (34, 5, 2)], ids=["tiles", "fold"])
+def test_bulk_sums_at_tile_edges(ctx, sizes, form):
+    """The bulk phase with blocks of 1 (partial), exactly 2 and a few tiles of
+    96 rows, and with a block of more tiles than the workgroups sum
+    themselves: the true residual of every column, recomputed here, meets the
+    tolerance and is the reported one (an FP64 residual's rounding is below
+    1 % of a tolerance of 1e-10)."""
+    import scipy.sparse as sp
+
+    from oofem_amd.rve import RVEBatch
+    B = RVEBatch(ctx, [(n, meshgen.LSPACE, 0.3, n) for n in sizes])
+    (c,) = B.chunks
+    B.set_options(tol=1e-10, split=0, bulk_form=form)
+    out = B.run()
+    rp, ci, val = c.K.download()
+    A = sp.csr_matrix((val, ci, rp), shape=(c.n, c.n))
+    b, x = c.b.download().reshape(c.n, 6), c.x.download().reshape(c.n, 6)
+    r = b - A @ x
+    for i in range(len(sizes)):
+        q = slice(c.rows[i], c.rows[i + 1])
+        res = (np.linalg.norm(r[q], axis=0) / np.linalg.norm(b[q], axis=0)).max()
+        assert 0 < out["resid"][i] <= 1e-10
+        assert abs(res - out["resid"][i]) <= 1e-12, (sizes[i], res, out["resid"][i])
+    B.close()
+
+
 def test_batch_autotune_picks_a_valid_shape(ctx):
     from oofem_amd.rve import RVEBatch
     B = RVEBatch(ctx, SPECS[:4])
