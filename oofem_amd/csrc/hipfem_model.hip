@@ -384,6 +384,12 @@ __global__ __launch_bounds__(64) void k_assemble(const int *__restrict__ elems, 
 }
 
 // ------------------------------------------------------ MisesMat surrogate
+// The acceptance counts are kept on SUR_LINES cache lines: atomics on one
+// address are served one after the other, about 12 ns each, and the blocks'
+// two atomics set the time of the whole kernel (1,048,576 hexahedron points:
+// 404 us with one pair, 71 with 64).
+constexpr int SUR_LINES = 64, SUR_LINE = 16;
+
 // Per-GP surrogate data of one internal-force evaluation.
 struct SurArgs {
     const int *slot = nullptr;   // queue slot of the GP's prediction, -1 none (nullptr: surrogate off)
@@ -391,8 +397,8 @@ struct SurArgs {
     float *dsur = nullptr;       // accepted tangent per GP, 21 x ngp_total (SoA, upper triangle)
     int8_t *flag = nullptr;      // 1: the GP's temp state and tangent come from the surrogate
     int8_t *rejected = nullptr;  // 1: rejected once in this load step (stays on the plain update)
-    unsigned long long *counts = nullptr;   // [0] accepted, [1] rejected by the residual check
-    float sig_scale = 1.f, tan_scale = 1.f;
+    unsigned long long *counts = nullptr;   // SUR_LINES x SUR_LINE: [0] accepted, [1] rejected by the residual check
+    double sig_inv = 1.0, tan_inv = 1.0;    // 1 / the scales of the predictions
     double tol = 0.0;
 };
 
@@ -405,9 +411,9 @@ struct SurArgs {
 // (misesmat.C:496-544; an indefinite prediction would break the linear
 // solver).  The temp state is then the one consistent with that stress:
 // kappa_n + Delta kappa and epsp = eps - C^-1 sigma.
-__device__ bool surrogate_update(double E, double nu, double sig0, double H, const double eps[6],
-                                 const double epsp_n[6], double kappa_n, const float *y, float sig_scale,
-                                 float tan_scale, double tol, MisesOut &o)
+__device__ __forceinline__ bool surrogate_update(double E, double nu, double sig0, double H, const double eps[6],
+                                 const double epsp_n[6], double kappa_n, const float *y, double sig_inv,
+                                 double tan_inv, double tol, MisesOut &o)
 {
     const double G = E / (2.0 * (1. + nu));
     const double K = E / (3.0 * (1. - 2. * nu));
@@ -422,9 +428,9 @@ __device__ bool surrogate_update(double E, double nu, double sig0, double H, con
     // network outputs are departures from the elastic trial
     double sp[6];
 #pragma unroll
-    for (int i = 0; i < 3; i++) sp[i] = st[i] + 3. * K * mean - (double)y[i] / (double)sig_scale;
+    for (int i = 0; i < 3; i++) sp[i] = st[i] + 3. * K * mean - (double)y[i] * sig_inv;
 #pragma unroll
-    for (int i = 3; i < 6; i++) sp[i] = st[i] - (double)y[i] / (double)sig_scale;
+    for (int i = 3; i < 6; i++) sp[i] = st[i] - (double)y[i] * sig_inv;
     const double pp = (sp[0] + sp[1] + sp[2]) / 3.0;
     const double dv[6] = {sp[0] - pp, sp[1] - pp, sp[2] - pp, sp[3], sp[4], sp[5]};
     const double nrm = sqrt(dv[0] * dv[0] + dv[1] * dv[1] + dv[2] * dv[2] +
@@ -446,13 +452,19 @@ __device__ bool surrogate_update(double E, double nu, double sig0, double H, con
     if (!(fmax(r1, fmax(r2, r3)) <= tol * sy)) return false;
     // the predicted tangent must match MisesMat's consistent tangent at the
     // accepted state (kappa_n + Delta kappa, trial deviator) within tol * E
-    double D[36];
-    mises_tangent(E, nu, sig0, H, kappa_n, kappa_n + dk, st, D);
+    double c, m[6];
+    mises_tangent_parts(E, nu, sig0, H, kappa_n, kappa_n + dk, st, c, m);
+    bool near = true;
     int k = 0;
-    for (int r = 0; r < 6; r++)
-        for (int c = r; c < 6; c++, k++)
-            if (!(fabs(elastic_upper(E, nu, k) - (double)y[6 + k] / (double)tan_scale - D[6 * r + c]) <= tol * E))
-                return false;
+#pragma unroll
+    for (int i = 0; i < 6; i++)
+#pragma unroll
+        for (int j = i; j < 6; j++, k++) {
+            const double dev = i != j ? (j < 3 ? -1. / 3. : 0.0) : i < 3 ? 2. / 3. : 0.5;
+            const double D = c * dev + (j < 3 ? K : 0.0) - m[i] * m[j];
+            near = near && fabs(elastic_upper(E, nu, k) - (double)y[6 + k] * tan_inv - D) <= tol * E;
+        }
+    if (!near) return false;
 #pragma unroll
     for (int i = 0; i < 6; i++) {
         o.sig[i] = sp[i];
@@ -465,86 +477,6 @@ __device__ bool surrogate_update(double E, double nu, double sig0, double H, con
     for (int i = 3; i < 6; i++) o.epsp[i] = eps[i] - dv[i] / G;
     o.kappa = kappa_n + dk;
     return true;
-}
-
-// Queue the MisesMat Gauss points whose trial state lies more than band *
-// sigma_y(kappa_n) outside the yield surface (the others stay with the
-// plain update: elastic, or within the band around the surface) and write
-// their scaled network inputs.  One thread per Gauss point, all elements.
-template <int ET>
-__global__ __launch_bounds__(256) void k_sur_classify(int nelem, const double *__restrict__ coords,
-                                                      const int *__restrict__ conn, const int *__restrict__ eqn,
-                                                      const int *__restrict__ emat, const double *__restrict__ mat,
-                                                      const double *__restrict__ u_free,
-                                                      const double *__restrict__ u_presc,
-                                                      const double *__restrict__ state, int ngp_total, double band,
-                                                      float in_scale, const int8_t *__restrict__ rejected,
-                                                      int *__restrict__ slot, int *__restrict__ count,
-                                                      float *__restrict__ X)
-{
-    constexpr int NEN = ElemT<ET>::NEN, NGP = ElemT<ET>::NGP, NC = 3 * NEN;
-    const int gp = blockIdx.x * blockDim.x + threadIdx.x;
-    if (gp >= ngp_total) return;
-    const int e = gp / NGP, g = gp % NGP;
-    const double *mp = mat + (size_t)HIPFEM_MATP * emat[e];
-    if ((int)mp[0] != HIPFEM_MAT_MISES || rejected[gp]) {
-        slot[gp] = -1;
-        return;
-    }
-    double X3[NC], ue[NC];
-    for (int a = 0; a < NEN; a++) {
-        const int node = conn[(size_t)e * NEN + a];
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            X3[3 * a + d] = coords[3 * (size_t)node + d];
-            const int q = eqn[3 * (size_t)node + d];
-            ue[3 * a + d] = (q > 0 && u_free) ? u_free[q - 1] : ((q < 0 && u_presc) ? u_presc[-q - 1] : 0.0);
-        }
-    }
-    double xi[3], w, detJ, dNdx[NC];
-    gauss_point(ET, g, xi, w);
-    if (!gp_geometry<ET>(X3, xi, dNdx, detJ)) {
-        slot[gp] = -1;
-        return;
-    }
-    double eps[6] = {0, 0, 0, 0, 0, 0};
-    for (int a = 0; a < NEN; a++) {
-        const double nx = dNdx[3 * a], ny = dNdx[3 * a + 1], nz = dNdx[3 * a + 2];
-        const double ux = ue[3 * a], uy = ue[3 * a + 1], uz = ue[3 * a + 2];
-        eps[0] += nx * ux;
-        eps[1] += ny * uy;
-        eps[2] += nz * uz;
-        eps[3] += nz * uy + ny * uz;
-        eps[4] += nz * ux + nx * uz;
-        eps[5] += ny * ux + nx * uy;
-    }
-    const double E = mp[1], nu = mp[2], sig0 = mp[3], H = mp[4];
-    const double G = E / (2.0 * (1. + nu));
-    double el[6], epsp_n[6];
-#pragma unroll
-    for (int i = 0; i < 6; i++) {
-        epsp_n[i] = state[(size_t)i * ngp_total + gp];
-        el[i] = eps[i] - epsp_n[i];
-    }
-    const double kappa_n = state[(size_t)6 * ngp_total + gp];
-    const double mean = (el[0] + el[1] + el[2]) / 3.0;
-    const double s0 = 2. * G * (el[0] - mean), s1 = 2. * G * (el[1] - mean), s2 = 2. * G * (el[2] - mean);
-    const double s3 = G * el[3], s4 = G * el[4], s5 = G * el[5];
-    const double trialS = sqrt(s0 * s0 + s1 * s1 + s2 * s2 + 2. * (s3 * s3 + s4 * s4 + s5 * s5));
-    const double sy = sig0 + H * kappa_n;
-    if (sqrt(1.5) * trialS - sy > band * sy) {
-        const int k = atomicAdd(count, 1);
-        slot[gp] = k;
-        float *x = X + (size_t)k * 13;
-#pragma unroll
-        for (int i = 0; i < 6; i++) {
-            x[i] = (float)(el[i] * in_scale);
-            x[6 + i] = (float)(epsp_n[i] * in_scale);
-        }
-        x[12] = (float)(kappa_n * in_scale);
-    } else {
-        slot[gp] = -1;
-    }
 }
 
 // -------------------------------------------------------- internal forces
@@ -617,7 +549,7 @@ __device__ __forceinline__ void point_stress(const IntArgs &A, const double *mp,
             const int sl = sur.slot[gp];
             if (sl >= 0) {
                 used = surrogate_update(E, nu, mp[3], mp[4], eps, epsp_n, kappa_n, sur.y + (size_t)27 * sl,
-                                        sur.sig_scale, sur.tan_scale, sur.tol, o);
+                                        sur.sig_inv, sur.tan_inv, sur.tol, o);
                 atomicAdd(&scount[used ? 0 : 1], 1u);
             }
             if (A.update_state) {
@@ -630,7 +562,7 @@ __device__ __forceinline__ void point_stress(const IntArgs &A, const double *mp,
 #pragma unroll
                     for (int k = 0; k < 21; k++)
                         sur.dsur[(size_t)k * ngp_total + gp] =
-                            (float)(elastic_upper(E, nu, k) - (double)yy[k] / (double)sur.tan_scale);
+                            (float)(elastic_upper(E, nu, k) - (double)yy[k] * sur.tan_inv);
                 }
             }
         }
@@ -699,8 +631,9 @@ __device__ __forceinline__ void add_sur_counts(const IntArgs &A, int t, const un
 {
     if constexpr (SUR)
         if (A.sur.counts && t == 0 && (scount[0] | scount[1])) {
-            atomicAdd(&A.sur.counts[0], (unsigned long long)scount[0]);
-            atomicAdd(&A.sur.counts[1], (unsigned long long)scount[1]);
+            unsigned long long *c = A.sur.counts + SUR_LINE * (blockIdx.x % SUR_LINES);
+            if (scount[0]) atomicAdd(&c[0], (unsigned long long)scount[0]);
+            if (scount[1]) atomicAdd(&c[1], (unsigned long long)scount[1]);
         }
 }
 
@@ -758,6 +691,199 @@ __global__ __launch_bounds__(64) void k_internal_tet(IntArgs A)
     store_element_forces<EPB, NGP, NC>(A, t, sF, sh);
 }
 
+// The linear hexahedron's Gauss point g with its element's node values in LDS,
+// value v of node a at sN[(v * 8 + a) * 8 + el]: coordinates, then
+// displacements.  I = J^-1, H_ij = du_i/dx_j.
+struct HexPoint {
+    double yz[4], xz[4], xy[4], I[9], H[9], det;
+    __device__ __forceinline__ void dndxi(int a, double dN[3]) const   // dndxi_hexlin at the lane's point
+    {
+        const int bx = (a & 3) >= 2, by = (a & 3) == 1 || (a & 3) == 2, bz = a < 4;
+        dN[0] = bx ? yz[2 * by + bz] : -yz[2 * by + bz];
+        dN[1] = by ? xz[2 * bx + bz] : -xz[2 * bx + bz];
+        dN[2] = bz ? xy[2 * bx + by] : -xy[2 * bx + by];
+    }
+    __device__ __forceinline__ HexPoint(const double *sN, int el, int g)
+    {
+        const double ga = 0.577350269189626;   // gauss_point
+        const double xi = (g & 4) ? ga : -ga, eta = (g & 2) ? ga : -ga, ze = (g & 1) ? ga : -ga;
+        const double xm = 1. - xi, xp = 1. + xi, ym = 1. - eta, yp = 1. + eta, zm = 1. - ze, zp = 1. + ze;
+        yz[0] = 0.125 * ym * zm, yz[1] = 0.125 * ym * zp, yz[2] = 0.125 * yp * zm, yz[3] = 0.125 * yp * zp;
+        xz[0] = 0.125 * xm * zm, xz[1] = 0.125 * xm * zp, xz[2] = 0.125 * xp * zm, xz[3] = 0.125 * xp * zp;
+        xy[0] = 0.125 * xm * ym, xy[1] = 0.125 * xm * yp, xy[2] = 0.125 * xp * ym, xy[3] = 0.125 * xp * yp;
+        double J[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, gu[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int a = 0; a < 8; a++) {
+            double dN[3];
+            dndxi(a, dN);
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                const double x = sN[(i * 8 + a) * 8 + el], u = sN[((3 + i) * 8 + a) * 8 + el];
+#pragma unroll
+                for (int j = 0; j < 3; j++) {
+                    J[3 * i + j] += x * dN[j];
+                    gu[3 * i + j] += u * dN[j];
+                }
+            }
+        }
+        // the cofactors times one reciprocal
+        I[0] = J[4] * J[8] - J[5] * J[7];
+        I[1] = J[2] * J[7] - J[1] * J[8];
+        I[2] = J[1] * J[5] - J[2] * J[4];
+        I[3] = J[5] * J[6] - J[3] * J[8];
+        I[4] = J[0] * J[8] - J[2] * J[6];
+        I[5] = J[2] * J[3] - J[0] * J[5];
+        I[6] = J[3] * J[7] - J[4] * J[6];
+        I[7] = J[1] * J[6] - J[0] * J[7];
+        I[8] = J[0] * J[4] - J[1] * J[3];
+        det = J[0] * I[0] + J[1] * I[3] + J[2] * I[6];
+        const double id = 1. / det;
+#pragma unroll
+        for (int i = 0; i < 9; i++) I[i] *= id;
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int j = 0; j < 3; j++)
+                H[3 * i + j] = gu[3 * i] * I[j] + gu[3 * i + 1] * I[3 + j] + gu[3 * i + 2] * I[6 + j];
+    }
+};
+
+// the node values of a wave's eight elements, lane (el, node); spare lanes
+// load the last element
+template <typename ARGS>
+__device__ __forceinline__ void hex_nodes(const ARGS &A, int e, int el, int a, double *sN)
+{
+    const int node = A.conn[(size_t)e * 8 + a];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        sN[(d * 8 + a) * 8 + el] = A.coords[3 * (size_t)node + d];
+        sN[((3 + d) * 8 + a) * 8 + el] = dof_value(A.eqn[3 * (size_t)node + d], A.u_free, A.u_presc);
+    }
+}
+
+// Queue the MisesMat Gauss points whose trial state lies more than band *
+// sigma_y(kappa_n) outside the yield surface (the others stay with the
+// plain update: elastic, or within the band around the surface) and write
+// their scaled network inputs.  All elements in one launch.
+struct ClassifyArgs {
+    int nelem;
+    const double *coords;
+    const int *conn, *eqn, *emat;
+    const double *mat, *u_free, *u_presc, *state;
+    int ngp_total;
+    double band;
+    float in_scale;
+    const int8_t *rejected;
+    int *slot, *count;
+    float *X;
+};
+
+// One point per thread (every thread of the block is here); ok: a MisesMat
+// point with a valid strain.  One atomic per block takes the places of its
+// points: they all go to one address, one after the other.
+template <int BS>
+__device__ __forceinline__ void classify_point(const ClassifyArgs &A, const double *mp, int gp, bool in, bool ok,
+                                               const double eps[6])
+{
+    double el[6], epsp_n[6], kappa_n = 0.0;
+    if (ok) {
+        const double E = mp[1], nu = mp[2], sig0 = mp[3], H = mp[4];
+        const double G = E / (2.0 * (1. + nu));
+#pragma unroll
+        for (int i = 0; i < 6; i++) {
+            epsp_n[i] = A.state[(size_t)i * A.ngp_total + gp];
+            el[i] = eps[i] - epsp_n[i];
+        }
+        kappa_n = A.state[(size_t)6 * A.ngp_total + gp];
+        const double mean = (el[0] + el[1] + el[2]) / 3.0;
+        const double s0 = 2. * G * (el[0] - mean), s1 = 2. * G * (el[1] - mean), s2 = 2. * G * (el[2] - mean);
+        const double s3 = G * el[3], s4 = G * el[4], s5 = G * el[5];
+        const double trialS = sqrt(s0 * s0 + s1 * s1 + s2 * s2 + 2. * (s3 * s3 + s4 * s4 + s5 * s5));
+        const double sy = sig0 + H * kappa_n;
+        ok = sqrt(1.5) * trialS - sy > A.band * sy;
+    }
+    __shared__ int place[BS / 64 + 1];
+    const unsigned long long m = __ballot(ok);
+    const int w = threadIdx.x / 64, lane = threadIdx.x % 64;
+    if (lane == 0) place[w] = __popcll(m);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int n = 0;
+        for (int i = 0; i < BS / 64; i++) n += place[i];
+        place[BS / 64] = n ? atomicAdd(A.count, n) : 0;
+    }
+    __syncthreads();
+    int k = place[BS / 64] + __popcll(m & ((1ull << lane) - 1));
+    for (int i = 0; i < w; i++) k += place[i];
+    if (in) A.slot[gp] = ok ? k : -1;
+    if (!ok) return;
+    float *x = A.X + (size_t)k * 13;
+#pragma unroll
+    for (int i = 0; i < 6; i++) {
+        x[i] = (float)(el[i] * A.in_scale);
+        x[6 + i] = (float)(epsp_n[i] * A.in_scale);
+    }
+    x[12] = (float)(kappa_n * A.in_scale);
+}
+
+template <int ET>
+__global__ __launch_bounds__(256) void k_sur_classify(ClassifyArgs A)
+{
+    constexpr int NEN = ElemT<ET>::NEN, NGP = ElemT<ET>::NGP, NC = 3 * NEN;
+    const int gp = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool in = gp < A.ngp_total;
+    const int e = in ? gp / NGP : 0, g = in ? gp % NGP : 0;
+    const double *mp = A.mat + (size_t)HIPFEM_MATP * A.emat[e];
+    bool ok = in && (int)mp[0] == HIPFEM_MAT_MISES && !A.rejected[gp];
+    double eps[6] = {0, 0, 0, 0, 0, 0};
+    if (ok) {
+        double X3[NC], ue[NC];
+        for (int a = 0; a < NEN; a++) {
+            const int node = A.conn[(size_t)e * NEN + a];
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                X3[3 * a + d] = A.coords[3 * (size_t)node + d];
+                ue[3 * a + d] = dof_value(A.eqn[3 * (size_t)node + d], A.u_free, A.u_presc);
+            }
+        }
+        double xi[3], w, detJ, dNdx[NC];
+        gauss_point(ET, g, xi, w);
+        ok = gp_geometry<ET>(X3, xi, dNdx, detJ);
+        if (ok)
+            for (int a = 0; a < NEN; a++) {
+                const double nx = dNdx[3 * a], ny = dNdx[3 * a + 1], nz = dNdx[3 * a + 2];
+                const double ux = ue[3 * a], uy = ue[3 * a + 1], uz = ue[3 * a + 2];
+                eps[0] += nx * ux;
+                eps[1] += ny * uy;
+                eps[2] += nz * uz;
+                eps[3] += nz * uy + ny * uz;
+                eps[4] += nz * ux + nx * uz;
+                eps[5] += ny * ux + nx * uy;
+            }
+    }
+    classify_point<256>(A, mp, gp, in, ok, eps);
+}
+
+// k_sur_classify for linear hexahedra: lane (el, g) loads node g of its
+// element once into LDS for the element's eight points.  With one atomic a
+// wave on the queue's count the atomics set the time (205 us for 1,048,576
+// points, whatever the loads); one a block of 1024: 48 us.
+__global__ __launch_bounds__(1024) void k_sur_classify_hex(ClassifyArgs A)
+{
+    __shared__ double sN[16 * 48 * 8];
+    const int gp = blockIdx.x * 1024 + threadIdx.x, el = (threadIdx.x % 64) >> 3, g = threadIdx.x & 7;
+    const bool in = gp < A.ngp_total;
+    const int e = in ? gp >> 3 : A.nelem - 1;
+    double *sW = sN + (threadIdx.x / 64) * (48 * 8);
+    hex_nodes(A, e, el, g, sW);
+    wave_lds_fence();
+    const HexPoint P(sW, el, g);
+    const double eps[6] = {P.H[0], P.H[4], P.H[8], P.H[5] + P.H[7], P.H[2] + P.H[6], P.H[1] + P.H[3]};
+    const double *mp = A.mat + (size_t)HIPFEM_MATP * A.emat[e];
+    const bool ok = in && (int)mp[0] == HIPFEM_MAT_MISES && fabs(P.det) > 1.e-30 && !A.rejected[gp];
+    classify_point<1024>(A, mp, gp, in, ok, eps);
+}
+
 // LSpace: 8 elements a wave, lane (el, g) is Gauss point g of element el and
 // loads node g's coordinates and displacements, which the element's lanes
 // share through LDS (10 loads a lane instead of 80).  Strain and force go
@@ -767,9 +893,10 @@ __global__ __launch_bounds__(64) void k_internal_tet(IntArgs A)
 // Bound: the 7 state values read and 25 written a point, 2.15 GB on the
 // 64x64x256 block: 0.62 ms (3.8 TB/s with the element forces).  With every
 // lane loading its element's eight nodes and holding the 24 dN/dx, 198 VGPRs
-// left two waves a SIMD: 1.04 ms.
+// left two waves a SIMD: 1.04 ms.  The surrogate's form is held to three waves
+// (36 bytes spilled): 62 against 71 us for 1,048,576 points.
 template <int OP, bool SUR>
-__global__ __launch_bounds__(64) void k_internal_hex(IntArgs A)
+__global__ __launch_bounds__(64, SUR ? 3 : 1) void k_internal_hex(IntArgs A)
 {
     __shared__ double sF[64 * 25];      // first: the nodes' coordinates and displacements
     __shared__ double sh[3];
@@ -782,62 +909,12 @@ __global__ __launch_bounds__(64) void k_internal_hex(IntArgs A)
     const int ei = blockIdx.x * 8 + el;
     const bool active = ei < A.nelem;
     const int e = active ? ei : A.nelem - 1;   // spare lanes of the last block load the last element
-    {
-        const int node = A.conn[(size_t)e * 8 + g];
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            sF[(d * 8 + g) * 8 + el] = A.coords[3 * (size_t)node + d];
-            sF[((3 + d) * 8 + g) * 8 + el] = dof_value(A.eqn[3 * (size_t)node + d], A.u_free, A.u_presc);
-        }
-    }
+    hex_nodes(A, e, el, g, sF);
     wave_lds_fence();
-    const double ga = 0.577350269189626;   // gauss_point
-    const double xi = (g & 4) ? ga : -ga, eta = (g & 2) ? ga : -ga, ze = (g & 1) ? ga : -ga;
-    const double xm = 1. - xi, xp = 1. + xi, ym = 1. - eta, yp = 1. + eta, zm = 1. - ze, zp = 1. + ze;
-    const double yz[4] = {0.125 * ym * zm, 0.125 * ym * zp, 0.125 * yp * zm, 0.125 * yp * zp};
-    const double xz[4] = {0.125 * xm * zm, 0.125 * xm * zp, 0.125 * xp * zm, 0.125 * xp * zp};
-    const double xy[4] = {0.125 * xm * ym, 0.125 * xm * yp, 0.125 * xp * ym, 0.125 * xp * yp};
-    auto dndxi = [&](int a, double dN[3]) {   // dndxi_hexlin at the lane's point
-        const int bx = (a & 3) >= 2, by = (a & 3) == 1 || (a & 3) == 2, bz = a < 4;
-        dN[0] = bx ? yz[2 * by + bz] : -yz[2 * by + bz];
-        dN[1] = by ? xz[2 * bx + bz] : -xz[2 * bx + bz];
-        dN[2] = bz ? xy[2 * bx + by] : -xy[2 * bx + by];
-    };
-    double J[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, gu[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-    for (int a = 0; a < 8; a++) {
-        double dN[3];
-        dndxi(a, dN);
-#pragma unroll
-        for (int i = 0; i < 3; i++) {
-            const double x = sF[(i * 8 + a) * 8 + el], u = sF[((3 + i) * 8 + a) * 8 + el];
-#pragma unroll
-            for (int j = 0; j < 3; j++) {
-                J[3 * i + j] += x * dN[j];
-                gu[3 * i + j] += u * dN[j];
-            }
-        }
-    }
-    double I[9];   // J^-1: the cofactors times one reciprocal
-    I[0] = J[4] * J[8] - J[5] * J[7];
-    I[1] = J[2] * J[7] - J[1] * J[8];
-    I[2] = J[1] * J[5] - J[2] * J[4];
-    I[3] = J[5] * J[6] - J[3] * J[8];
-    I[4] = J[0] * J[8] - J[2] * J[6];
-    I[5] = J[2] * J[3] - J[0] * J[5];
-    I[6] = J[3] * J[7] - J[4] * J[6];
-    I[7] = J[1] * J[6] - J[0] * J[7];
-    I[8] = J[0] * J[4] - J[1] * J[3];
-    const double det = J[0] * I[0] + J[1] * I[3] + J[2] * I[6];
-    if (active && !(fabs(det) > 1.e-30)) atomicMin(A.bad, e);
-    const double id = 1. / det, dV = fabs(det);   // the rule's weights are 1
-#pragma unroll
-    for (int i = 0; i < 9; i++) I[i] *= id;
-    double H[9];   // du_i/dx_j
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-        for (int j = 0; j < 3; j++) H[3 * i + j] = gu[3 * i] * I[j] + gu[3 * i + 1] * I[3 + j] + gu[3 * i + 2] * I[6 + j];
+    const HexPoint P(sF, el, g);
+    if (active && !(fabs(P.det) > 1.e-30)) atomicMin(A.bad, e);
+    const double dV = fabs(P.det);   // the rule's weights are 1
+    const double *I = P.I, *H = P.H;
     const double eps[6] = {H[0], H[4], H[8], H[5] + H[7], H[2] + H[6], H[1] + H[3]};
     double sig[6] = {0, 0, 0, 0, 0, 0};
     if (active) point_stress<OP, SUR>(A, A.mat + (size_t)HIPFEM_MATP * A.emat[e], (size_t)e * 8 + g, eps, scount, sig);
@@ -852,7 +929,7 @@ __global__ __launch_bounds__(64) void k_internal_hex(IntArgs A)
 #pragma unroll
     for (int a = 0; a < 8; a++) {
         double dN[3];
-        dndxi(a, dN);
+        P.dndxi(a, dN);
 #pragma unroll
         for (int i = 0; i < 3; i++)
             sF[t * 25 + 3 * a + i] = T[3 * i] * dN[0] + T[3 * i + 1] * dN[1] + T[3 * i + 2] * dN[2];
@@ -2269,14 +2346,12 @@ static int internal_dev(hfem_model *md, const double *uf, const double *up, doub
         // queue the points beyond the band, infer them in one BF16 batch
         HIPFEM_CHECK(hipMemsetAsync(md->d_qcount, 0, sizeof(int), st));
         const int g2 = (md->ngp_total + 255) / 256;
-#define LAUNCH_CLS(ET)                                                                                           \
-    k_sur_classify<ET><<<g2, 256, 0, st>>>(md->nelem, md->d_coords, md->d_conn, md->d_eqn, md->d_emat, md->d_mat, \
-                                           uf, up, md->d_state, md->ngp_total, md->sur_band, md->sur_scales[0],   \
-                                           md->d_srej, md->d_slot, md->d_qcount, md->d_sx)
-        if (md->etype == HIPFEM_LSPACE) LAUNCH_CLS(HIPFEM_LSPACE);
-        else if (md->etype == HIPFEM_LTRSPACE) LAUNCH_CLS(HIPFEM_LTRSPACE);
-        else LAUNCH_CLS(HIPFEM_QSPACE);
-#undef LAUNCH_CLS
+        const ClassifyArgs C = {md->nelem, md->d_coords, md->d_conn, md->d_eqn, md->d_emat, md->d_mat, uf, up,
+                                md->d_state, md->ngp_total, md->sur_band, md->sur_scales[0], md->d_srej, md->d_slot,
+                                md->d_qcount, md->d_sx};
+        if (md->etype == HIPFEM_LSPACE) k_sur_classify_hex<<<(md->ngp_total + 1023) / 1024, 1024, 0, st>>>(C);
+        else if (md->etype == HIPFEM_LTRSPACE) k_sur_classify<HIPFEM_LTRSPACE><<<g2, 256, 0, st>>>(C);
+        else k_sur_classify<HIPFEM_QSPACE><<<g2, 256, 0, st>>>(C);
         HIPFEM_CHECK(hipGetLastError());
         int nq = 0;
         HIPFEM_CHECK(hipMemcpyAsync(md->ctx->h_pinned, md->d_qcount, sizeof(int), hipMemcpyDeviceToHost, st));
@@ -2292,8 +2367,8 @@ static int internal_dev(hfem_model *md, const double *uf, const double *up, doub
         sur.flag = md->d_sflag;
         sur.rejected = md->d_srej;
         sur.counts = md->d_scounts;
-        sur.sig_scale = md->sur_scales[1];
-        sur.tan_scale = md->sur_scales[2];
+        sur.sig_inv = 1.0 / (double)md->sur_scales[1];
+        sur.tan_inv = 1.0 / (double)md->sur_scales[2];
         sur.tol = md->sur_tol;
     }
     if (md->nelem) {
@@ -2396,10 +2471,10 @@ extern "C" int hfem_model_set_surrogate(hfem_model *md, hfem_mlp *net, double ba
         HIPFEM_CHECK(hipMalloc(&md->d_dsnap, sizeof(float) * n * 21));
         HIPFEM_CHECK(hipMalloc(&md->d_sflag, n));
         HIPFEM_CHECK(hipMalloc(&md->d_srej, n));
-        HIPFEM_CHECK(hipMalloc(&md->d_scounts, 2 * sizeof(unsigned long long)));
+        HIPFEM_CHECK(hipMalloc(&md->d_scounts, SUR_LINES * SUR_LINE * sizeof(unsigned long long)));
         HIPFEM_CHECK(hipMemset(md->d_sflag, 0, n));
         HIPFEM_CHECK(hipMemset(md->d_srej, 0, n));
-        HIPFEM_CHECK(hipMemset(md->d_scounts, 0, 2 * sizeof(unsigned long long)));
+        HIPFEM_CHECK(hipMemset(md->d_scounts, 0, SUR_LINES * SUR_LINE * sizeof(unsigned long long)));
     }
     md->sur = net;
     md->sur_band = band;
@@ -2419,12 +2494,15 @@ extern "C" int hfem_model_surrogate_stats(hfem_model *md, int64_t *counts3, int 
 {
     HIPFEM_REQUIRE(md && counts3, HIPFEM_EINVAL, "surrogate_stats: null argument");
     DeviceGuard g(md->ctx->device);
-    unsigned long long c[2] = {0, 0};
+    unsigned long long c[SUR_LINES * SUR_LINE] = {};
     HIPFEM_CHECK(hipStreamSynchronize(md->ctx->stream));
     if (md->d_scounts) HIPFEM_CHECK(hipMemcpy(c, md->d_scounts, sizeof c, hipMemcpyDeviceToHost));
     counts3[0] = (int64_t)md->queued_total;
-    counts3[1] = (int64_t)c[0];
-    counts3[2] = (int64_t)c[1];
+    counts3[1] = counts3[2] = 0;
+    for (int i = 0; i < SUR_LINES; i++) {
+        counts3[1] += (int64_t)c[SUR_LINE * i];
+        counts3[2] += (int64_t)c[SUR_LINE * i + 1];
+    }
     if (reset) {
         md->queued_total = 0;
         if (md->d_scounts) HIPFEM_CHECK(hipMemset(md->d_scounts, 0, sizeof c));

@@ -199,6 +199,45 @@ def test_surrogate_update_is_checked_and_falls_back(ctx, trained, tol):
     ev.set_surrogate(None)
 
 
+@pytest.mark.parametrize("kind", ["hex", "tet", "quad"])
+def test_queue_holds_the_points_beyond_the_band(ctx, trained, kind):
+    """The queue of each element type's classification, on point counts that
+    leave part of a block empty and with an elastic second material: exactly
+    the points whose plain return map (from a zero state, kappa = excess /
+    (3G + H)) exceeds the band, and after a rejection only the others."""
+    from oofem_amd import meshgen
+    from oofem_amd.hipfem import BatchedEvaluator, HipCSRSparseMtrx
+    if kind == "quad":
+        et, (coords, conn) = meshgen.QSPACE, meshgen._rve_mesh(2, meshgen.QSPACE)[:2]
+    elif kind == "tet":
+        et, (coords, conn) = meshgen.LTRSPACE, meshgen.kuhn_tets(5, 4, 4, 1.0, 1.0, 1.0, jitter=0.1, seed=4)
+    else:
+        b = meshgen.cantilever_hex(5, 5, 7, jitter=0.2, seed=5)
+        et, coords, conn = meshgen.LSPACE, b.coords, b.conn
+    rng = np.random.default_rng(6)
+    emat = (rng.random(len(conn)) < 0.2).astype(np.int32)
+    mat = np.array([MP, [meshgen.MAT_ISOLE, 70e3, 0.2, 0, 0, 0, 0, 0]])
+    d = meshgen.Deck(kind, et, coords, conn, emat, mat, np.zeros(coords.shape, bool), np.zeros_like(coords))
+    ev = BatchedEvaluator(ctx, d)
+    K = HipCSRSparseMtrx(ctx)
+    ev.build_structure(K)
+    u = 0.25 * SIG0 / E * rng.standard_normal(d.neq)
+    ev.internal_forces(u, np.zeros(d.npeq), update_state=True)
+    excess = ev.get_state()[:, 13] * (1.5 * E / (1 + NU) + H)
+    assert (np.abs(excess - 0.05 * SIG0) > 1e-9 * SIG0).all()
+    ev.reset_state()
+    ev.set_surrogate(trained, band=0.05, tol=3e-3)
+    queued = int((excess > 0.05 * SIG0).sum())
+    assert 0 < queued < len(excess)
+    for _ in range(2):
+        ev.surrogate_stats(reset=True)
+        ev.internal_forces(u, np.zeros(d.npeq), update_state=True)
+        st = ev.surrogate_stats()
+        assert st["queued"] == queued and st["accepted"] + st["rejected"] == queued
+        queued = st["accepted"]
+    ev.set_surrogate(None)
+
+
 def test_trained_network_gains_over_untrained(ctx, trained):
     """What training buys: at a loose acceptance tolerance (3e-2) the trained
     network serves a share of the plastic points that pass every residual and
