@@ -122,16 +122,19 @@ __device__ __forceinline__ void add_parts(const double n[3], const double m[3], 
                 fma(-va[i], vb[j], fma(kd, P[3 * i + j], cd * (i == j ? P[4 * i] + nm : P[3 * j + i])));
 }
 
-// block += dV (lambda n m^T + G (m n^T + (n.m) I)), the isotropic elastic D
-__device__ __forceinline__ void add_elastic(const double n[3], const double m[3], double lam, double G, double dV,
-                                            double K[9])
+// block += dV (lambda n m^T + G (m n^T + (n.m) I)), the isotropic elastic D.
+// ln lm = lambda: lambda goes to the gradient of the lower local node and 1 to
+// the other, so that the blocks (a, b) and (b, a), formed by different waves,
+// are transposes bit for bit (a block (a, a) is symmetric to rounding only).
+__device__ __forceinline__ void add_elastic(const double n[3], const double m[3], double ln, double lm, double G,
+                                            double dV, double K[9])
 {
     const double nm = n[0] * m[0] + n[1] * m[1] + n[2] * m[2];
 #pragma unroll
     for (int i = 0; i < 3; i++)
 #pragma unroll
         for (int j = 0; j < 3; j++)
-            K[3 * i + j] += dV * (lam * n[i] * m[j] + G * (n[j] * m[i] + (i == j ? nm : 0.0)));
+            K[3 * i + j] += dV * (ln * n[i] * (lm * m[j]) + G * (n[j] * m[i] + (i == j ? nm : 0.0)));
 }
 
 // block += dV B_a^T D B_b with the general symmetric D of a surrogate point
@@ -172,8 +175,9 @@ __device__ __forceinline__ void clear_codes(int t, int L, uint64_t *codes)
 }
 
 // One pass's element rows (sV: SLOTS x 3 x NC doubles) summed into the node's
-// rows, in slot order.  Passes after the first add to what the lane itself
-// has written.  (Adding slot after slot into LDS rows instead moves 8 of 64
+// rows, in slot order.  Passes after the first go on from what the lane itself
+// has written: one running sum per entry in ascending element order, the same
+// for (i, j) and (j, i).  (Adding slot after slot into LDS rows instead moves 8 of 64
 // lanes at a time: 1.9 ms for the 1,085,825 nodes of the 64x64x256 block.)
 //
 // Hexahedra, 81 columns of up to 8 sources: each lane owns entries t, t + 64,
@@ -194,12 +198,12 @@ __device__ __forceinline__ void rows_sum_entries(int t, int q0, int q1, int q2, 
             const int c = (int)(w >> (8 * k)) & 255;
             v[k] = sV[c != 255 ? (k * 3 + i) * NC + c : zero];
         }
-        double s = 0.0;
-#pragma unroll
-        for (int k = 0; k < 8; k++) s += v[k];
         if (qi > 0) {
             double *o = val + rowptr[qi - 1] + p;
-            *o = first ? s : *o + s;
+            double s = first ? 0.0 : *o;
+#pragma unroll
+            for (int k = 0; k < 8; k++) s += v[k];
+            *o = s;
         }
     }
 }
@@ -214,6 +218,11 @@ __device__ __forceinline__ void rows_sum_columns(int t, const int q[3], int L, c
 {
     for (int p = t; p < L; p += 64) {
         double s[3] = {0.0, 0.0, 0.0};
+        if (!first) {
+#pragma unroll
+            for (int i = 0; i < 3; i++)
+                if (q[i] > 0) s[i] = val[rowptr[q[i] - 1] + p];
+        }
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             const uint64_t w = codes[2 * p + h];
@@ -228,10 +237,7 @@ __device__ __forceinline__ void rows_sum_columns(int t, const int q[3], int L, c
         }
 #pragma unroll
         for (int i = 0; i < 3; i++)
-            if (q[i] > 0) {
-                double *o = val + rowptr[q[i] - 1] + p;
-                *o = first ? s[i] : *o + s[i];
-            }
+            if (q[i] > 0) val[rowptr[q[i] - 1] + p] = s[i];
     }
 }
 
@@ -241,8 +247,11 @@ __device__ __forceinline__ void rows_sum_columns(int t, const int q[3], int L, c
 // lanes of a slot form J^-1 and the tangent parts of its four Gauss points
 // into LDS, and every lane then runs over those points, forming the gradients
 // g (and M g) of its two nodes and of the row's node a: one read of a point
-// serves two blocks.  The arithmetic of the elastic blocks is that of
-// k_assemble.
+// serves two blocks.  J^-1 (nine divisions), the gradients and the elastic
+// blocks are formed by the operations of gp_geometry and k_assemble in their
+// order, and the rows summed in ascending element order: K keeps the bits of
+// stored element matrices.  A mixed-precision solve to 1e-8 determines its
+// solution to about 1e-9, and one rounding of K moves it by as much.
 //
 // Bound: the latency of its loads and LDS round trips at two to three waves a
 // SIMD (202 VGPRs with the tangent, 164 without; bounding it to three or four
@@ -335,21 +344,9 @@ __global__ __launch_bounds__(64) void k_assemble_rows_hex(AsmArgs A)
                     }
                     if (c & 1) __builtin_amdgcn_sched_barrier(0);   // keeps two nodes' loads in flight
                 }
-                double P[NP];   // J^-1: the cofactors times one reciprocal
-                P[0] = J[4] * J[8] - J[5] * J[7];
-                P[1] = J[2] * J[7] - J[1] * J[8];
-                P[2] = J[1] * J[5] - J[2] * J[4];
-                P[3] = J[5] * J[6] - J[3] * J[8];
-                P[4] = J[0] * J[8] - J[2] * J[6];
-                P[5] = J[2] * J[3] - J[0] * J[5];
-                P[6] = J[3] * J[7] - J[4] * J[6];
-                P[7] = J[1] * J[6] - J[0] * J[7];
-                P[8] = J[0] * J[4] - J[1] * J[3];
-                const double det = J[0] * P[0] + J[1] * P[3] + J[2] * P[6];
-                if (!(fabs(det) > 1.e-30)) atomicMin(A.bad, e);
-                const double id = 1. / det, dV = fabs(det);   // the rule's weights are 1
-#pragma unroll
-                for (int i = 0; i < 9; i++) P[i] *= id;
+                double P[NP] = {}, dV = 0.0;
+                if (!hex_inverse(J, P, dV)) atomicMin(A.bad, e);
+                dV = fabs(dV);   // the rule's weights are 1
                 if constexpr (TAN) {
                     const size_t gp = (size_t)e * 8 + 4 * hx + q;
                     point_parts(mp, dV, ps, P[15], P[16], P + 9);
@@ -383,9 +380,8 @@ __global__ __launch_bounds__(64) void k_assemble_rows_hex(AsmArgs A)
 #pragma unroll
                     for (int j = 0; j < 3; j++) {
                         n[j] = cx * za * R[j] + cy * za * R[3 + j] + cz * R[6 + j];
-                        const double u = bx * R[j] + by * R[3 + j], v = bz * R[6 + j];
-                        m0[j] = zp * u + v;
-                        m1[j] = zm * u - v;
+                        m0[j] = bx * zp * R[j] + by * zp * R[3 + j] + bz * R[6 + j];
+                        m1[j] = bx * zm * R[j] + by * zm * R[3 + j] + -bz * R[6 + j];
                     }
                     if constexpr (TAN) {
                         if (SUR && R[17] < 0.0) {
@@ -401,8 +397,8 @@ __global__ __launch_bounds__(64) void k_assemble_rows_hex(AsmArgs A)
                             add_parts(n, m1, R[15], R[16], va, vb, K1);
                         }
                     } else {
-                        add_elastic(n, m0, lam, G, R[9], K0);
-                        add_elastic(n, m1, lam, G, R[9], K1);
+                        add_elastic(n, m0, a <= q ? lam : 1.0, a <= q ? 1.0 : lam, G, R[9], K0);
+                        add_elastic(n, m1, a <= q + 4 ? lam : 1.0, a <= q + 4 ? 1.0 : lam, G, R[9], K1);
                     }
                 }
             }
@@ -510,7 +506,8 @@ __global__ __launch_bounds__(64) void k_assemble_rows_tet(AsmArgs A)
                 add_parts(na, m, cd, kd, va, vb, K);
         } else {
             const double G = mp[1] / (2.0 * (1. + mp[2]));
-            add_elastic(na, m, mp[1] / (3.0 * (1. - 2. * mp[2])) - 2.0 * G / 3.0, G, dV, K);
+            const double lam = mp[1] / (3.0 * (1. - 2. * mp[2])) - 2.0 * G / 3.0;
+            add_elastic(na, m, a <= b ? lam : 1.0, a <= b ? 1.0 : lam, G, dV, K);
         }
         clear_codes<16>(t, L, sCodes);
 #pragma unroll
@@ -625,7 +622,7 @@ __global__ __launch_bounds__(256) void k_element_matrices_quad(AsmArgs A, double
                 add_parts(n, m, sQ[g][1], sQ[g][2], va, vb, K);
             }
         } else {
-            add_elastic(n, m, lam, G, sQ[g][0], K);
+            add_elastic(n, m, lam, 1.0, G, sQ[g][0], K);
         }
     }
     double *o = kbuf + (size_t)e * 3600;

@@ -144,10 +144,32 @@ struct ElemT<HIPFEM_QSPACE> {
     static constexpr int NEN = 20, NGP = 27;
 };
 
+// J^-1 of a hexahedron's point by cofactors (floatmatrix.C:768-815) and detJ by
+// FloatMatrix::giveDeterminant (floatmatrix.C:1085-1101); false where degenerate
+__device__ __forceinline__ bool hex_inverse(const double J[9], double I[9], double &detJ)
+{
+#define S(r, c) J[3 * ((r)-1) + ((c)-1)]
+    const double det = S(1, 1) * S(2, 2) * S(3, 3) + S(1, 2) * S(2, 3) * S(3, 1) + S(1, 3) * S(2, 1) * S(3, 2) -
+                       S(1, 3) * S(2, 2) * S(3, 1) - S(2, 3) * S(3, 2) * S(1, 1) - S(3, 3) * S(1, 2) * S(2, 1);
+    if (!(fabs(det) > 1.e-30)) return false;
+    I[0] = (S(2, 2) * S(3, 3) - S(2, 3) * S(3, 2)) / det;
+    I[3] = (S(2, 3) * S(3, 1) - S(2, 1) * S(3, 3)) / det;
+    I[6] = (S(2, 1) * S(3, 2) - S(2, 2) * S(3, 1)) / det;
+    I[1] = (S(1, 3) * S(3, 2) - S(1, 2) * S(3, 3)) / det;
+    I[4] = (S(1, 1) * S(3, 3) - S(1, 3) * S(3, 1)) / det;
+    I[7] = (S(1, 2) * S(3, 1) - S(1, 1) * S(3, 2)) / det;
+    I[2] = (S(1, 2) * S(2, 3) - S(1, 3) * S(2, 2)) / det;
+    I[5] = (S(1, 3) * S(2, 1) - S(1, 1) * S(2, 3)) / det;
+    I[8] = (S(1, 1) * S(2, 2) - S(1, 2) * S(2, 1)) / det;
+#undef S
+    detJ = J[0] * J[4] * J[8] + J[3] * J[7] * J[2] + J[6] * J[1] * J[5] - J[2] * J[4] * J[6] -
+           J[5] * J[7] * J[0] - J[8] * J[1] * J[3];
+    return true;
+}
+
 // Geometry at one Gauss point: dNdx (NEN x 3) and detJ.  Hexahedra:
-// J = X dN/dxi, closed-form inverse (floatmatrix.C:768-815), dNdx = dN/dxi J^-1,
-// detJ by FloatMatrix::giveDeterminant (floatmatrix.C:1085-1101).  Tetrahedra:
-// cofactor form of FEI3dTetLin::evaldNdx (fei3dtetlin.C:116-168).
+// J = X dN/dxi, dNdx = dN/dxi J^-1.  Tetrahedra: cofactor form of
+// FEI3dTetLin::evaldNdx (fei3dtetlin.C:116-168).
 // X is NEN x 3 (row-major).  Returns false for a degenerate element.
 template <int ET>
 __device__ bool gp_geometry(const double *X, const double xi[3], double *dNdx, double &detJ)
@@ -188,23 +210,8 @@ __device__ bool gp_geometry(const double *X, const double xi[3], double *dNdx, d
 #pragma unroll
                 for (int j = 0; j < 3; j++) J[3 * i + j] += X[3 * a + i] * dN[3 * a + j];
         }
-#define S(r, c) J[3 * ((r)-1) + ((c)-1)]
-        const double det = S(1, 1) * S(2, 2) * S(3, 3) + S(1, 2) * S(2, 3) * S(3, 1) + S(1, 3) * S(2, 1) * S(3, 2) -
-                           S(1, 3) * S(2, 2) * S(3, 1) - S(2, 3) * S(3, 2) * S(1, 1) - S(3, 3) * S(1, 2) * S(2, 1);
-        if (!(fabs(det) > 1.e-30)) return false;
         double I[9];
-        I[0] = (S(2, 2) * S(3, 3) - S(2, 3) * S(3, 2)) / det;
-        I[3] = (S(2, 3) * S(3, 1) - S(2, 1) * S(3, 3)) / det;
-        I[6] = (S(2, 1) * S(3, 2) - S(2, 2) * S(3, 1)) / det;
-        I[1] = (S(1, 3) * S(3, 2) - S(1, 2) * S(3, 3)) / det;
-        I[4] = (S(1, 1) * S(3, 3) - S(1, 3) * S(3, 1)) / det;
-        I[7] = (S(1, 2) * S(3, 1) - S(1, 1) * S(3, 2)) / det;
-        I[2] = (S(1, 2) * S(2, 3) - S(1, 3) * S(2, 2)) / det;
-        I[5] = (S(1, 3) * S(2, 1) - S(1, 1) * S(2, 3)) / det;
-        I[8] = (S(1, 1) * S(2, 2) - S(1, 2) * S(2, 1)) / det;
-#undef S
-        detJ = J[0] * J[4] * J[8] + J[3] * J[7] * J[2] + J[6] * J[1] * J[5] - J[2] * J[4] * J[6] -
-               J[5] * J[7] * J[0] - J[8] * J[1] * J[3];
+        if (!hex_inverse(J, I, detJ)) return false;
 #pragma unroll
         for (int a = 0; a < NEN; a++)
 #pragma unroll

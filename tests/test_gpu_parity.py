@@ -9,6 +9,7 @@ import os
 
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
 from oofem_amd import meshgen
 from oofem_amd.deck import evaluate_checks, read_deck
@@ -684,3 +685,44 @@ def test_row_assembly_edges_match_oracle(ctx, kind, tangent):
         assert np.abs(gval - val).max() <= (1e-12 if tangent else 1e-13) * np.abs(val).max()
         assert _ == 0 or np.array_equal(gval, first)
         first = gval
+
+
+def test_elastic_rows_keep_the_bits_of_the_element_matrices(ctx):
+    """Elastic LSpace rows against the color form on the same elements: a
+    chain of distorted hexahedra assembled alone (row form), and beside a star
+    whose centre row sends the whole mesh to the color form.  At most two
+    elements share a node, so the order of the sums does not matter, and the
+    blocks (a, b), a <= b (the same order in both elements of a shared face),
+    agree bit for bit; a block (b, a) of the row form is the transpose."""
+    from oofem_amd.hipfem import BatchedEvaluator, HipCSRSparseMtrx
+    rng = np.random.default_rng(3)
+    c = meshgen.cantilever_hex(1, 1, 9, jitter=0.3, e_sigma=0.5, seed=8)
+    star = _row_form_deck("hex_star")
+    nn, ne = len(c.coords), len(c.conn)
+    elastic = np.array([[meshgen.MAT_ISOLE, 70e3, 0.2, 0, 0, 0, 0, 0]])
+    mat = np.concatenate([c.mat, elastic])
+
+    def rows(coords, conn, emat):
+        bc = np.zeros((len(coords), 3), bool)
+        ev = BatchedEvaluator(ctx, meshgen.Deck("k", meshgen.LSPACE, coords, conn, emat, mat, bc, np.zeros_like(coords)))
+        K = HipCSRSparseMtrx(ctx)
+        ev.build_structure(K)
+        ev.assemble_stiffness(K)
+        rp, ci, val = K.download()
+        return sp.csr_matrix((val, ci, rp))[:3 * nn, :3 * nn].toarray(), np.diff(rp).max()
+
+    row, longest = rows(c.coords, c.conn, c.emat)
+    assert longest <= 512
+    both = np.concatenate([c.coords, star.coords + 20.0 + rng.random(3)])
+    color, longest = rows(both, np.concatenate([c.conn, star.conn + nn]),
+                          np.concatenate([c.emat, np.full(len(star.conn), len(mat) - 1, np.int32)]))
+    assert longest > 512
+    checked = set()
+    for e in range(ne):
+        for a in range(8):
+            for b in range(a, 8):
+                i, j = 3 * int(c.conn[e, a]), 3 * int(c.conn[e, b])
+                assert np.array_equal(row[i:i + 3, j:j + 3], color[i:i + 3, j:j + 3]), (e, a, b)
+                assert a == b or np.array_equal(row[j:j + 3, i:i + 3], row[i:i + 3, j:j + 3].T), (e, a, b)
+                checked.add((i, j))
+    assert len(checked) == nn + (28 * ne - 6 * (ne - 1)) and np.abs(row).max() > 0
