@@ -100,8 +100,9 @@ __device__ __forceinline__ void tensor_times(const double m[6], const double g[3
 
 // block += cd ((n.m) I + m n^T) + kd n m^T - va vb^T (n = g_a, m = g_b).  The
 // products n_i m_j are shared by the entries (i, j) and (j, i), and the block
-// (b, a) of another wave gets the same bits transposed: K is exactly
-// symmetric.  Each point's contribution is formed apart and added once: with
+// (b, a) of another wave gets the same bits transposed (the gradient of a node
+// is the same expression as row and as column): a tangent without surrogate
+// points is exactly symmetric.  Each point's contribution is formed apart and added once: with
 // its terms chained into the block by FMAs, the roundings of the larger
 // partial sums leave a rigid translation five times as far from force-free
 // (displacements of the 10x10x40 cantilever 5e-12 off instead of 5e-13).
@@ -137,18 +138,25 @@ __device__ __forceinline__ void add_elastic(const double n[3], const double m[3]
             K[3 * i + j] += dV * (ln * n[i] * (lm * m[j]) + G * (n[j] * m[i] + (i == j ? nm : 0.0)));
 }
 
-// block += dV B_a^T D B_b with the general symmetric D of a surrogate point
-__device__ __forceinline__ void add_general(const double n[3], const double m[3], double dV,
+// block += dV B_a^T D B_b with the general symmetric D of a surrogate point;
+// lower: a <= b.  The product is formed with the lower local node on the left
+// and transposed for b < a, so that (a, b) and (b, a) are transposes bit for bit.
+__device__ __forceinline__ void add_general(const double ga[3], const double gb[3], bool lower, double dV,
                                             const float *__restrict__ dsur, size_t ngp_total, size_t gp, double K[9])
 {
-    double D[36];
+    double D[36], n[3], m[3];
     int k = 0;
 #pragma unroll
     for (int r = 0; r < 6; r++)
 #pragma unroll
         for (int c = r; c < 6; c++, k++) D[6 * r + c] = D[6 * c + r] = (double)dsur[(size_t)k * ngp_total + gp];
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        n[i] = lower ? ga[i] : gb[i];
+        m[i] = lower ? gb[i] : ga[i];
+    }
     // columns of B_b: x (m0,0,0,0,m2,m1), y (0,m1,0,m2,0,m0), z (0,0,m2,m1,m0,0)
-    double DB[6][3];
+    double DB[6][3], V[9];
 #pragma unroll
     for (int r = 0; r < 6; r++) {
         DB[r][0] = D[6 * r + 0] * m[0] + D[6 * r + 4] * m[2] + D[6 * r + 5] * m[1];
@@ -157,10 +165,14 @@ __device__ __forceinline__ void add_general(const double n[3], const double m[3]
     }
 #pragma unroll
     for (int j = 0; j < 3; j++) {
-        K[0 + j] += dV * (n[0] * DB[0][j] + n[2] * DB[4][j] + n[1] * DB[5][j]);
-        K[3 + j] += dV * (n[1] * DB[1][j] + n[2] * DB[3][j] + n[0] * DB[5][j]);
-        K[6 + j] += dV * (n[2] * DB[2][j] + n[1] * DB[3][j] + n[0] * DB[4][j]);
+        V[0 + j] = n[0] * DB[0][j] + n[2] * DB[4][j] + n[1] * DB[5][j];
+        V[3 + j] = n[1] * DB[1][j] + n[2] * DB[3][j] + n[0] * DB[5][j];
+        V[6 + j] = n[2] * DB[2][j] + n[1] * DB[3][j] + n[0] * DB[4][j];
     }
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) K[3 * i + j] += dV * (lower ? V[3 * i + j] : V[3 * j + i]);
 }
 
 // The sources of a node's columns in one pass of SLOTS elements: byte slot of
@@ -386,8 +398,8 @@ __global__ __launch_bounds__(64) void k_assemble_rows_hex(AsmArgs A)
                     if constexpr (TAN) {
                         if (SUR && R[17] < 0.0) {
                             const size_t gp = (size_t)e * 8 + 4 * hx + 2 * hy + hz;
-                            add_general(n, m0, -R[17], A.dsur, A.ngp_total, gp, K0);
-                            add_general(n, m1, -R[17], A.dsur, A.ngp_total, gp, K1);
+                            add_general(n, m0, a <= q, -R[17], A.dsur, A.ngp_total, gp, K0);
+                            add_general(n, m1, a <= q + 4, -R[17], A.dsur, A.ngp_total, gp, K1);
                         } else {
                             double va[3], vb[3];
                             tensor_times(R + 9, n, va);
@@ -501,7 +513,7 @@ __global__ __launch_bounds__(64) void k_assemble_rows_tet(AsmArgs A)
         }
         if constexpr (TAN) {
             if (SUR && A.sflag[e])
-                add_general(na, m, dV, A.dsur, A.ngp_total, e, K);
+                add_general(na, m, a <= b, dV, A.dsur, A.ngp_total, e, K);
             else
                 add_parts(na, m, cd, kd, va, vb, K);
         } else {
@@ -529,7 +541,7 @@ __global__ __launch_bounds__(64) void k_assemble_rows_tet(AsmArgs A)
 // K_e of every QSpace element, 60 x 60 row-major: 256 threads an element.
 // The (point, node) pairs, the 9 entries of every point's J and the 210 node
 // pairs a <= b are each shared out over the threads; a block is stored with
-// its transpose, so every element matrix is exactly symmetric.
+// its transpose.
 //
 // Bound: LDS reads of the gradients (7 doubles a pair and point, 15 with the
 // tangent).  9,261 elements: 0.157 ms and 0.153 ms for the rows summed from
@@ -614,7 +626,7 @@ __global__ __launch_bounds__(256) void k_element_matrices_quad(AsmArgs A, double
         const double m[3] = {sN[g][3 * b], sN[g][3 * b + 1], sN[g][3 * b + 2]};
         if constexpr (TAN) {
             if (SUR && sQ[g][0] < 0.0) {
-                add_general(n, m, -sQ[g][0], A.dsur, A.ngp_total, (size_t)e * NGP + g, K);
+                add_general(n, m, true, -sQ[g][0], A.dsur, A.ngp_total, (size_t)e * NGP + g, K);
             } else {
                 double va[3], vb[3];
                 tensor_times(&sQ[g][3], n, va);

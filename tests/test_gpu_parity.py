@@ -726,3 +726,33 @@ def test_elastic_rows_keep_the_bits_of_the_element_matrices(ctx):
                 assert a == b or np.array_equal(row[j:j + 3, i:i + 3], row[i:i + 3, j:j + 3].T), (e, a, b)
                 checked.add((i, j))
     assert len(checked) == nn + (28 * ne - 6 * (ne - 1)) and np.abs(row).max() > 0
+
+
+@pytest.mark.parametrize("tangent", [False, True])
+@pytest.mark.parametrize("kind", ["hex_partial", "hex_repeated", "tet_partial", "tet_repeated", "quad_partial",
+                                  "quad_repeated"])
+def test_row_blocks_are_transposes(ctx, kind, tangent):
+    """The rows of two nodes are formed by different waves, in several passes
+    where a node has more elements than one takes: their blocks (I, J) and
+    (J, I) are transposes bit for bit, and the tangent of MisesMat and elastic
+    points is symmetric bit for bit altogether (an elastic matrix to rounding
+    within the blocks (I, I))."""
+    from oofem_amd.hipfem import BatchedEvaluator, HipCSRSparseMtrx
+    d = _row_form_deck(kind)
+    ev = BatchedEvaluator(ctx, d)
+    K = HipCSRSparseMtrx(ctx)
+    ev.build_structure(K)
+    if tangent:
+        u = np.random.default_rng(5).standard_normal(d.neq) * 4e-3
+        ev.internal_forces(u, np.zeros(d.npeq), update_state=True)
+        assert (ev.get_state()[:, 13] > 0).any()
+    ev.assemble_stiffness(K, tangent=tangent)
+    rp, ci, val = K.download()
+    A = sp.csr_matrix((val, ci, rp), (d.neq, d.neq)).toarray()
+    node = np.zeros(d.neq, np.int64)
+    n, c = np.nonzero(d.eqn > 0)
+    node[d.eqn[n, c] - 1] = n
+    same = node[:, None] == node[None, :]
+    asym = A != A.T
+    assert not (asym & ~same).any()
+    assert not (asym & same).any() if tangent else np.abs((A - A.T)[same]).max() <= 1e-13 * np.abs(A).max()

@@ -238,6 +238,102 @@ def test_queue_holds_the_points_beyond_the_band(ctx, trained, kind):
     ev.set_surrogate(None)
 
 
+def _typed_block(ctx, kind, n):
+    """A distorted block of one element type, a fifth of it elastic."""
+    from oofem_amd import meshgen
+    from oofem_amd.hipfem import BatchedEvaluator, HipCSRSparseMtrx
+    if kind == "quad":
+        et, (coords, conn) = meshgen.QSPACE, meshgen._rve_mesh(n, meshgen.QSPACE)[:2]
+    elif kind == "tet":
+        et, (coords, conn) = meshgen.LTRSPACE, meshgen.kuhn_tets(n, n, n, 1.0, 1.0, 1.0, jitter=0.1, seed=4)
+    else:
+        b = meshgen.cantilever_hex(n, n, n, jitter=0.2, seed=5)
+        et, coords, conn = meshgen.LSPACE, b.coords, b.conn
+    emat = (np.random.default_rng(6).random(len(conn)) < 0.2).astype(np.int32)
+    mat = np.array([MP, [meshgen.MAT_ISOLE, 70e3, 0.2, 0, 0, 0, 0, 0]])
+    d = meshgen.Deck(kind, et, coords, conn, emat, mat, np.zeros(coords.shape, bool), np.zeros_like(coords))
+    ev = BatchedEvaluator(ctx, d)
+    K = HipCSRSparseMtrx(ctx)
+    ev.build_structure(K)
+    return d, ev, K
+
+
+@pytest.mark.parametrize("kind,n", [("hex", 4), ("tet", 5), ("quad", 3)])
+def test_accepted_points_in_state_forces_and_tangent(ctx, trained, kind, n):
+    """What an accepted prediction becomes, for every element type.  From a
+    zero state the network's input is the strain alone, so the predictions are
+    recomputed here from the stored strains with the same BF16 inference.
+    Accepted points hold the predicted stress and its plastic strain, all
+    others the plain update bit for bit; the forces are those of the stored
+    stresses; and the matrix is assembled here from the predicted tangents
+    (kept in FP32, 6e-8 of an entry) and the consistent ones of the others.
+    Blocks (I, J) and (J, I) of the matrix are transposes bit for bit."""
+    import scipy.sparse as sp
+
+    d, ev, K = _typed_block(ctx, kind, n)
+    u = 0.25 * SIG0 / E * np.random.default_rng(6).standard_normal(d.neq)
+    up = np.zeros(d.npeq)
+    ev.internal_forces(u, up, update_state=True)
+    plain = ev.get_state()
+    ev.reset_state()
+    ev.set_surrogate(trained, band=0.05, tol=6e-2)
+    ev.surrogate_stats(reset=True)
+    f, _, _ = ev.internal_forces(u, up, update_state=True)
+    ev.assemble_stiffness(K, tangent=True)
+    s, st = ev.get_state(), ev.surrogate_stats()
+    acc = (s[:, 20:26] != plain[:, 20:26]).any(axis=1)
+    assert st["accepted"] == acc.sum() > 0 and st["rejected"] > 0
+    assert np.array_equal(s[~acc], plain[~acc])
+    # the predictions of the accepted points
+    eps = s[acc, 26:32]
+    in_scale, sig_scale, tan_scale = (float(np.float32(v)) for v in (E / SIG0, 1 / SIG0, 1 / E))
+    X = np.zeros((acc.sum(), 13), np.float32)
+    X[:, :6] = (eps * in_scale).astype(np.float32)
+    Y = trained.infer_bf16(X).astype(np.float64)
+    De = oracle.isole_D(E, NU)
+    sig = eps @ De - Y[:, :6] / sig_scale
+    assert np.abs(s[acc, 20:26] - sig).max() <= 1e-9 * SIG0
+    epsp = eps - np.linalg.solve(De, sig.T).T
+    assert np.abs(s[acc, 7:13] - epsp).max() <= 1e-9 * SIG0 / E
+    iu = np.triu_indices(6)
+    D, Da = np.zeros((len(s), 6, 6)), np.zeros((acc.sum(), 6, 6))
+    Da[:, iu[0], iu[1]] = Da[:, iu[1], iu[0]] = De[iu] - Y[:, 6:] / tan_scale
+    D[acc] = Da
+    xi, w = oracle.gauss(d.etype)
+    ng = len(w)
+    fo = np.zeros(d.neq)
+    rows, cols, vals = [], [], []
+    for e in range(d.nelem):
+        mp = d.mat[d.emat[e]]
+        X3 = d.coords[d.conn[e]]
+        q = d.eqn[d.conn[e]].ravel() - 1
+        for g in range(ng):
+            i = e * ng + g
+            if not acc[i]:
+                D[i] = oracle.isole_D(mp[1], mp[2]) if mp[0] == 0 else oracle.mises_tangent(mp, 0.0, s[i, 13], s[i, 14:20])
+            det, dN, _ = oracle.dndx(d.etype, X3, xi[g])
+            B = np.zeros((6, q.size))
+            for r, (a, b) in enumerate([(0, 0), (1, 1), (2, 2), (1, 2), (0, 2), (0, 1)]):
+                B[r, a::3] += dN[:, b]
+                if a != b:
+                    B[r, b::3] += dN[:, a]
+            fo[q] += B.T @ s[i, 20:26] * abs(det) * w[g]
+        Ke = oracle.element_stiffness(d.etype, X3, D[e * ng:(e + 1) * ng], symmetric=False)
+        rows.append(np.repeat(q, q.size))
+        cols.append(np.tile(q, q.size))
+        vals.append(Ke.ravel())
+    assert np.abs(f - fo).max() <= 1e-12 * np.abs(fo).max()
+    A = sp.csr_matrix((np.concatenate(vals), (np.concatenate(rows), np.concatenate(cols))), (d.neq, d.neq)).toarray()
+    rp, ci, val = K.download()
+    G = sp.csr_matrix((val, ci, rp), (d.neq, d.neq)).toarray()
+    assert np.abs(G - A).max() <= 1e-6 * np.abs(A).max()
+    node = np.zeros(d.neq, np.int64)
+    nn, c = np.nonzero(d.eqn > 0)
+    node[d.eqn[nn, c] - 1] = nn
+    assert not ((G != G.T) & (node[:, None] != node[None, :])).any()
+    ev.set_surrogate(None)
+
+
 def test_trained_network_gains_over_untrained(ctx, trained):
     """What training buys: at a loose acceptance tolerance (3e-2) the trained
     network serves a share of the plastic points that pass every residual and
