@@ -227,6 +227,25 @@ __device__ bool gp_geometry(const double *X, const double xi[3], double *dNdx, d
 
 namespace hipfem {
 
+// The geometry check of the elements that no row visits (every dof
+// prescribed); one thread an element
+template <int ET>
+__global__ __launch_bounds__(64) void k_check_elements(const int *__restrict__ elems, int n,
+                                                       const double *__restrict__ coords, const int *__restrict__ conn,
+                                                       int *__restrict__ bad)
+{
+    constexpr int NEN = ElemT<ET>::NEN, NGP = ElemT<ET>::NGP;
+    const int i = blockIdx.x * 64 + threadIdx.x;
+    if (i >= n) return;
+    const int e = elems[i];
+    double X[NEN * 3], dNdx[NEN * 3], xi[3], w, detJ;
+    for (int k = 0; k < NEN * 3; k++) X[k] = coords[3 * (size_t)conn[(size_t)e * NEN + k / 3] + k % 3];
+    for (int g = 0; g < NGP; g++) {
+        gauss_point(ET, g, xi, w);
+        if (!gp_geometry<ET>(X, xi, dNdx, detJ)) atomicMin(bad, e);
+    }
+}
+
 // ------------------------------------------------------------ assembly kernel
 template <int ET>
 __global__ __launch_bounds__(64) void k_assemble(const int *__restrict__ elems, int nelem_color,
@@ -1693,6 +1712,9 @@ struct hfem_model {
     double *d_kbuf = nullptr;
     bool kbuf_failed = false;
     int max_rowlen = 0;
+    // elements without a free dof, which no row visits
+    int *d_norow = nullptr;
+    int n_norow = 0;
     // per element and k_mf_hex lane g: first free equation (0-based, bits
     // 0..28) and free-dof mask (bits 29..31) of the lane's node; built once
     // per mesh when every node numbers its free dofs consecutively
@@ -1729,7 +1751,7 @@ static int model_free(hfem_model *md)
     void *ps[] = {md->d_coords, md->d_mat, md->d_state, md->d_conn, md->d_emat, md->d_eqn, md->d_bad,
                   md->d_eoff,   md->d_colors, md->d_uf, md->d_up, md->d_ff, md->d_fp, md->d_out3, md->d_dofid,
                   md->d_tdesc, md->d_nptr, md->d_nadj, md->d_ebuf, md->d_ecolor, md->d_eqmask, md->d_yslot,
-                  md->d_erel, md->d_eloc, md->d_fnptr, md->d_fnadj, md->d_fbuf, md->d_kbuf};
+                  md->d_erel, md->d_eloc, md->d_fnptr, md->d_fnadj, md->d_fbuf, md->d_kbuf, md->d_norow};
     for (void *p : ps)
         if (p) HIPFEM_CHECK(hipFree(p));
     md->d_tdesc = nullptr;
@@ -1746,6 +1768,8 @@ static int model_free(hfem_model *md)
     md->d_kbuf = nullptr;
     md->kbuf_failed = false;
     md->max_rowlen = 0;
+    md->d_norow = nullptr;
+    md->n_norow = 0;
     md->d_coords = md->d_mat = md->d_state = md->d_uf = md->d_up = md->d_ff = md->d_fp = md->d_out3 = nullptr;
     md->d_conn = md->d_emat = md->d_eqn = md->d_bad = md->d_colors = nullptr;
     md->d_dofid = nullptr;
@@ -2001,15 +2025,29 @@ extern "C" int hfem_model_build_structure(hfem_model *md, hipcsr_mtx *K)
         std::vector<int> fill(cptr.begin(), cptr.end() - 1);
         for (int e = 0; e < nelem; e++) clist[fill[color[e]]++] = e;
     }
+    std::vector<int> norow;
+    for (int e = 0; e < nelem; e++) {
+        bool free = false;
+        for (int a = 0; a < nen; a++) free = free || nfree(conn[(size_t)e * nen + a]);
+        if (!free) norow.push_back(e);
+    }
     int rc = csr_alloc(K, neq, rowptr, colind);
     if (rc) return rc;
     hipStream_t st = md->ctx->stream;
     if (md->d_eoff) HIPFEM_CHECK(hipFree(md->d_eoff));
     if (md->d_colors) HIPFEM_CHECK(hipFree(md->d_colors));
+    if (md->d_norow) HIPFEM_CHECK(hipFree(md->d_norow));
     md->d_eoff = nullptr;
     md->d_colors = nullptr;
+    md->d_norow = nullptr;
+    md->n_norow = 0;
     HIPFEM_CHECK(hipMalloc(&md->d_eoff, sizeof(uint16_t) * std::max<size_t>(1, eoff.size())));
     HIPFEM_CHECK(hipMalloc(&md->d_colors, sizeof(int) * std::max(1, nelem)));
+    if (!norow.empty()) {
+        HIPFEM_CHECK(hipMalloc(&md->d_norow, sizeof(int) * norow.size()));
+        HIPFEM_CHECK(hipMemcpyAsync(md->d_norow, norow.data(), sizeof(int) * norow.size(), hipMemcpyHostToDevice, st));
+        md->n_norow = (int)norow.size();
+    }
     if (!eoff.empty())
         HIPFEM_CHECK(hipMemcpyAsync(md->d_eoff, eoff.data(), sizeof(uint16_t) * eoff.size(), hipMemcpyHostToDevice, st));
     if (nelem) HIPFEM_CHECK(hipMemcpyAsync(md->d_colors, clist.data(), sizeof(int) * nelem, hipMemcpyHostToDevice, st));
@@ -2091,6 +2129,16 @@ extern "C" int hfem_model_assemble_stiffness(hfem_model *md, hipcsr_mtx *K, int 
         }
 #undef LAUNCH_ROWS
         HIPFEM_CHECK(hipGetLastError());
+        if (md->n_norow && !quad) {   // k_element_matrices_quad sees every element
+            const int nb = (md->n_norow + 63) / 64;
+            if (hex)
+                k_check_elements<HIPFEM_LSPACE><<<nb, 64, 0, st>>>(md->d_norow, md->n_norow, md->d_coords, md->d_conn,
+                                                                   md->d_bad);
+            else
+                k_check_elements<HIPFEM_LTRSPACE><<<nb, 64, 0, st>>>(md->d_norow, md->n_norow, md->d_coords,
+                                                                     md->d_conn, md->d_bad);
+            HIPFEM_CHECK(hipGetLastError());
+        }
         if (quad) {
             k_assemble_gather<20><<<md->nnode, 64, 8 * (size_t)md->max_rowlen, st>>>(A, md->d_kbuf);
             HIPFEM_CHECK(hipGetLastError());

@@ -756,3 +756,32 @@ def test_row_blocks_are_transposes(ctx, kind, tangent):
     asym = A != A.T
     assert not (asym & ~same).any()
     assert not (asym & same).any() if tangent else np.abs((A - A.T)[same]).max() <= 1e-13 * np.abs(A).max()
+
+
+@pytest.mark.parametrize("fixed", [False, True])
+@pytest.mark.parametrize("kind", ["hex", "tet", "quad"])
+def test_assembly_refuses_a_degenerate_element(ctx, kind, fixed):
+    """A flat (hexahedra) or inverted (tetrahedra) element is refused by the
+    assembly with its number, also where all its nodes are prescribed, so that
+    it has no row; without it the same mesh is assembled."""
+    from oofem_amd.hipfem import BatchedEvaluator, HipCSRSparseMtrx, HipFemError
+    d = _row_form_deck(f"{kind}_partial")
+    nn = len(d.coords)
+    xyz = d.coords[d.conn[0]].copy()
+    if kind == "tet":
+        xyz = xyz[[1, 0, 2, 3]]
+    else:
+        xyz[:, 2] = 0.0   # det J is exactly zero
+    coords = np.concatenate([d.coords, xyz + [30.0, 30.0, 0.0]])
+    bad = np.arange(nn, nn + d.conn.shape[1])[None, :]
+    bc = np.concatenate([d.bc_mask, np.full(xyz.shape, fixed)])
+    for n, conn in ((0, d.conn), (3, np.concatenate([d.conn[:2], bad, d.conn[2:]]))):
+        emat = np.zeros(len(conn), np.int32)
+        ev = BatchedEvaluator(ctx, meshgen.Deck("bad", d.etype, coords, conn, emat, d.mat, bc, np.zeros_like(coords)))
+        K = HipCSRSparseMtrx(ctx)
+        ev.build_structure(K)
+        if n:
+            with pytest.raises(HipFemError, match=f"degenerate or inverted element {n}"):
+                ev.assemble_stiffness(K)
+        else:
+            ev.assemble_stiffness(K)
