@@ -538,7 +538,7 @@ __global__ __launch_bounds__(64) void k_assemble_rows_tet(AsmArgs A)
     }
 }
 
-// K_e of every QSpace element, 60 x 60 row-major: 256 threads an element.
+// K_e of the QSpace elements from e0 on, 60 x 60 row-major: 256 threads an element.
 // The (point, node) pairs, the 9 entries of every point's J and the 210 node
 // pairs a <= b are each shared out over the threads; a block is stored with
 // its transpose.
@@ -548,14 +548,14 @@ __global__ __launch_bounds__(64) void k_assemble_rows_tet(AsmArgs A)
 // them (267 MB each way); eight color launches of one wave an element, which
 // leave a SIMD one wave, took 0.78 ms.
 template <bool TAN, bool SUR>
-__global__ __launch_bounds__(256) void k_element_matrices_quad(AsmArgs A, double *__restrict__ kbuf)
+__global__ __launch_bounds__(256) void k_element_matrices_quad(AsmArgs A, double *__restrict__ kbuf, int e0)
 {
     constexpr int NGP = 27, NEN = 20;
     __shared__ double sX[60];
     __shared__ double sN[NGP][60];    // dN/dxi, then dN/dx
     __shared__ double sJ[NGP][9];     // J, then J^-1
     __shared__ double sQ[NGP][TAN ? 10 : 2];   // dV (< 0: surrogate D), [cd, kd, M (6)]
-    const int e = blockIdx.x, t = threadIdx.x;
+    const int e = e0 + blockIdx.x, t = threadIdx.x;
     for (int k = t; k < 60; k += 256) sX[k] = A.coords[3 * (size_t)A.conn[(size_t)e * NEN + k / 3] + k % 3];
     for (int k = t; k < NGP * NEN; k += 256) {
         double xi[3], w, d[3];
@@ -637,7 +637,7 @@ __global__ __launch_bounds__(256) void k_element_matrices_quad(AsmArgs A, double
             add_elastic(n, m, lam, 1.0, G, sQ[g][0], K);
         }
     }
-    double *o = kbuf + (size_t)e * 3600;
+    double *o = kbuf + (size_t)blockIdx.x * 3600;
 #pragma unroll
     for (int i = 0; i < 3; i++)
 #pragma unroll
@@ -650,11 +650,13 @@ __global__ __launch_bounds__(256) void k_element_matrices_quad(AsmArgs A, double
     }
 }
 
-// The rows of node n from the stored element matrices: eight elements a pass,
-// whose three rows (3 x 3 NEN contiguous doubles) go to LDS as they lie; the
-// columns are then summed and written once.  One wave per node.
+// The rows of node n from the stored matrices of elements [e0, e1): eight
+// elements a pass, whose three rows (3 x 3 NEN contiguous doubles) go to LDS as
+// they lie; the columns are then summed and written.  One wave per node.  The
+// running sums of a node whose elements lie in several ranges go on from val,
+// so the ranges do not change the result.
 template <int NEN>
-__global__ __launch_bounds__(64) void k_assemble_gather(AsmArgs A, const double *__restrict__ kbuf)
+__global__ __launch_bounds__(64) void k_assemble_gather(AsmArgs A, const double *__restrict__ kbuf, int e0, int e1)
 {
     constexpr int NC = 3 * NEN, ROW2 = 3 * NC / 2;   // 16-byte words of an element's three rows
     __shared__ __align__(16) double sV[8 * 3 * NC + 2];
@@ -670,14 +672,28 @@ __global__ __launch_bounds__(64) void k_assemble_gather(AsmArgs A, const double 
     const int r0 = q[0] > 0 ? q[0] : q[1] > 0 ? q[1] : q[2];
     if (r0 <= 0) return;   // no free dof: no rows
     const int L = A.rowptr[r0] - A.rowptr[r0 - 1];
-    const int j0 = A.nptr[n], cnt = A.nptr[n + 1] - j0;
+    const int jn = A.nptr[n];
+    int j0 = jn, j1 = A.nptr[n + 1];
+    if (e0 > 0 || e1 < A.nelem) {   // the list ascends: its part in [e0, e1)
+        for (int hi = j1; j0 < hi;) {
+            const int mid = (j0 + hi) / 2;
+            if (A.nadj[mid] < (int64_t)e0 * NEN) j0 = mid + 1;
+            else hi = mid;
+        }
+        for (int lo = j0; lo < j1;) {
+            const int mid = (lo + j1) / 2;
+            if (A.nadj[mid] < (int64_t)e1 * NEN) lo = mid + 1;
+            else j1 = mid;
+        }
+    }
+    const int cnt = j1 - j0;
     for (int base = 0; base < cnt; base += 8) {
         const int ns = min(8, cnt - base);
         d2_t v[(8 * ROW2 + 63) / 64];
 #pragma unroll
         for (int u = 0; u < (8 * ROW2 + 63) / 64; u++) {
             const int idx = u * 64 + t, s = min(idx / ROW2, ns - 1);
-            v[u] = reinterpret_cast<const d2_t *>(kbuf + (size_t)A.nadj[j0 + base + s] * (3 * NC))[idx % ROW2];
+            v[u] = reinterpret_cast<const d2_t *>(kbuf + ((size_t)A.nadj[j0 + base + s] - (size_t)e0 * NEN) * (3 * NC))[idx % ROW2];
         }
         clear_codes<8>(t, L, sCodes);
         uint8_t *bytes = reinterpret_cast<uint8_t *>(sCodes);
@@ -696,7 +712,7 @@ __global__ __launch_bounds__(64) void k_assemble_gather(AsmArgs A, const double 
             if (idx / ROW2 < ns) reinterpret_cast<d2_t *>(sV)[idx] = v[u];
         }
         wave_lds_fence();
-        rows_sum_entries<NC>(t, q[0], q[1], q[2], L, sV, 8 * 3 * NC, sCodes, A.rowptr, A.val, base == 0);
+        rows_sum_entries<NC>(t, q[0], q[1], q[2], L, sV, 8 * 3 * NC, sCodes, A.rowptr, A.val, j0 + base == jn);
     }
 }
 

@@ -464,6 +464,7 @@ static void ctx_free(hipfem_ctx *c)
     DeviceGuard g(c->device);
     (void)hipStreamSynchronize(c->stream);
     if (c->d_partials) (void)hipFree(c->d_partials);
+    if (c->d_elmat) (void)hipFree(c->d_elmat);
     if (c->h_pinned) (void)hipHostFree(c->h_pinned);
     (void)hipStreamDestroy(c->stream);
     delete c;

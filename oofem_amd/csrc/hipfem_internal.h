@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -111,6 +112,12 @@ struct hipfem_ctx {
     hipStream_t stream = nullptr;
     double *d_partials = nullptr;   // per-block partial sums (reduction scratch)
     size_t partials_cap = 0;        // in doubles
+    // element matrices of one QSpace assembly at a time (hipfem_model.hip):
+    // grown on use, bounded, shared by the context's models; the mutex is held
+    // from its growth to the last launch that uses it (the stream orders those)
+    double *d_elmat = nullptr;
+    size_t elmat_cap = 0;           // in bytes
+    std::mutex elmat_mutex;
     double *h_pinned = nullptr;     // small pinned host buffer for scalar readback
     // Objects created on the context hold a reference; hipfem_ctx_destroy on a
     // context with live objects only marks it, and the last object's destroy

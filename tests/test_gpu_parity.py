@@ -785,3 +785,38 @@ def test_assembly_refuses_a_degenerate_element(ctx, kind, fixed):
                 ev.assemble_stiffness(K)
         else:
             ev.assemble_stiffness(K)
+
+
+def test_quad_assembly_workspace_is_bounded(ctx):
+    """The element matrices of QSpace meshes with more elements than the
+    512 MiB workspace takes at once (18,641) go through it in ranges: the
+    stiffness times a vector is the evaluator's own product, the device memory
+    grows by the workspace at most, and a second evaluator adds none."""
+    import ctypes
+
+    from oofem_amd.hipfem import BatchedEvaluator, HipCSRSparseMtrx
+    hip = ctypes.CDLL("libamdhip64.so.7")   # the runtime that the library has loaded
+
+    def free_bytes():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    d = meshgen.rve(27, meshgen.QSPACE, 0.3, 1)
+    assert d.nelem > 18641
+    x = np.random.default_rng(2).standard_normal(d.neq)
+    free, keep = [], []
+    for _ in range(2):
+        ev = BatchedEvaluator(ctx, d)
+        K = HipCSRSparseMtrx(ctx)
+        ev.build_structure(K)
+        y = ev.tangent_product(x, np.zeros(d.npeq))[0]   # allocates the force buffers too
+        before = free_bytes()
+        ev.assemble_stiffness(K)
+        free.append(before - free_bytes())
+        assert np.abs(K.times(x) - y).max() <= 1e-12 * np.abs(y).max()
+        keep.append((ev, K))
+    assert free[0] <= (513 << 20) and free[1] <= (1 << 20), free
+    for ev, K in keep:
+        K.close()
+        ev.close()
