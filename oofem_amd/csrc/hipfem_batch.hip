@@ -326,7 +326,6 @@ struct BulkArgs {
     double *x;
     float *r, *z, *p, *q;
     double *part, *part_rz, *part_tr;   // [tile][NPART]: p.q; r.z and r.r; those of a reliable update
-    int fold;                // the partials of a block are summed into its first tile's by a launch of their own
     double tol, delta;
     int maxit;
     int *iters, *updates;
@@ -411,14 +410,18 @@ __global__ __launch_bounds__(BULK_TILE) void k_bulk_spmv(BulkArgs A)
 // needs them (a fixed order): no launch of its own for the reductions, whose
 // cost (5 to 7 us each) was its latency.  A thread sums one value over every SUM_GROUPS-th tile
 // (coalesced, no wave reduction), then one thread per value sums the groups.
+// folded: a large block's sums, which k_bulk_fold has left in its first tile's
+// place; decided per block, so that its bits do not depend on its neighbours.
 template <int NV, int G = SUM_GROUPS>
-__device__ __forceinline__ void tile_sums(const BulkArgs &A, int pos, const double *part, bool fold, double *sh,
+__device__ __forceinline__ void tile_sums(const BulkArgs &A, int pos, const double *part, bool folded, double *sh,
                                           double *red)
 {
     const int g = threadIdx.x / NV, k = threadIdx.x % NV;
     if (g < G) {
         double s = 0.0;
-        const int t0 = A.act_t0[pos], t1 = fold ? t0 + 1 : A.act_t0[pos + 1];
+        const int t0 = A.act_t0[pos];
+        int t1 = A.act_t0[pos + 1];
+        if (folded && t1 - t0 > FOLD_TILES) t1 = t0 + 1;
         for (int ti = t0 + g; ti < t1; ti += 8 * G) {   // eight loads in flight
             double w[8];
 #pragma unroll
@@ -438,12 +441,13 @@ __device__ __forceinline__ void tile_sums(const BulkArgs &A, int pos, const doub
     __syncthreads();
 }
 
-// The same sums once per block (one workgroup), left in its first tile's place
+// The same sums once per large block (one workgroup), left in its first tile's place
 template <int NV>
 __global__ __launch_bounds__(1024) void k_bulk_fold(BulkArgs A, const BulkBlock *st, double *part, bool refreshed)
 {
     __shared__ double sh[NV * (1024 / NV)];
     __shared__ double red[NV];
+    if (A.act_t0[blockIdx.x + 1] - A.act_t0[blockIdx.x] <= FOLD_TILES) return;
     const BulkBlock &S = st[A.act[blockIdx.x]];
     if (S.done || (refreshed && !S.refresh)) return;
     tile_sums<NV, 1024 / NV>(A, blockIdx.x, part, false, sh, red);
@@ -460,7 +464,7 @@ __global__ __launch_bounds__(BULK_TILE) void k_bulk_update(BulkArgs A)
     const int4 t = A.tiles[blockIdx.x];
     const BulkBlock &S = A.st[t.z];
     if (S.done) return;
-    tile_sums<NRHS>(A, t.w, A.part, A.fold, sh, red);
+    tile_sums<NRHS>(A, t.w, A.part, true, sh, red);
     double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     const int i = t.x + threadIdx.x / 2, h = 3 * (threadIdx.x % 2);
     if (i < t.y) {
@@ -526,7 +530,7 @@ __device__ __forceinline__ bool bulk_step(const BulkArgs &A, const int4 &t, doub
         if (writer) A.st1[t.z] = S;
         return false;
     }
-    tile_sums<NPART>(A, t.w, A.part_rz, A.fold, sh, red);
+    tile_sums<NPART>(A, t.w, A.part_rz, true, sh, red);
     bool refresh = false;
     double res[NRHS];
     float beta[NRHS];
@@ -566,7 +570,7 @@ __global__ __launch_bounds__(BULK_TILE) void k_bulk_finish(BulkArgs A)
         if (writer) A.st[t.z] = S;
         return;
     }
-    tile_sums<NPART>(A, t.w, A.part_tr, A.fold, sh, red);
+    tile_sums<NPART>(A, t.w, A.part_tr, true, sh, red);
     bool all = true;
     int conv = 0;
     double res[NRHS];
@@ -1325,7 +1329,7 @@ static int bulk_solve(hfem_batch *bt, const double *db, double *dx, int maxit)
         return m;
     };
     int ntiles = (int)bt->h_tiles.size(), nact = nbulk;
-    A.fold = most_tiles() > FOLD_TILES;
+    bool fold = most_tiles() > FOLD_TILES;   // a block that k_bulk_fold sums
     k_bulk_init<<<ntiles, BULK_TILE, 0, st>>>(A);
     k_bulk_start<<<nact, BULK_TILE, 0, st>>>(A);
     HIPFEM_CHECK(hipGetLastError());
@@ -1356,18 +1360,18 @@ static int bulk_solve(hfem_batch *bt, const double *db, double *dx, int maxit)
                 if (rc) return rc;
                 ntiles = (int)bt->h_tiles.size();
                 nact = (int)act.size();
-                A.fold = most_tiles() > FOLD_TILES;
+                fold = most_tiles() > FOLD_TILES;
             }
         }
         const bool timed = bt->profiling && bt->ev_used < BULK_CHECK;
         if (timed) HIPFEM_CHECK(hipEventRecord(bt->ev[2 * bt->ev_used], st));
         hipLaunchKernelGGL(spmv, dim3(ntiles), dim3(BULK_TILE), 0, st, A);
         if (timed) HIPFEM_CHECK(hipEventRecord(bt->ev[2 * bt->ev_used++ + 1], st));
-        if (A.fold) k_bulk_fold<NRHS><<<nact, 1024, 0, st>>>(A, A.st, A.part, false);
+        if (fold) k_bulk_fold<NRHS><<<nact, 1024, 0, st>>>(A, A.st, A.part, false);
         k_bulk_update<<<ntiles, BULK_TILE, 0, st>>>(A);
-        if (A.fold) k_bulk_fold<NPART><<<nact, 1024, 0, st>>>(A, A.st, A.part_rz, false);
+        if (fold) k_bulk_fold<NPART><<<nact, 1024, 0, st>>>(A, A.st, A.part_rz, false);
         hipLaunchKernelGGL(refresh, dim3(ntiles), dim3(BULK_TILE), 0, st, A);
-        if (A.fold) k_bulk_fold<NPART><<<nact, 1024, 0, st>>>(A, A.st1, A.part_tr, true);
+        if (fold) k_bulk_fold<NPART><<<nact, 1024, 0, st>>>(A, A.st1, A.part_tr, true);
         k_bulk_finish<<<ntiles, BULK_TILE, 0, st>>>(A);
         HIPFEM_CHECK(hipGetLastError());
     }

@@ -81,6 +81,27 @@ def test_bulk_sums_at_tile_edges(ctx, sizes, form):
     B.close()
 
 
+@pytest.mark.parametrize("form", [0, 1, 2])
+def test_bulk_bits_do_not_depend_on_the_neighbours(ctx, form):
+    """An RVE of 42 tiles in the bulk phase (two terms in every group of the
+    sums) beside one of more tiles than its workgroups sum themselves (1,124
+    of 96 rows), which leaves the tile list at another time: the same
+    iterations and solution bits as alone."""
+    from oofem_amd.rve import RVEBatch
+    got = []
+    for sizes in ((12,), (34, 12)):
+        B = RVEBatch(ctx, [(n, meshgen.LSPACE, 0.3, n) for n in sizes])
+        (c,) = B.chunks
+        B.set_options(tol=1e-10, split=0, bulk_form=form)
+        out = B.run()
+        x = c.x.download().reshape(c.n, 6)
+        i = len(sizes) - 1
+        got.append((out["iters"][i], out["resid"][i], x[c.rows[i]:c.rows[i + 1]]))
+        B.close()
+    (ia, ra, xa), (ib, rb, xb) = got
+    assert ia == ib and ra == rb and np.array_equal(xa, xb)
+
+
 def test_batch_autotune_picks_a_valid_shape(ctx):
     from oofem_amd.rve import RVEBatch
     B = RVEBatch(ctx, SPECS[:4])
