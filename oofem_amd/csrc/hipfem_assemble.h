@@ -259,11 +259,11 @@ __device__ __forceinline__ void rows_sum_columns(int t, const int q[3], int L, c
 // lanes of a slot form J^-1 and the tangent parts of its four Gauss points
 // into LDS, and every lane then runs over those points, forming the gradients
 // g (and M g) of its two nodes and of the row's node a: one read of a point
-// serves two blocks.  J^-1 (nine divisions), the gradients and the elastic
+// serves two blocks.  Elastic: J^-1 (nine divisions), the gradients and the
 // blocks are formed by the operations of gp_geometry and k_assemble in their
-// order, and the rows summed in ascending element order: K keeps the bits of
-// stored element matrices.  A mixed-precision solve to 1e-8 determines its
-// solution to about 1e-9, and one rounding of K moves it by as much.
+// order, and the rows summed in ascending element order, so that K keeps the
+// bits of stored element matrices.  A mixed-precision solve to 1e-8 determines
+// its solution to about 1e-9, and one rounding of K moves it by as much.
 //
 // Bound: the latency of its loads and LDS round trips at two to three waves a
 // SIMD (202 VGPRs with the tangent, 164 without; bounding it to three or four
@@ -357,7 +357,7 @@ __global__ __launch_bounds__(64) void k_assemble_rows_hex(AsmArgs A)
                     if (c & 1) __builtin_amdgcn_sched_barrier(0);   // keeps two nodes' loads in flight
                 }
                 double P[NP] = {}, dV = 0.0;
-                if (!hex_inverse(J, P, dV)) atomicMin(A.bad, e);
+                if (!(TAN ? hex_inverse_rcp(J, P, dV) : hex_inverse(J, P, dV))) atomicMin(A.bad, e);
                 dV = fabs(dV);   // the rule's weights are 1
                 if constexpr (TAN) {
                     const size_t gp = (size_t)e * 8 + 4 * hx + q;
@@ -575,24 +575,14 @@ __global__ __launch_bounds__(256) void k_element_matrices_quad(AsmArgs A, double
     __syncthreads();
     const double *mp = A.mat + (size_t)HIPFEM_MATP * A.emat[e];
     if (t < NGP) {
-        double J[9], I[9], xi[3], w;
+        double J[9], I[9], xi[3], w, det;
         gauss_point(HIPFEM_QSPACE, t, xi, w);
 #pragma unroll
         for (int i = 0; i < 9; i++) J[i] = sJ[t][i];
-        I[0] = J[4] * J[8] - J[5] * J[7];
-        I[1] = J[2] * J[7] - J[1] * J[8];
-        I[2] = J[1] * J[5] - J[2] * J[4];
-        I[3] = J[5] * J[6] - J[3] * J[8];
-        I[4] = J[0] * J[8] - J[2] * J[6];
-        I[5] = J[2] * J[3] - J[0] * J[5];
-        I[6] = J[3] * J[7] - J[4] * J[6];
-        I[7] = J[1] * J[6] - J[0] * J[7];
-        I[8] = J[0] * J[4] - J[1] * J[3];
-        const double det = J[0] * I[0] + J[1] * I[3] + J[2] * I[6];
-        if (!(fabs(det) > 1.e-30)) atomicMin(A.bad, e);
-        const double id = 1. / det, dV = fabs(det) * w;
+        if (!hex_inverse_rcp(J, I, det)) atomicMin(A.bad, e);
+        const double dV = fabs(det) * w;
 #pragma unroll
-        for (int i = 0; i < 9; i++) sJ[t][i] = I[i] * id;
+        for (int i = 0; i < 9; i++) sJ[t][i] = I[i];
         sQ[t][0] = dV;
         if constexpr (TAN) {
             const size_t gp = (size_t)e * NGP + t;
