@@ -222,18 +222,18 @@ __device__ __forceinline__ void rows_sum_entries(int t, int q0, int q1, int q2, 
 
 // Tetrahedra, 45 columns with few of 16 slots each: a lane owns a column of
 // all three rows and reads the sources it has (1.06 against 1.19 ms for the
-// 412,000 nodes of the 70x70x82 block with one entry a lane).
+// 412,000 nodes of the 70x70x82 block with one entry a lane).  The lane's first
+// column stays in acc over the passes.
 template <int NC>
 __device__ __forceinline__ void rows_sum_columns(int t, const int q[3], int L, const double *sV, const uint64_t *codes,
                                                  const int32_t *__restrict__ rowptr, double *__restrict__ val,
-                                                 bool first)
+                                                 bool first, bool last, double acc[3])
 {
     for (int p = t; p < L; p += 64) {
-        double s[3] = {0.0, 0.0, 0.0};
-        if (!first) {
+        double s[3] = {acc[0], acc[1], acc[2]};
+        if (p != t) {
 #pragma unroll
-            for (int i = 0; i < 3; i++)
-                if (q[i] > 0) s[i] = val[rowptr[q[i] - 1] + p];
+            for (int i = 0; i < 3; i++) s[i] = !first && q[i] > 0 ? val[rowptr[q[i] - 1] + p] : 0.0;
         }
 #pragma unroll
         for (int h = 0; h < 2; h++) {
@@ -248,8 +248,10 @@ __device__ __forceinline__ void rows_sum_columns(int t, const int q[3], int L, c
             }
         }
 #pragma unroll
-        for (int i = 0; i < 3; i++)
-            if (q[i] > 0) val[rowptr[q[i] - 1] + p] = s[i];
+        for (int i = 0; i < 3; i++) {
+            if (p == t) acc[i] = s[i];
+            if ((p != t || last) && q[i] > 0) val[rowptr[q[i] - 1] + p] = s[i];
+        }
     }
 }
 
@@ -458,6 +460,7 @@ __global__ __launch_bounds__(64) void k_assemble_rows_tet(AsmArgs A)
     if (r0 <= 0) return;
     const int L = A.rowptr[r0] - A.rowptr[r0 - 1];
     const int j0 = A.nptr[n], cnt = A.nptr[n + 1] - j0;
+    double acc[3] = {0.0, 0.0, 0.0};
     for (int base = 0; base < cnt; base += 16) {
         const int slot = base + k;
         const bool valid = slot < cnt;
@@ -534,7 +537,7 @@ __global__ __launch_bounds__(64) void k_assemble_rows_tet(AsmArgs A)
                 if (qb[j] > 0) bytes[(off + rk++) * 16 + k] = (uint8_t)(3 * b + j);
         }
         wave_lds_fence();
-        rows_sum_columns<12>(t, q, L, sV, sCodes, A.rowptr, A.val, base == 0);
+        rows_sum_columns<12>(t, q, L, sV, sCodes, A.rowptr, A.val, base == 0, base + 16 >= cnt, acc);
     }
 }
 

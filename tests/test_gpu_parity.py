@@ -615,21 +615,26 @@ def test_pcg_multiple_right_hand_sides(ctx, precision):
 def _row_form_deck(kind):
     """Meshes at the edges of the assembly by rows: every node's elements
     repeated (more elements at a node than one pass takes), random partly
-    fixed nodes, a node without elements, an odd node count, and a star whose
-    centre row is longer than the row form takes (the color form)."""
+    fixed nodes, a node without elements, an odd node count, a fan whose centre
+    has more than one pass of elements and more columns than lanes, and a star
+    whose centre row is longer than the row form takes (the color form)."""
     rng = np.random.default_rng(11)
     hexes = kind.startswith("hex")
     mat = np.array([[meshgen.MAT_MISES, 210e3, 0.3, 250.0, 2e3, 0, 0, 0],
                     [meshgen.MAT_ISOLE, 70e3, 0.2, 0, 0, 0, 0, 0]])
-    if kind.startswith("quad"):
+    if kind.startswith("quad") and not kind.endswith("star"):
         coords, conn = meshgen._rve_mesh(2, meshgen.QSPACE)
         coords = np.concatenate([coords + 0.02 * rng.standard_normal(coords.shape), [[9.0, 9.0, 9.0]]])
         conn = np.concatenate([conn] * (2 if kind.endswith("repeated") else 1))
         return meshgen.Deck(kind, meshgen.QSPACE, coords, conn, (rng.random(len(conn)) < 0.2).astype(np.int32), mat,
                             rng.random((len(coords), 3)) < 0.2, np.zeros_like(coords))
-    if kind.endswith("star"):
-        m, nen = 60, 8 if hexes else 4
-        ref = meshgen._rve_mesh(1, meshgen.LSPACE) if hexes else meshgen.kuhn_tets(1, 1, 1, 1.0, 1.0, 1.0)
+    if kind.endswith(("star", "fan")):
+        m = {"hex_fan": 12, "tet_fan": 25, "quad_star": 10}.get(kind, 60)
+        if kind == "quad_star":
+            ref = meshgen._rve_mesh(1, meshgen.QSPACE)
+        else:
+            ref = meshgen._rve_mesh(1, meshgen.LSPACE) if hexes else meshgen.kuhn_tets(1, 1, 1, 1.0, 1.0, 1.0)
+        nen = len(ref[1][0])
         conn0, xyz = ref[1][0], ref[0]
         coords, conn = [xyz[conn0[0]]], np.zeros((m, nen), np.int64)
         for e in range(m):
@@ -648,14 +653,15 @@ def _row_form_deck(kind):
         coords = np.concatenate([coords, [[9.0, 9.0, 9.0]]])
         if len(coords) % 2 == 0:
             coords = np.concatenate([coords, [[9.0, 9.0, 8.0]]])
-    bc = rng.random((len(coords), 3)) < (0.02 if kind.endswith("star") else 0.2)
-    return meshgen.Deck(kind, meshgen.LSPACE if hexes else meshgen.LTRSPACE, coords, conn,
+    bc = rng.random((len(coords), 3)) < (0.02 if kind.endswith(("star", "fan")) else 0.2)
+    et = meshgen.LSPACE if hexes else meshgen.QSPACE if kind == "quad_star" else meshgen.LTRSPACE
+    return meshgen.Deck(kind, et, coords, conn,
                         (rng.random(len(conn)) < 0.2).astype(np.int32), mat, bc, np.zeros_like(coords))
 
 
 @pytest.mark.parametrize("tangent", [False, True])
-@pytest.mark.parametrize("kind", ["hex_partial", "hex_repeated", "hex_star", "tet_partial", "tet_repeated", "tet_star",
-                                  "quad_partial", "quad_repeated"])
+@pytest.mark.parametrize("kind", ["hex_partial", "hex_repeated", "hex_fan", "hex_star", "tet_partial", "tet_repeated",
+                                  "tet_fan", "tet_star", "quad_partial", "quad_repeated", "quad_star"])
 def test_row_assembly_edges_match_oracle(ctx, kind, tangent):
     """The row form (and the color form behind it) against the oracle, with
     the tolerances of the plain meshes: 1e-13 of the largest entry for the
@@ -677,6 +683,8 @@ def test_row_assembly_edges_match_oracle(ctx, kind, tangent):
             assert np.abs(a - b).max() <= 1e-12 * np.abs(fo).max()
         np.testing.assert_allclose(ebe, ebeo, rtol=1e-12)
     rp, ci, val = oracle.csr(d, state=st, tangent=tangent)
+    longest = np.diff(rp).max()
+    assert longest > 512 if kind.endswith("star") else 64 < longest <= 512 if kind.endswith("fan") else longest <= 512
     for _ in range(2):
         ev.assemble_stiffness(K, tangent=tangent)
         grp, gci, gval = K.download()
@@ -729,8 +737,8 @@ def test_elastic_rows_keep_the_bits_of_the_element_matrices(ctx):
 
 
 @pytest.mark.parametrize("tangent", [False, True])
-@pytest.mark.parametrize("kind", ["hex_partial", "hex_repeated", "tet_partial", "tet_repeated", "quad_partial",
-                                  "quad_repeated"])
+@pytest.mark.parametrize("kind", ["hex_partial", "hex_repeated", "hex_fan", "tet_partial", "tet_repeated", "tet_fan",
+                                  "quad_partial", "quad_repeated"])
 def test_row_blocks_are_transposes(ctx, kind, tangent):
     """The rows of two nodes are formed by different waves, in several passes
     where a node has more elements than one takes: their blocks (I, J) and
