@@ -148,6 +148,30 @@ def test_merged_iteration_matches_separate_reductions(ctx, name, form, maxit):
     assert np.array_equal(xa, xb) and np.array_equal(ha, hb)
 
 
+@pytest.mark.parametrize("name,form", [("lspace", 1), ("qspace", 2)])
+def test_merged_fp32_iteration_matches_separate_reductions(ctx, name, form):
+    """The same for the FP32 inner solves of iterative refinement (precision
+    1): the same corrections, iterations and solution bits."""
+    from oofem_amd.hipfem import HipCSRSparseMtrx, HipPCGSolver
+    d = SHAPE_DECKS[name]
+    rp, ci, val = oracle.csr(d)
+    K = HipCSRSparseMtrx(ctx)
+    K.buildInternalStructureCSR(rp, ci)
+    K.upload_values(val)
+    assert K.is_nodeblocked() == form
+    b = np.random.default_rng(4).standard_normal(d.neq)
+    out = []
+    for fused in (0, 1):
+        s = HipPCGSolver(ctx, lstol=1e-10, lsiter=20000, lsprecond=1, precision=1)
+        s.set_fused(fused)
+        x = np.zeros(d.neq)
+        reason, it, res = s.solve(K, b, x)
+        assert reason == 1 and it > 0
+        out.append((it, res, s.last_outer(), x))
+    (ia, ea, oa, xa), (ib, eb, ob, xb) = out
+    assert (ia, ea, oa) == (ib, eb, ob) and oa > 1 and np.array_equal(xa, xb)
+
+
 def test_config0_linear_static_parity(ctx):
     from oofem_amd.drivers import linear_static, reaction_sums
     d = meshgen.config0()
