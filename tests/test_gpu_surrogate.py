@@ -66,6 +66,20 @@ def test_step_edges_match_oracle(net, rows):
     assert loss2 == loss and np.array_equal(g2, g)
 
 
+def test_bias_gradient_sums_to_fp32_rounding(net):
+    """The bias gradients sum every row of the batch.  The output layer's
+    (targets with a mean, so that partial sums grow) is within 7e-8 of the FP64
+    gradient in the norm: 4.5e-8 from pairwise sums, 1e-8 from 1 / (27 B)
+    rounded; 64 slabs added one after the other miss it by 1e-7."""
+    rng = np.random.default_rng(12)
+    X = rng.standard_normal((4096, 13)).astype(np.float32)
+    Y = (rng.standard_normal((4096, 27)) + 0.3).astype(np.float32)
+    _, g = net.gradients(X, Y)
+    _, gref = M.loss_and_grad(net.params().astype(np.float64), X.astype(np.float64), Y.astype(np.float64))
+    a = sum(int(np.prod(s)) for s in M.SHAPES[:-1])
+    assert np.linalg.norm(g[a:] - gref[a:]) <= 7e-8 * np.linalg.norm(gref[a:])
+
+
 def test_training_samples_follow_the_return_mapping(net):
     """Every generated sample is the plain return mapping (oracle) of its own
     inputs: stress and consistent tangent at (eps, epsp_n, kappa_n)."""
