@@ -54,10 +54,12 @@ constexpr int GRP_MAX_GRID = 16384;   // row-group and node-block PCG products: 
 // Up to this product grid the one-block reductions go into the kernels that
 // follow them (merged iteration), every workgroup summing all partials: the
 // launches saved are worth about 8 us an iteration, the sums cost grid^2.
-// Measured for a whole solve, five launches / merged: hex 6x6x22 (grid 198)
-// 5.47 / 4.25 ms, hex 16x16x64 (1088) 16.8 / 14.8, tet 35x35x41 (3300)
-// 33.5 / 33.2; beyond the limit hex 26x26x100 (9112) 49.7 / 54.5 and tet
-// 50x50x60 87.8 / 105.8.
+// Measured for a whole solve, five launches / merged: hexahedra (node blocks)
+// 6x6x22 (grid 135) 4.36 / 3.19 ms, 16x16x64 (2,312) 15.6 / 13.6, 20x20x80
+// (4,410) 25.9 / 23.6, 22x22x88 (5,819) 32.9 / 33.2, 26x26x100 (9,113) 49.1 /
+// 52.9; tetrahedra (row groups) 24x24x28 (1,094) 10.0 / 9.0, 33x33x39 (2,818)
+// 16.7 / 16.4, 35x35x41 (3,321) 19.7 / 19.7, 37x37x44 (3,971) 22.1 / 21.7,
+// 38x38x45 (4,250) 23.0 / 24.7, 50x50x60 46.7 / 56.4.
 constexpr int MERGE_MAX = 4096;
 
 template <typename T>
