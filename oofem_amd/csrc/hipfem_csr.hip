@@ -36,6 +36,7 @@ int ensure_partials(hipfem_ctx *ctx, size_t n)
     if (ctx->partials_cap >= n) return 0;
     if (ctx->d_partials) HIPFEM_CHECK(hipFree(ctx->d_partials));
     ctx->d_partials = nullptr;
+    ctx->partials_cap = 0;   // if the allocation fails, the next call must not take the old size for granted
     size_t cap = std::max<size_t>(n, 8192);
     HIPFEM_CHECK(hipMalloc(&ctx->d_partials, cap * sizeof(double)));
     ctx->partials_cap = cap;
