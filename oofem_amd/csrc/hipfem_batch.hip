@@ -30,8 +30,8 @@
 // stopping rule as the persistent kernel live in a BulkBlock record per
 // block.  An iteration is four launches: every workgroup of a block sums the
 // block's tile partials itself at the start of the kernel that needs them
-// (large blocks: a launch for it, FOLD_TILES), and the block's first one
-// writes the record, to the other of two places.  Finished blocks drop out of
+// (large blocks and many tiles: a launch for it, FOLD_TILES), and the block's
+// first one writes the record, to the other of two places.  Finished blocks drop out of
 // the tile list when the host next looks (every BULK_CHECK iterations); until
 // then their tiles return at once.
 
@@ -284,24 +284,30 @@ __global__ __launch_bounds__(BS) void k_batch_pcg(int nblocks, const int *__rest
 // ------------------------------------------------------------ bulk phase
 constexpr int BULK_TILE = 256;   // threads per workgroup
 // rows per tile: 32 whole nodes, eight lanes each; two threads per row
-// elsewhere.  24 RVEs of n = 8 to 16, all six solves: 96 rows 29.4 ms, 255
-// rows (85 nodes in three uneven passes, 1.7 workgroups per CU) 37.2, 126
-// rows 32.6 (before the loads of the sums were batched, where 96 took 31.9),
-// 48 rows 36.2 (twice the partials to sum).
+// elsewhere.  Six solves, tiles of 48 / 96 / 126 rows / 255 rows and seven
+// launches: 24 RVEs of n = 8 to 16 (1,852 tiles of 96) 32.6 / 27.5 / 29.7 /
+// 37.3 ms, 94 RVEs of n = 16 to 32 (38,795) 203 / 152 / 165 / 164, 512 RVEs of
+// n = 8 to 32 842 / 934 / 906 / 868 solves/s.
 constexpr int TILE_ROWS = 96;
 constexpr int SUM_GROUPS = 21;   // BULK_TILE / NPART
+constexpr int SUM_CLASSES = 84;  // classes of a block's tiles in the sums
 // Blocks of up to FOLD_TILES tiles are summed by each of their workgroups;
-// beyond it, where that costs tiles^2, by a launch per sum.  Measured for one
-// RVE's six solves, summed by all / by a launch / with seven launches and tiles
-// of 255 rows: LSpace n = 16 (105 tiles) 3.3 / 3.9 / 5.9 ms, QSpace 16 (442)
-// 15.1 / 17.3 / 23.4, LSpace 32 (930) 13.0 / 13.6 / 14.3, QSpace 22 (1198)
-// 41.4 / 41.3 / 41.1, LSpace 48 (3244) 65 / 40.6 / 40.6.
-constexpr int FOLD_TILES = 1024;
+// beyond it, where that costs tiles^2, by a launch per sum.  One RVE's six
+// solves, summed by all / by a launch: LSpace n = 16 (106 tiles) 3.4 / 4.4 ms,
+// QSpace 16 (443) 14.9 / 16.7, LSpace 32 (931) 11.8 / 12.4, QSpace 22 (1,199)
+// 37.5 / 37.7, LSpace 48 (3,245; with an earlier kernel) 65 / 40.6.
+// A launch of more than FOLD_ALL tiles holds more workgroups than run at once,
+// each repeating the sums: there every block of more tiles than one sum reads
+// at once (FOLD_MIN) has them from a launch.  1,852 tiles 27.7 / 30.9 ms, 3,715
+// 17.5 / 17.5, 4,715 21.8 / 21.5, 7,416 35.8 / 33.5, QSpace 4,311 97.0 / 85.4,
+// 38,795 199 / 152.
+constexpr int FOLD_TILES = 1024, FOLD_ALL = 4096, FOLD_MIN = SUM_GROUPS;
 constexpr int BULK_CHECK = 16;   // iterations between host looks at the done flags
 constexpr int NPART = 2 * NRHS;  // partial sums per tile
 
 struct BulkBlock {
     double rho[NRHS], normb[NRHS], rmax[NRHS], res[NRHS];
+    float beta[NRHS];   // of an iteration without a reliable update
     int conv;      // bit k: column k meets the tolerance
     int it, nupd;
     int refresh;   // 1: this iteration replaces the residuals by b - A x
@@ -326,6 +332,7 @@ struct BulkArgs {
     double *x;
     float *r, *z, *p, *q;
     double *part, *part_rz, *part_tr;   // [tile][NPART]: p.q; r.z and r.r; those of a reliable update
+    int fold;                // blocks of more tiles than this are summed by k_bulk_fold
     double tol, delta;
     int maxit;
     int *iters, *updates;
@@ -407,51 +414,58 @@ __global__ __launch_bounds__(BULK_TILE) void k_bulk_spmv(BulkArgs A)
 }
 
 // The sums of a block's tile partials, by every workgroup of the block that
-// needs them (a fixed order): no launch of its own for the reductions, whose
-// cost (5 to 7 us each) was its latency.  A thread sums one value over every SUM_GROUPS-th tile
-// (coalesced, no wave reduction), then one thread per value sums the groups.
-// folded: a large block's sums, which k_bulk_fold has left in its first tile's
-// place; decided per block, so that its bits do not depend on its neighbours.
-template <int NV, int G = SUM_GROUPS>
-__device__ __forceinline__ void tile_sums(const BulkArgs &A, int pos, const double *part, bool folded, double *sh,
-                                          double *red)
+// needs them: no launch of its own for the reductions, whose cost (5 to 7 us
+// each) was its latency.  The tiles fall into 84 classes (every 84th tile, in
+// order; coalesced, no wave reduction), and the class sums are added in one
+// fixed order, the same here and in k_bulk_fold: which of them sums a block
+// does not show in its bits.  TG thread groups take 84 / TG classes each.
+template <int NV, int TG>
+__device__ __forceinline__ void class_sums(const double *part, int t0, int t1, double *sh, double *red)
 {
+    constexpr int C = SUM_CLASSES / TG;
+    static_assert(TG * C == SUM_CLASSES && (TG == 21 || TG == 42 || TG == 84), "thread groups");
     const int g = threadIdx.x / NV, k = threadIdx.x % NV;
-    if (g < G) {
-        double s = 0.0;
-        const int t0 = A.act_t0[pos];
-        int t1 = A.act_t0[pos + 1];
-        if (folded && t1 - t0 > FOLD_TILES) t1 = t0 + 1;
-        for (int ti = t0 + g; ti < t1; ti += 8 * G) {   // eight loads in flight
+    if (g < TG) {
+        double s[C];
+#pragma unroll
+        for (int j = 0; j < C; j++) s[j] = 0.0;
+        for (int ti = t0 + g; ti < t1; ti += 8 * TG) {   // eight loads in flight
             double w[8];
 #pragma unroll
-            for (int j = 0; j < 8; j++) w[j] = part[(size_t)min(ti + j * G, t1 - 1) * NPART + k];
+            for (int j = 0; j < 8; j++) w[j] = part[(size_t)min(ti + j * TG, t1 - 1) * NPART + k];
 #pragma unroll
-            for (int j = 0; j < 8; j++) s += ti + j * G < t1 ? w[j] : 0.0;
+            for (int j = 0; j < 8; j++) s[j % C] += ti + j * TG < t1 ? w[j] : 0.0;
         }
-        sh[g * NV + k] = s;
+        if constexpr (C == 4) sh[g * NV + k] = (s[0] + s[2]) + (s[1] + s[3]);
+        else if constexpr (C == 2) sh[g * NV + k] = s[0] + s[1];
+        else sh[g * NV + k] = s[0];
     }
     __syncthreads();
     if (threadIdx.x < NV) {
+        const double *v = sh + threadIdx.x;
         double s = 0.0;
 #pragma unroll
-        for (int i = 0; i < G; i++) s += sh[i * NV + threadIdx.x];
+        for (int i = 0; i < 21; i++) {
+            if constexpr (TG == 21) s += v[i * NV];
+            else if constexpr (TG == 42) s += v[i * NV] + v[(i + 21) * NV];
+            else s += (v[i * NV] + v[(i + 42) * NV]) + (v[(i + 21) * NV] + v[(i + 63) * NV]);
+        }
         red[threadIdx.x] = s;
     }
     __syncthreads();
 }
 
-// The same sums once per large block (one workgroup), left in its first tile's place
 template <int NV>
-__global__ __launch_bounds__(1024) void k_bulk_fold(BulkArgs A, const BulkBlock *st, double *part, bool refreshed)
+__device__ __forceinline__ void tile_sums(const BulkArgs &A, int pos, const double *part, bool folded, double *sh,
+                                          double *red)
 {
-    __shared__ double sh[NV * (1024 / NV)];
-    __shared__ double red[NV];
-    if (A.act_t0[blockIdx.x + 1] - A.act_t0[blockIdx.x] <= FOLD_TILES) return;
-    const BulkBlock &S = st[A.act[blockIdx.x]];
-    if (S.done || (refreshed && !S.refresh)) return;
-    tile_sums<NV, 1024 / NV>(A, blockIdx.x, part, false, sh, red);
-    if (threadIdx.x < NV) part[(size_t)A.act_t0[blockIdx.x] * NPART + threadIdx.x] = red[threadIdx.x];
+    const int t0 = A.act_t0[pos], t1 = A.act_t0[pos + 1];
+    if (folded && t1 - t0 > A.fold) {   // the sums stand in the first tile's place
+        if (threadIdx.x < NV) red[threadIdx.x] = part[(size_t)t0 * NPART + threadIdx.x];
+        __syncthreads();
+    } else {
+        class_sums<NV, NV == NRHS ? 42 : 21>(part, t0, t1, sh, red);
+    }
 }
 
 // alpha from the product's partials (0 for a converged column and where the
@@ -518,46 +532,85 @@ __device__ __forceinline__ void tile_direction(const BulkArgs &A, const int4 &t,
     for (int k = 0; k < 3; k++) A.p[o + k] = fmaf(h ? beta[3 + k] : beta[k], A.p[o + k], A.z[o + k]);
 }
 
-// After the update: does the block ask for a reliable update (a residual met
-// the tolerance or dropped by delta)?  Returns true for its tiles if so, which
-// then form b - A x; else the direction is updated here.  The block's first
-// tile writes the new state to st1.
+// After the update, from its sums: does the block ask for a reliable update (a
+// residual met the tolerance or dropped by delta)?  With write, the new state,
+// with beta where there is no update, goes to st1.
+__device__ __forceinline__ bool step_state(const BulkArgs &A, int b, const double *red, bool write)
+{
+    const BulkBlock &S = A.st[b];
+    bool refresh = false;
+    double res[NRHS];
+#pragma unroll
+    for (int k = 0; k < NRHS; k++) {
+        res[k] = sqrt(red[NRHS + k]) / S.normb[k];
+        if (!(S.conv >> k & 1) && (res[k] <= A.tol || res[k] < A.delta * S.rmax[k])) refresh = true;
+    }
+    if (write) {
+        BulkBlock &N = A.st1[b];
+        N = S;
+        N.it = S.it + 1;
+        N.refresh = refresh;
+#pragma unroll
+        for (int k = 0; k < NRHS; k++) {
+            const bool c = S.conv >> k & 1;
+            N.res[k] = res[k];
+            N.beta[k] = c ? 0.f : (float)(red[k] / S.rho[k]);
+            if (!refresh && !c) N.rho[k] = red[k];
+        }
+        if (!refresh && N.it >= A.maxit) bulk_finish(A, N, false);
+    }
+    return refresh;
+}
+
+// The step of a tile's block: true where the tile then forms b - A x.  The
+// block's first tile writes the state (k_bulk_fold where it has the sums);
+// k_bulk_finish forms the direction.  (In the kernels of the reliable update,
+// which hold few waves, the direction took 90 us instead of 30 for 25,000 tiles.)
 __device__ __forceinline__ bool bulk_step(const BulkArgs &A, const int4 &t, double *sh, double *red)
 {
+    if (A.act_t0[t.w + 1] - A.act_t0[t.w] > A.fold) {
+        const BulkBlock &N = A.st1[t.z];
+        return !N.done && N.refresh;
+    }
     const BulkBlock &S = A.st[t.z];
     const bool writer = (int)blockIdx.x == A.act_t0[t.w] && threadIdx.x == 0;
     if (S.done) {
         if (writer) A.st1[t.z] = S;
         return false;
     }
-    tile_sums<NPART>(A, t.w, A.part_rz, true, sh, red);
-    bool refresh = false;
-    double res[NRHS];
-    float beta[NRHS];
-#pragma unroll
-    for (int k = 0; k < NRHS; k++) {
-        const bool c = S.conv >> k & 1;
-        res[k] = sqrt(red[NRHS + k]) / S.normb[k];
-        if (!c && (res[k] <= A.tol || res[k] < A.delta * S.rmax[k])) refresh = true;
-        beta[k] = c ? 0.f : (float)(red[k] / S.rho[k]);
-    }
-    if (writer) {
-        BulkBlock &N = A.st1[t.z];
-        N = S;
-        N.it = S.it + 1;
-        N.refresh = refresh;
-#pragma unroll
-        for (int k = 0; k < NRHS; k++) {
-            N.res[k] = res[k];
-            if (!refresh && !(S.conv >> k & 1)) N.rho[k] = red[k];
-        }
-        if (!refresh && N.it >= A.maxit) bulk_finish(A, N, false);
-    }
-    if (!refresh) tile_direction(A, t, beta);
-    return refresh;
+    tile_sums<NPART>(A, t.w, A.part_rz, false, sh, red);
+    return step_state(A, t.z, red, writer);
 }
 
-// After a reliable update: beta from the true residual and the direction; for
+// What a large block's sums are needed for: the update, the step after it
+// (done here), the direction after a reliable update
+enum FoldFor { FOLD_UPDATE, FOLD_STEP, FOLD_FINISH };
+
+// The same sums once per large block (one workgroup), left in its first tile's place
+template <FoldFor F>
+__global__ __launch_bounds__((F == FOLD_UPDATE ? NRHS : NPART) * SUM_CLASSES) void k_bulk_fold(BulkArgs A)
+{
+    constexpr int NV = F == FOLD_UPDATE ? NRHS : NPART;
+    __shared__ double sh[NV * SUM_CLASSES];
+    __shared__ double red[NV];
+    const int t0 = A.act_t0[blockIdx.x], t1 = A.act_t0[blockIdx.x + 1], b = A.act[blockIdx.x];
+    if (t1 - t0 <= A.fold) return;
+    const BulkBlock &S = F == FOLD_FINISH ? A.st1[b] : A.st[b];
+    if (S.done) {
+        if (F == FOLD_STEP && threadIdx.x == 0) A.st1[b] = S;
+        return;
+    }
+    if (F == FOLD_FINISH && !S.refresh) return;
+    double *part = F == FOLD_UPDATE ? A.part : F == FOLD_STEP ? A.part_rz : A.part_tr;
+    class_sums<NV, SUM_CLASSES>(part, t0, t1, sh, red);
+    if (F == FOLD_STEP) {
+        if (threadIdx.x == 0) step_state(A, b, red, true);
+    } else if (threadIdx.x < NV) {
+        part[(size_t)t0 * NPART + threadIdx.x] = red[threadIdx.x];
+    }
+}
+
+// The direction, after a reliable update with beta from the true residual; for
 // every block its first tile brings the state back to st
 __global__ __launch_bounds__(BULK_TILE) void k_bulk_finish(BulkArgs A)
 {
@@ -568,6 +621,7 @@ __global__ __launch_bounds__(BULK_TILE) void k_bulk_finish(BulkArgs A)
     const bool writer = (int)blockIdx.x == A.act_t0[t.w] && threadIdx.x == 0;
     if (S.done || !S.refresh) {
         if (writer) A.st[t.z] = S;
+        if (!S.done) tile_direction(A, t, S.beta);
         return;
     }
     tile_sums<NPART>(A, t.w, A.part_tr, true, sh, red);
@@ -1329,7 +1383,12 @@ static int bulk_solve(hfem_batch *bt, const double *db, double *dx, int maxit)
         return m;
     };
     int ntiles = (int)bt->h_tiles.size(), nact = nbulk;
-    bool fold = most_tiles() > FOLD_TILES;   // a block that k_bulk_fold sums
+    bool fold = false;   // a block that k_bulk_fold sums
+    auto set_fold = [&] {
+        A.fold = ntiles > FOLD_ALL ? FOLD_MIN : FOLD_TILES;
+        fold = most_tiles() > A.fold;
+    };
+    set_fold();
     k_bulk_init<<<ntiles, BULK_TILE, 0, st>>>(A);
     k_bulk_start<<<nact, BULK_TILE, 0, st>>>(A);
     HIPFEM_CHECK(hipGetLastError());
@@ -1360,18 +1419,18 @@ static int bulk_solve(hfem_batch *bt, const double *db, double *dx, int maxit)
                 if (rc) return rc;
                 ntiles = (int)bt->h_tiles.size();
                 nact = (int)act.size();
-                fold = most_tiles() > FOLD_TILES;
+                set_fold();
             }
         }
         const bool timed = bt->profiling && bt->ev_used < BULK_CHECK;
         if (timed) HIPFEM_CHECK(hipEventRecord(bt->ev[2 * bt->ev_used], st));
         hipLaunchKernelGGL(spmv, dim3(ntiles), dim3(BULK_TILE), 0, st, A);
         if (timed) HIPFEM_CHECK(hipEventRecord(bt->ev[2 * bt->ev_used++ + 1], st));
-        if (fold) k_bulk_fold<NRHS><<<nact, 1024, 0, st>>>(A, A.st, A.part, false);
+        if (fold) k_bulk_fold<FOLD_UPDATE><<<nact, NRHS * SUM_CLASSES, 0, st>>>(A);
         k_bulk_update<<<ntiles, BULK_TILE, 0, st>>>(A);
-        if (fold) k_bulk_fold<NPART><<<nact, 1024, 0, st>>>(A, A.st, A.part_rz, false);
+        if (fold) k_bulk_fold<FOLD_STEP><<<nact, NPART * SUM_CLASSES, 0, st>>>(A);
         hipLaunchKernelGGL(refresh, dim3(ntiles), dim3(BULK_TILE), 0, st, A);
-        if (fold) k_bulk_fold<NPART><<<nact, 1024, 0, st>>>(A, A.st1, A.part_tr, true);
+        if (fold) k_bulk_fold<FOLD_FINISH><<<nact, NPART * SUM_CLASSES, 0, st>>>(A);
         k_bulk_finish<<<ntiles, BULK_TILE, 0, st>>>(A);
         HIPFEM_CHECK(hipGetLastError());
     }

@@ -83,23 +83,25 @@ def test_bulk_sums_at_tile_edges(ctx, sizes, form):
 
 @pytest.mark.parametrize("form", [0, 1, 2])
 def test_bulk_bits_do_not_depend_on_the_neighbours(ctx, form):
-    """An RVE of 42 tiles in the bulk phase (two terms in every group of the
-    sums) beside one of more tiles than its workgroups sum themselves (1,124
-    of 96 rows), which leaves the tile list at another time: the same
-    iterations and solution bits as alone."""
+    """RVEs of 42 tiles (two terms in every class of the sums, or a launch of
+    their own for them) and of two tiles in the bulk phase: alone, beside one
+    of more tiles than its workgroups sum themselves (1,124 of 96 rows), and
+    beside four of them (more than 4,096 tiles in a launch), which leave the
+    tile list at another time: the same iterations and solution bits."""
     from oofem_amd.rve import RVEBatch
     got = []
-    for sizes in ((12,), (34, 12)):
-        B = RVEBatch(ctx, [(n, meshgen.LSPACE, 0.3, n) for n in sizes])
+    for others in ((), (34,), (34,) * 4):
+        B = RVEBatch(ctx, [(n, meshgen.LSPACE, 0.3, n) for n in others + (12, 5)])
         (c,) = B.chunks
         B.set_options(tol=1e-10, split=0, bulk_form=form)
         out = B.run()
         x = c.x.download().reshape(c.n, 6)
-        i = len(sizes) - 1
-        got.append((out["iters"][i], out["resid"][i], x[c.rows[i]:c.rows[i + 1]]))
+        i = len(others)
+        assert (out["resid"] > 0).all()
+        got.append((out["iters"][i:], out["updates"][i:], out["resid"][i:], x[c.rows[i]:]))
         B.close()
-    (ia, ra, xa), (ib, rb, xb) = got
-    assert ia == ib and ra == rb and np.array_equal(xa, xb)
+    for g in got[1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(got[0], g))
 
 
 def test_batch_autotune_picks_a_valid_shape(ctx):
