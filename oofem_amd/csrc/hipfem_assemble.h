@@ -223,11 +223,11 @@ __device__ __forceinline__ void rows_sum_entries(int t, int q0, int q1, int q2, 
 // Tetrahedra, 45 columns with few of 16 slots each: a lane owns a column of
 // all three rows and reads the sources it has (1.06 against 1.19 ms for the
 // 412,000 nodes of the 70x70x82 block with one entry a lane).  The lane's first
-// column stays in acc over the passes.
+// column stays in acc over the passes: 0.96 ms.
 template <int NC>
-__device__ __forceinline__ void rows_sum_columns(int t, const int q[3], int L, const double *sV, const uint64_t *codes,
-                                                 const int32_t *__restrict__ rowptr, double *__restrict__ val,
-                                                 bool first, bool last, double acc[3])
+__device__ __forceinline__ void rows_sum_columns(int t, const int q[3], int L, const double *sV,
+                                                 const uint64_t *codes, const int32_t *__restrict__ rowptr,
+                                                 double *__restrict__ val, bool first, bool last, double acc[3])
 {
     for (int p = t; p < L; p += 64) {
         double s[3] = {acc[0], acc[1], acc[2]};
@@ -267,13 +267,15 @@ __device__ __forceinline__ void rows_sum_columns(int t, const int q[3], int L, c
 // bits of stored element matrices.  A mixed-precision solve to 1e-8 determines
 // its solution to about 1e-9, and one rounding of K moves it by as much.
 //
-// Bound: the latency of its loads and LDS round trips at two to three waves a
-// SIMD (202 VGPRs with the tangent, 164 without; bounding it to three or four
-// waves spills and is slower).  Plastic 1,048,576-element block: tangent 3.92
-// ms, elastic 2.46 ms.  Before, storing every element's matrix (4.8 GB) and
-// summing the rows from them: 4.90 and 4.18 ms; with eight elements a wave in
-// that form 1.87 + 2.03 ms, and no buffer to hold here.  One node a wave: 4.2
-// and 2.6 ms.
+// Bound, by counters on the plastic 1,048,576-element block: FP64 issue, 66 %
+// of the cycles, and what two waves a SIMD leave uncovered (40 % of the waves'
+// time is waiting; 206 VGPRs with the tangent, 172 without; bounding it to
+// three or four waves spills and is slower); 4.9 GB of traffic are 1.1 TB/s.
+// Tangent 4.0 ms, elastic 3.4 ms.  Before, storing every element's matrix (4.8
+// GB) and summing the rows from them: 4.90 and 3.8 ms; with eight elements a
+// wave in that form 1.87 + 2.03 ms, and no buffer to hold here.  One node a
+// wave: 4.2 ms for the tangent.  With one reciprocal for the nine divisions the
+// elastic form takes 2.6 ms, in other bits.
 template <bool TAN, bool SUR>
 __global__ __launch_bounds__(64) void k_assemble_rows_hex(AsmArgs A)
 {
@@ -440,9 +442,10 @@ __global__ __launch_bounds__(64) void k_assemble_rows_hex(AsmArgs A)
 // x_i) / det J of the opposite face (the cofactor form of
 // fei3dtetlin.C:116-168), the row's node a shares g_a and M g_a through LDS.
 //
-// Bound: FP64 issue (about 500 instructions a node) and the LDS reads of the
-// row sums.  Plastic 2,410,800-element block: tangent 1.06 ms, elastic 0.79 ms;
-// 31 color launches adding 24-byte pieces into the zeroed values took 5.8 ms.
+// Bound, by counters on the plastic 2,410,800-element block: VALU issue, 69 % of
+// the cycles, with 60 % of the waves' time spent waiting for the gathers and
+// LDS.  Tangent 0.96 ms; 31 color launches adding 24-byte pieces into the
+// zeroed values took 5.8 ms.
 template <bool TAN, bool SUR>
 __global__ __launch_bounds__(64) void k_assemble_rows_tet(AsmArgs A)
 {
@@ -546,10 +549,10 @@ __global__ __launch_bounds__(64) void k_assemble_rows_tet(AsmArgs A)
 // pairs a <= b are each shared out over the threads; a block is stored with
 // its transpose.
 //
-// Bound: LDS reads of the gradients (7 doubles a pair and point, 15 with the
-// tangent).  9,261 elements: 0.157 ms and 0.153 ms for the rows summed from
-// them (267 MB each way); eight color launches of one wave an element, which
-// leave a SIMD one wave, took 0.78 ms.
+// Bound, by counters on 9,261 elements: VALU issue, 84 % of the cycles: 0.153
+// ms.  The rows summed from the matrices (267 MB each way) wait for their
+// loads, 69 % of the waves' time: 0.150 ms.  Eight color launches of one wave an
+// element, which leave a SIMD one wave, took 0.78 ms.
 template <bool TAN, bool SUR>
 __global__ __launch_bounds__(256) void k_element_matrices_quad(AsmArgs A, double *__restrict__ kbuf, int e0)
 {
@@ -686,7 +689,8 @@ __global__ __launch_bounds__(64) void k_assemble_gather(AsmArgs A, const double 
 #pragma unroll
         for (int u = 0; u < (8 * ROW2 + 63) / 64; u++) {
             const int idx = u * 64 + t, s = min(idx / ROW2, ns - 1);
-            v[u] = reinterpret_cast<const d2_t *>(kbuf + ((size_t)A.nadj[j0 + base + s] - (size_t)e0 * NEN) * (3 * NC))[idx % ROW2];
+            const size_t ea = (size_t)A.nadj[j0 + base + s] - (size_t)e0 * NEN;
+            v[u] = reinterpret_cast<const d2_t *>(kbuf + ea * (3 * NC))[idx % ROW2];
         }
         clear_codes<8>(t, L, sCodes);
         uint8_t *bytes = reinterpret_cast<uint8_t *>(sCodes);

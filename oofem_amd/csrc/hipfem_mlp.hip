@@ -200,7 +200,7 @@ struct StepArgs {
 // Bound: the chain of seven dependent products, each 32 matrix instructions
 // a wave and its weights from L2: 21 us for 4,096 rows (256 workgroups).  With
 // one launch a product (64 x 64 tiles on the vector units, 64 to 128 workgroups)
-// and one for each elementwise pass a training step took 503 us; it takes 50.
+// and one for each elementwise pass a training step took 503 us; it takes 46.
 template <bool BWD>
 __global__ __launch_bounds__(512) void k_mlp_step(StepArgs A)
 {
@@ -353,8 +353,9 @@ __device__ __forceinline__ void store_tiles(const f32x16 acc[NM][NN], int l, flo
 // 64 x 64 quarter a wave; block (2, z): layer 1 (32 units a wave) and the
 // output layer (32 inputs a wave).
 //
-// Bound: the latency of the row loads, 32 pairs of rows a slab: 23 us for 4,096
-// rows in 64 slabs.
+// Bound: the latency of the row loads (70 % of the waves' time is waiting, the
+// vector units issue in 7 % of the cycles), eight pairs of rows in flight: 19 us
+// for 4,096 rows in 64 slabs.
 __global__ __launch_bounds__(256) void k_mlp_wgrad(int B16, int rows, const float *__restrict__ xb,
                                                    const float *__restrict__ h, const float *__restrict__ dz,
                                                    const float *__restrict__ dy, float *__restrict__ slabs)

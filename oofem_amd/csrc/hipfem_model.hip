@@ -22,18 +22,20 @@
 //            temp strain, 32-37 committed stress.
 //
 // Kernels
-//   k_assemble<ET>   one 64-lane wave per element.  Lanes first compute the
-//                    Gauss-point geometry (dN/dx, dV) into LDS, then each lane
-//                    owns node pairs (a,b) and accumulates the 3x3 block
-//                    B_a^T D B_b dV over the Gauss points in registers before
-//                    scattering it.  IsoLE uses the closed form
-//                    lambda n_i m_j + G (n_j m_i + delta_ij n.m); MisesMat
-//                    the parts c I_dev + K 1x1 - m m^T of its tangent.
+//   k_assemble_rows_hex, _tet, k_element_matrices_quad + k_assemble_gather
+//                    stiffness by rows (hipfem_assemble.h).  IsoLE uses the
+//                    closed form lambda n_i m_j + G (n_j m_i + delta_ij n.m);
+//                    MisesMat the parts c I_dev + K 1x1 - m m^T of its tangent.
+//   k_assemble<ET>   the color form behind them: one 64-lane wave per element.
+//                    Lanes first compute the Gauss-point geometry (dN/dx, dV)
+//                    into LDS, then each lane owns node pairs (a,b) and
+//                    accumulates the 3x3 block B_a^T D B_b dV over the Gauss
+//                    points in registers before scattering it.
 //   k_internal*      one thread per Gauss point: geometry, strain B u_e, the
 //                    material update (radial return for MisesMat), B^T sigma dV
 //                    into LDS; then per element the Gauss-point sums in
 //                    ascending order are stored, and k_gather_nodal sums them
-//                    per node in ascending element order.
+//                    per node in a fixed order.
 
 #include <algorithm>
 #include <cmath>
