@@ -7,15 +7,6 @@
 
 namespace hipfem {
 
-// LDS stores of one wave complete in order, so a compiler-level fence is
-// enough between a wave's stores and its own loads (one-wave workgroups)
-__device__ __forceinline__ void wave_lds_fence()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // a double from another lane of the quad
 template <int CTRL>
 __device__ __forceinline__ double dpp_d(double v)

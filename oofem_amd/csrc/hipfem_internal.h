@@ -134,6 +134,22 @@ void ctx_release(hipfem_ctx *c);
 struct hfem_model;
 
 namespace hipfem {
+// LDS stores of one wave complete in order, so a compiler-level fence is
+// enough between a wave's stores and its own loads where no other wave uses
+// the same LDS
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// a fill instead of a memset, which a captured graph would record wrongly
+static __global__ void k_zero_f32(int64_t n, float *__restrict__ a)
+{
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) a[i] = 0.f;
+}
+
 // Device-resident scalars of one PCG solve.
 struct PcgState {
     double rho, alpha, beta, normb, res, tol;

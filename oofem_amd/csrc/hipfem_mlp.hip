@@ -128,12 +128,6 @@ __device__ __forceinline__ int aux_of(int i)
     return -1;
 }
 
-__global__ void k_zero_pad(int n, float *__restrict__ a)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) a[i] = 0.f;
-}
-
 __global__ void k_mlp_aux(const float *__restrict__ p, float *__restrict__ aux)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -467,16 +461,6 @@ __device__ __forceinline__ float bf2f(uint16_t b)
     return f;
 }
 
-// the activation tile of a wave is private to it: LDS operations of one
-// wave complete in order, so a wave-level barrier (no block barrier) orders
-// its stores before its own loads of the next layer
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // z silu(z) = z / (1 + e^-z) with the hardware exp2 and reciprocal (the
 // result is rounded to BF16, 8 bits, right after), then to BF16 by
 // v_cvt_pk_bf16_f32 (round to nearest even, as f2bf)
@@ -537,7 +521,7 @@ __global__ __launch_bounds__(64 * BF_WAVES) void k_mlp_bf16(int n, const float *
 #pragma unroll
                 for (int r = 0; r < 16; r++) act[tile_row(l, r) * ACT_LD + j] = silu_bf16(acc[nt][r] + bj);
             }
-            wave_lds_sync();
+            wave_lds_fence();   // the activation tile is the wave's own
             const uint16_t *Wn = layer == 0 ? W2 : layer == 1 ? W3 : W4;
 #pragma unroll
             for (int nt = 0; nt < 4; nt++) acc[nt] = (f32x16){0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -561,7 +545,7 @@ __global__ __launch_bounds__(64 * BF_WAVES) void k_mlp_bf16(int n, const float *
                     acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, b, acc[0], 0, 0, 0);
                 }
             }
-            wave_lds_sync();
+            wave_lds_fence();   // the activation tile is the wave's own
         }
         // output layer: 27 of 32 columns
         const int j = l & 31;
@@ -662,7 +646,7 @@ static int mlp_ensure_aux(hfem_mlp *m)
     hipStream_t s = m->ctx->stream;
     if (!m->d_aux) {
         HIPFEM_CHECK(hipMalloc(&m->d_aux, sizeof(float) * MLP_NAUX));
-        k_zero_pad<<<(MLP_NAUX + 255) / 256, 256, 0, s>>>(MLP_NAUX, m->d_aux);
+        k_zero_f32<<<(MLP_NAUX + 255) / 256, 256, 0, s>>>(MLP_NAUX, m->d_aux);
     }
     k_mlp_aux<<<(MLP_NPARAM + 255) / 256, 256, 0, s>>>(m->d_p, m->d_aux);
     HIPFEM_CHECK(hipGetLastError());

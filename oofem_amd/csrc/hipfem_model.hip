@@ -1531,11 +1531,6 @@ __global__ void k_fill(int64_t n, double v, double *__restrict__ a)
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) a[i] = v;
 }
 
-__global__ void k_zero_f32(int64_t n, float *__restrict__ a)
-{
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) a[i] = 0.f;
-}
-
 // out[k] = sum of partials[k np .. k np + np), block k; eight loads of a thread
 // in flight before their adds (one block for all three, one load at a time,
 // took 168 us for the 3 x 131,072 partials of the 64x64x256 block)
